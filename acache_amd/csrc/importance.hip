@@ -5,22 +5,25 @@
 //   w[r, h, a]       = softmax_a( q[r, h] . rot(K[a, kv(h)], shift_b) * scale )     a in [0, A)
 //   importance[b, a] += sum_{r in mask rows of b} sum_h w[r, h, a]
 //
-// Relocation is applied on the query side: q . rot(k, +s) = rot(q, -s) . k.  A first launch writes each request's
-// [MASK] queries, packed in mask-row order and (with relocation) rotated by minus the request's shift, into the
-// workspace (a few hundred rows per request); every launch after it reads that copy without an index in between
-// and the cached affix keys as they lie in the cache: one copy of the keys, shared by all requests and resident
-// in L2, instead of one re-rotated copy per request.  Three more launches, no atomics, so the result does not
-// depend on scheduling:
+// Relocation is applied on the query side: q . rot(k, +s) = rot(q, -s) . k, so that every launch reads the cached
+// affix keys as they lie in the cache: one copy, shared by all requests and resident in L2.  Scores come from the
+// matrix core (S^T = K Q^T, keys as rows, one query column per lane).  No atomics anywhere: the result does not
+// depend on scheduling.
+//
+// Head dims of 64 and 128 with affixes of up to 1280 keys: importance_fused_kernel, one pass over the scores, then
+// importance_reduce_kernel, which adds the per-head partial sums to importance[b, :] in a fixed order.
+//
+// Everything else, two passes: a first launch writes each request's [MASK] queries, packed in mask-row order and
+// (with relocation) rotated by minus the request's shift, into the workspace; then
 //   1. statistics pass: the mask rows of a wave stay in registers, the affix keys stream by, and the wave
 //      leaves log2 of each row's sum of 2^(score * c) in the workspace;
 //   2. column pass: the affix keys of a wave stay in registers, the request's mask rows stream by, the scores
 //      are recomputed, normalised with the stored row statistic (one subtraction in the exponent) and summed
 //      per key; each wave is the only writer of its entries of the per-head partial sums in the workspace;
-//   3. importance_reduce_kernel adds the per-head partial sums, in head order, to importance[b, :].
-// Scores come from the matrix core (S^T = K Q^T, keys as rows, one query column per lane).  Both passes exist
-// twice: for head dims of 64, 128 and 256 the streamed operand is staged through LDS by the copy engine and
-// shared by the four waves of a workgroup (importance_*_lds_kernel, further down); every other head dim loads
-// its fragments straight from global memory in operand layout, 16 bytes per lane, without LDS or barriers
+//   3. importance_reduce_kernel.
+// Both passes exist twice: for head dims of 64, 128 and 256 the streamed operand is staged through LDS by the copy
+// engine and shared by the four waves of a workgroup (importance_*_lds_kernel, further down); every other head dim
+// loads its fragments straight from global memory in operand layout, 16 bytes per lane, without LDS or barriers
 // (importance_stats_kernel, importance_colsum_kernel).
 #include <mutex>
 #include <type_traits>
@@ -589,18 +592,271 @@ __global__ __launch_bounds__(256) void importance_colsum_lds_kernel(ImportancePa
     }
 }
 
-// importance[b, a] += sum over heads of partial[b, h, a], in a fixed order: four lanes take every fourth head
-// each (their loads all in flight together), then the four shares are added in lane order.
-__global__ __launch_bounds__(256) void importance_reduce_kernel(ImportanceParams p) {
+// ---------------------------------------------------------------------------------------------------
+// Affixes of up to 1280 keys at head dims of 64 and 128: one pass over the scores.
+//
+// What bounds the two passes above is issue time per score (matrix product, multiply-add, exponential) and both
+// spend it.  The column sums need every row's denominator first, so one pass has to keep a row's probabilities
+// until the row is complete.  The register file of a CU can: the eight waves of a workgroup (two per SIMD, 256
+// registers each) share a head's keys, each holds its 16 * NB of them as operands (NB * D / 8 registers) and the
+// 4 * NB scores per lane of a 16-row query tile; the waves exchange (maximum, sum) per row through LDS, one barrier
+// per tile, and add the normalised probabilities to per-lane column sums.  The keys are read once per workgroup,
+// which takes the rows of several requests in turn (one workgroup per CU); the queries go straight from q to LDS by
+// the copy engine while the item before is scored, and are counter-rotated there, so the packed copy in memory and
+// its launch are gone too.  Key blocks past the eighth of a wave sit in LDS in fragment order (NBL of them), because
+// operands, scores, column sums and the query fragment have to share the 256 registers.
+//
+// LLaDA probe (16 requests x 256 rows x 1000 keys x 32 heads, relocated), all launches of the call and the zeroing
+// of the sums: 120 -> 65 us; 300 / 600 / 768 / 1200 keys: 70 / 93 / 100 / 140 -> 40 / 49 / 54 / 92 us; one request:
+// 58 -> 24 us.  Of the fused launch's 60 us 40 are the scoring loop (1.25 us per 16-row tile: 512 matrix-pipe cycles
+// and 170 vector instructions per wave, two waves per SIMD), 9 the keys on their way into registers, 5 the rotation.
+// Measured and not taken: the two waves of a SIMD at different priorities (no change); scoring a wave's keys in two
+// halves with references of their own, the first half's exponentials between the matrix instructions of the second
+// (66.5 -> 68.5 us).
+constexpr int kFusedWaves = 8;
+constexpr int kFusedThreads = 64 * kFusedWaves;
+// Query rows staged at a time: two buffers of them share the 160 KiB of LDS with the key blocks.
+constexpr int fused_stage_rows(int head_dim, int lds_key_blocks) {
+  return lds_key_blocks == 0 ? 256 : (lds_key_blocks == 2 || head_dim == 64 ? 128 : 96);
+}
+
+// Maximum / sum over the four lanes that share lane & 15 (the lane groups of one query column), in every lane.
+template <class Op>
+__device__ __forceinline__ float across_groups(float v, Op op) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  u32x2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(r.x), __uint_as_float(r.y));
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return op(__uint_as_float(r.x), __uint_as_float(r.y));
+}
+
+template <int DTYPE, int D, int NBR, int NBL>
+__global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(ImportanceParams p, int chunk_rows, int chunks,
+                                                                        int groups) {
+  constexpr int NB = NBR + NBL, KS = D / 32;
+  constexpr int TR = NB <= 5 ? 2 : 1;            // 16-row tiles per step: two where the registers allow
+  constexpr bool AHEAD = NB <= 6;                // query fragments of the next step loaded during this one, likewise
+  constexpr int STAGE_ROWS = fused_stage_rows(D, NBL);   // query rows staged at a time; chunk_rows is at most this
+  constexpr int PAIRS = D / 16;                  // (d, d + D/2) chunk pairs per row
+  constexpr int CHUNKS = D / 8;                  // 16-byte chunks per row
+  constexpr int COPY_ROWS = 64 / CHUNKS;         // rows per wave copy
+  constexpr int COPIES = STAGE_ROWS / COPY_ROWS / kFusedWaves;  // copies of a wave per item
+  static_assert(COPIES * COPY_ROWS * kFusedWaves == STAGE_ROWS, "whole copies");
+  using M = Mma<DTYPE>;
+  using G = StageGeometry<D, 16>;
+  __shared__ __attribute__((aligned(1024))) char q_stage[2][STAGE_ROWS * D * 2];
+  __shared__ __attribute__((aligned(1024))) char k_rows[NBL ? kFusedWaves * NBL * KS * 1024 : 16];
+  __shared__ __attribute__((aligned(16))) float row_max[2][16 * TR][kFusedWaves], row_sum[2][16 * TR][kFusedWaves];
+  __shared__ float row_weight[2][STAGE_ROWS];    // 1, or 0 for a row that is absent
+  __shared__ __attribute__((aligned(16))) float rope[2][2 * D];  // cos and sin row of the request's shift
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const int h = blockIdx.x % p.H, group = blockIdx.x / p.H;
+  const int kvh = h / (p.H / p.H_kv);
+  // Keys dealt evenly: every wave's blocks are full except for the last one, whose absent rows start from -inf
+  // (a masking step costs as much as the maximum, and the other waves would wait for the one that takes it).
+  const int share = p.A / kFusedWaves, spare = p.A % kFusedWaves;
+  const int a_wave = wave * share + (wave < spare ? wave : spare);
+  const int n_keys = share + (wave < spare ? 1 : 0);   // 16 * (NB - 1) <= n_keys <= 16 * NB
+  const float c = p.scale_log2e;
+
+  // One item = (request, chunk of its mask rows).  Its rows go from q to LDS by the copy engine while the item before
+  // is scored: indices first (fetch), the copies once those have arrived (issue), the rotation in LDS when the item's
+  // turn has come.  Copy j of a wave covers COPY_ROWS rows; the swizzle is applied on the global side.
+  struct Item { int m0, rows, shift; };
+  auto item_of = [&](int item) __attribute__((always_inline)) {
+    Item it{0, 0, 0};
+    if (item < p.B * chunks) {
+      const int b = item / chunks, first = (item - b * chunks) * chunk_rows;
+      request_rows(p, b, it.m0, it.rows);
+      it.m0 += first;
+      it.rows -= first;
+      it.rows = it.rows > chunk_rows ? chunk_rows : (it.rows < 0 ? 0 : it.rows);
+      it.shift = p.shifts ? p.shifts[b] : 0;
+      if (it.shift < 0 || it.shift >= p.rope_rows) it.shift = 0;
+    }
+    return it;
+  };
+  int32_t src_row[COPIES];
+  vec16 rope_part{{0, 0, 0, 0}};
+  auto fetch = [&](const Item &it) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < COPIES; ++j) {
+      const int r = (wave * COPIES + j) * COPY_ROWS + lane / CHUNKS;
+      src_row[j] = r < it.rows ? p.mask_rows[it.m0 + r] : -1;
+    }
+    if (it.shift != 0 && tid < 2 * D / 4)
+      rope_part = load16((tid < D / 4 ? p.cos_tab : p.sin_tab) + (int64_t)it.shift * D + (tid % (D / 4)) * 4);
+  };
+  auto issue = [&](const Item &it, int buf) __attribute__((always_inline)) {
+    if (it.shift != 0 && tid < 2 * D / 4) store16(rope[buf] + tid * 4, rope_part);
+#pragma unroll
+    for (int j = 0; j < COPIES; ++j) {
+      const int first = (wave * COPIES + j) * COPY_ROWS, r = first + lane / CHUNKS;
+      const bool present = src_row[j] >= 0 && src_row[j] < p.total_q;
+      const char *src = present ? p.q + src_row[j] * p.q_token_bytes + (int64_t)h * p.q_head_bytes +
+                                      (((lane % CHUNKS) ^ (r & (CHUNKS - 1))) << 4)
+                                : (const char *)kZeroRow + ((lane % CHUNKS) << 4);
+      if (first < (it.rows + 16 * TR - 1) / (16 * TR) * (16 * TR)) {  // wave-uniform: rows that some tile reads
+        lds_dma16(src, q_stage[buf] + first * D * 2);
+        if (lane % CHUNKS == 0) row_weight[buf][r] = present ? 1.0f : 0.0f;
+      }
+    }
+  };
+  Item next = item_of(group);
+  fetch(next);
+
+  // the wave's keys; past the affix they repeat the last one and their scores are masked
+  const char *k_base = p.k_cache + p.affix_slot0 * p.kv_slot_bytes + (int64_t)kvh * p.kv_head_bytes;
+  auto key_row = [&](int nt) __attribute__((always_inline)) {
+    const int a = a_wave + 16 * nt + li;
+    return k_base + (int64_t)(a < p.A ? a : p.A - 1) * p.kv_slot_bytes;
+  };
+  f32x4 absent;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) absent[i] = 16 * (NB - 1) + 4 * lg + i < n_keys ? 0.0f : -INFINITY;
+  vec16 kf[NBR][KS];
+#pragma unroll
+  for (int nt = 0; nt < NBR; ++nt) load_rows<D>(kf[nt], key_row(nt), lg);
+  issue(next, 0);  // behind the key loads: the wait for the row indices does not hold those up
+  char *const k_mine = k_rows + wave * NBL * KS * 1024 + lane * 16;
+#pragma unroll
+  for (int nt = 0; nt < NBL; ++nt) {
+    vec16 f[KS];
+    load_rows<D>(f, key_row(NBR + nt), lg);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) store16(k_mine + (nt * KS + ks) * 1024, f[ks]);
+  }
+#pragma unroll
+  for (int nt = 0; nt < NBR; ++nt)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) settle(kf[nt][ks]);
+
+  for (int item = group, turn = 0; item < p.B * chunks; item += groups, ++turn) {
+    const int stage_buf = turn & 1;
+    const Item now = next;
+    next = item_of(item + groups);
+    char *const q_rows = q_stage[stage_buf];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies of the item have landed ...
+    __syncthreads();                                    // ... and everybody's; the other buffer is no longer read
+    fetch(next);
+    const int tiles = (now.rows + 16 * TR - 1) / (16 * TR) * TR;
+    if (now.shift != 0) {
+      const int ch = tid % PAIRS;
+      float cs[16], sn[16];  // cos and sin of this thread's elements: first half of the row, second half
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        cs[j] = rope[stage_buf][ch * 8 + j];
+        cs[8 + j] = rope[stage_buf][D / 2 + ch * 8 + j];
+        sn[j] = rope[stage_buf][D + ch * 8 + j];
+        sn[8 + j] = rope[stage_buf][D + D / 2 + ch * 8 + j];
+      }
+#pragma nounroll
+      for (int r = tid / PAIRS; r < now.rows; r += kFusedThreads / PAIRS) {
+        vec16 lo = load16(q_rows + G::offset(r, ch)), hi = load16(q_rows + G::offset(r, ch + PAIRS));
+        rotate_pair_half<DTYPE>(lo, hi, cs, sn, 0, 8, -1.0f);
+        store16(q_rows + G::offset(r, ch), lo);
+        store16(q_rows + G::offset(r, ch + PAIRS), hi);
+      }
+      __syncthreads();
+    }
+    issue(next, stage_buf ^ 1);
+    float *const dst = p.partial + ((int64_t)item * p.H + h) * p.A;
+
+    float col[NB][4] = {};
+    vec16 qf[TR][KS];
+    if (AHEAD) {
+#pragma unroll
+      for (int u = 0; u < TR; ++u) load_rows_lds<D>(qf[u], q_rows, u, li, lg);
+    }
+    for (int t = 0; t < tiles; t += TR) {
+      const int buf = (t / TR) & 1;
+      f32x4 sc[TR][NB];
+      if (!AHEAD) {
+#pragma unroll
+        for (int u = 0; u < TR; ++u) load_rows_lds<D>(qf[u], q_rows, t + u, li, lg);
+      }
+#pragma unroll
+      for (int u = 0; u < TR; ++u)
+#pragma unroll
+        for (int nt = 0; nt < NB; ++nt) sc[u][nt] = nt == NB - 1 ? absent : f32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int nt = 0; nt < NB; ++nt) {
+          const vec16 k = nt < NBR ? kf[nt < NBR ? nt : 0][ks] : load16(k_mine + ((nt - NBR) * KS + ks) * 1024);
+#pragma unroll
+          for (int u = 0; u < TR; ++u) sc[u][nt] = M::run(k, qf[u][ks], sc[u][nt]);
+        }
+      if (AHEAD) {  // the next tiles' rows (past the last: rows that exist in LDS, never used)
+#pragma unroll
+        for (int u = 0; u < TR; ++u) load_rows_lds<D>(qf[u], q_rows, (t + TR + u) % (STAGE_ROWS / 16), li, lg);
+      }
+      float ref[TR];  // this wave's maximum per row; a wave without keys has -inf and probabilities of 0
+#pragma unroll
+      for (int u = 0; u < TR; ++u) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[u][nt][i]);
+        mx = across_groups(mx, [](float x, float y) { return fmaxf(x, y); }) * c;
+        ref[u] = mx;
+        mx = mx == -INFINITY ? 0.0f : mx;
+        float add[4] = {};
+#pragma unroll
+        for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            sc[u][nt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[u][nt][i], c, -mx));
+            add[i] += sc[u][nt][i];
+          }
+        const float sum = across_groups((add[0] + add[1]) + (add[2] + add[3]), [](float x, float y) { return x + y; });
+        if (lg == 0) { row_max[buf][16 * u + li][wave] = ref[u]; row_sum[buf][16 * u + li][wave] = sum; }
+      }
+      __syncthreads();  // the other buffer is free: everybody has read it before arriving here
+      // lane group lg merges waves 2 lg and 2 lg + 1, the groups meet in registers
+#pragma unroll
+      for (int u = 0; u < TR; ++u) {
+        const float2 m2 = *(const float2 *)&row_max[buf][16 * u + li][2 * lg];
+        const float2 s2 = *(const float2 *)&row_sum[buf][16 * u + li][2 * lg];
+        const float m = across_groups(fmaxf(m2.x, m2.y), [](float x, float y) { return fmaxf(x, y); });
+        const float total = across_groups(s2.x * __builtin_amdgcn_exp2f(m2.x - m) + s2.y * __builtin_amdgcn_exp2f(m2.y - m),
+                                          [](float x, float y) { return x + y; });
+        const float f = row_weight[stage_buf][16 * (t + u) + li] * (__builtin_amdgcn_exp2f(ref[u] - m) * __builtin_amdgcn_rcpf(total));
+#pragma unroll
+        for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) col[nt][i] = __builtin_fmaf(sc[u][nt][i], f, col[nt][i]);
+      }
+    }
+    int left = li == 0 ? n_keys - 4 * lg : 0;  // keys this lane stores, counted from its first
+    asm volatile("" : "+v"(left));
+#pragma unroll
+    for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = row_sum16(col[nt][i]);
+        if (16 * nt + i < left) dst[a_wave + 4 * lg + 16 * nt + i] = v;
+      }
+  }
+}
+
+// importance[b, a] += sum over the row chunks and heads of partial[b, chunk, h, a], in a fixed order: four lanes
+// take every fourth partial row each (their loads all in flight together), then the four shares are added in
+// lane order.
+__global__ __launch_bounds__(256) void importance_reduce_kernel(ImportanceParams p, int rows) {
   __shared__ float share[4][64];
   const int a = blockIdx.x * 64 + (threadIdx.x & 63);
   const int part = threadIdx.x >> 6;
   const int b = blockIdx.y;
   float acc = 0.0f;
   if (a < p.A) {
-    const float *src = p.partial + (int64_t)b * p.H * p.A + a;
+    const float *src = p.partial + (int64_t)b * rows * p.A + a;
 #pragma unroll 8
-    for (int h = part; h < p.H; h += 4) acc += src[(int64_t)h * p.A];
+    for (int r = part; r < rows; r += 4) acc += src[(int64_t)r * p.A];
   }
   share[part][threadIdx.x & 63] = acc;
   __syncthreads();
@@ -629,6 +885,54 @@ extern "C" int64_t acache_affix_importance_workspace_bytes(int64_t total_mask_ro
   (void)H_kv;
   (void)relocated;  // the packed copy of the mask queries (2-byte elements) is made with and without relocation
   return stats_bytes(total_mask_rows, H) + partial_bytes(B, H, affix_len) + total_mask_rows * H * D * 2;
+}
+
+// Launches of the one-pass form, or kNotFused when the shape is not one of its shapes.
+constexpr int kNotFused = -1000;
+constexpr int kFusedWorkgroups = 256;  // one per CU: eight waves of 256 registers fill it
+
+static int launch_fused(ImportanceParams p, int32_t dtype, int32_t D, dim3 reduce_grid, int64_t workspace_bytes,
+                        hipStream_t s) {
+  if ((D != 128 && D != 64) || p.A > 1280) return kNotFused;
+  // Work items are (request, chunk of its mask rows); `groups` workgroups per head take them in turn.  The chunk is
+  // the multiple of 16 rows with the shortest busiest workgroup, an item's own cost (staging, partial sums) being
+  // worth about 16 rows; the partial sums of all chunks have to fit the workspace.
+  int groups = kFusedWorkgroups / p.H;
+  groups = groups < 1 ? 1 : groups;
+  const int blocks = ((p.A + kFusedWaves - 1) / kFusedWaves + 15) / 16;  // 16-key blocks of the waves with most keys
+  const int stage_rows = fused_stage_rows(D, blocks > 8 ? blocks - 7 : 0);
+  int chunk_rows = 0, chunks = 0;
+  int64_t best = INT64_MAX;
+  for (int rows = 16; rows <= stage_rows; rows += 16) {
+    const int64_t n = (p.max_mask_rows + rows - 1) / rows;
+    if (n * p.B * p.H * p.A * (int64_t)sizeof(float) > workspace_bytes) continue;
+    const int used = n == 1 && p.max_mask_rows < rows ? (p.max_mask_rows + 15) / 16 * 16 : rows;
+    const int64_t span = (n * p.B + groups - 1) / groups * (used + 16);
+    if (span < best) { best = span; chunk_rows = rows; chunks = (int)n; }
+  }
+  if (chunk_rows == 0 || (int64_t)chunks * p.B > 0x7fffffffLL / 2) return kNotFused;
+  if ((int64_t)groups > (int64_t)chunks * p.B) groups = chunks * p.B;
+  p.partial = (float *)p.stats;  // the whole workspace: this form needs neither row statistics nor packed queries
+  const dim3 grid((unsigned)(p.H * groups));
+#define ACACHE_FUSED(DT, HD, NBR, NBL)                                                                        \
+  if (dtype == DT && D == HD && blocks == NBR + NBL) {                                                       \
+    hipLaunchKernelGGL((importance_fused_kernel<DT, HD, NBR, NBL>), grid, dim3(kFusedThreads), 0, s, p, chunk_rows, chunks, groups); \
+    const int rc = launch_status("importance_fused_kernel");                                                  \
+    if (rc) return rc;                                                                                        \
+    hipLaunchKernelGGL(importance_reduce_kernel, reduce_grid, dim3(256), 0, s, p, chunks * p.H);              \
+    return launch_status("importance_reduce_kernel");                                                         \
+  }
+#define ACACHE_FUSED_SIZES(DT, HD) \
+  ACACHE_FUSED(DT, HD, 1, 0) ACACHE_FUSED(DT, HD, 2, 0) ACACHE_FUSED(DT, HD, 3, 0) ACACHE_FUSED(DT, HD, 4, 0) \
+  ACACHE_FUSED(DT, HD, 5, 0) ACACHE_FUSED(DT, HD, 6, 0) ACACHE_FUSED(DT, HD, 7, 0) ACACHE_FUSED(DT, HD, 8, 0) \
+  ACACHE_FUSED(DT, HD, 7, 2) ACACHE_FUSED(DT, HD, 7, 3)
+  ACACHE_FUSED_SIZES(ACACHE_BF16, 128)
+  ACACHE_FUSED_SIZES(ACACHE_BF16, 64)
+  ACACHE_FUSED_SIZES(ACACHE_F16, 128)
+  ACACHE_FUSED_SIZES(ACACHE_F16, 64)
+#undef ACACHE_FUSED_SIZES
+#undef ACACHE_FUSED
+  return kNotFused;
 }
 
 // Argument checks and the launches; `workspace` is caller memory or this library's file-scope scratch.
@@ -695,6 +999,9 @@ static int importance_launch(
   const int row_groups_staged = (p.max_row_tiles + 4 * kRowTilesPerWave - 1) / (4 * kRowTilesPerWave);
   const dim3 grid1s((unsigned)((int64_t)B * row_groups_staged), (unsigned)H);
   const dim3 grid2s((unsigned)((affix_len + 4 * kKeysPerStep - 1) / (4 * kKeysPerStep)), (unsigned)H, (unsigned)B);
+  // One pass where a head's keys fit the registers (and LDS) of one workgroup.
+  const int fused_rc = launch_fused(p, dtype, D, grid3, workspace_bytes, s);
+  if (fused_rc != kNotFused) return fused_rc;
 #define ACACHE_CASE(DT, HD)                                                                       \
   if (dtype == DT && D == HD) {                                                                   \
     hipLaunchKernelGGL((importance_rotate_kernel<DT>), grid0, dim3(256), 0, s, p);                \
@@ -715,7 +1022,7 @@ static int importance_launch(
       const int rc2 = launch_status("importance_colsum_kernel");                                  \
       if (rc2) return rc2;                                                                        \
     }                                                                                             \
-    hipLaunchKernelGGL(importance_reduce_kernel, grid3, dim3(256), 0, s, p);                      \
+    hipLaunchKernelGGL(importance_reduce_kernel, grid3, dim3(256), 0, s, p, p.H);                 \
     return launch_status("importance_reduce_kernel");                                             \
   }
 #define ACACHE_DIMS(DT)                                                                             \

@@ -635,8 +635,8 @@ def kernel_sweep(torch, device, ops, steps):
     imp = torch.zeros(B, A, dtype=torch.float32, device=device)
     ws = torch.empty(ops.affix_importance_workspace_bytes(B * M, B, H, H, D, A, True), dtype=torch.uint8, device=device)
     us = timed(lambda: ops.affix_importance(imp, qp, kp, rows_p, cu_p, A, M, None, sh_p, cos, sin, 0, ws))
-    flops = 2 * 2 * B * M * A * H * D   # the scores are computed twice (row statistics, then column sums)
-    out.append({"kernel": "importance kernels (pack + counter-rotate queries, stats, colsum, reduce)", "us": round(us, 1),
+    flops = 2 * B * M * A * H * D
+    out.append({"kernel": "importance kernels (scores, row statistics and column sums in one pass; reduce)", "us": round(us, 1),
                 "TFLOPs": round(flops / us / 1e6, 1), "flops": flops,
                 "workload": "one layer: 16 requests x 256 mask queries x 1 000 affix keys, 32 heads x 128, bf16, relocated (shifts 1-255)"})
     logits = torch.randn(512, 126464, generator=gen, device=device).to(torch.bfloat16)

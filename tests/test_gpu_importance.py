@@ -38,6 +38,16 @@ def test_importance_matches_oracle(device, H, Hkv, D):
     _case(device, H, Hkv, D, A=203, mask_counts=[32, 0, 17, 64, 1], shifts=[0, 3, 40, 7, 0], slot0=5, seed=H)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("A,masks", [(1, [3, 1]), (7, [16, 0, 2]), (16 * 8, [17]), (16 * 8 + 1, [33, 300, 1]),
+                                     (16 * 8 * 5 + 3, [40]), (1024, [31, 65]), (1025, [20]), (1152, [9, 130]),
+                                     (1153, [97]), (1280, [16]), (1281, [16])])
+def test_affix_lengths_on_both_sides_of_the_key_block_counts(device, D, A, masks):
+    """One to eight 16-key blocks per wave in registers, two or three more in LDS, beyond that two passes; row counts
+    on both sides of a 16-row tile and of the staged rows."""
+    _case(device, 2, 1, D, A=A, mask_counts=masks, shifts=[(7 * i) % 50 for i in range(len(masks))], slot0=3, seed=A)
+
+
 def test_llada_shape_and_accumulation_over_layers(device):
     imp, want, (q, kc, rows, cu, args) = _case(device, 32, 32, 128, A=1000, mask_counts=[256, 200], shifts=[64, 255], seed=3)
     # a second call (the next layer) adds to the same buffer
