@@ -35,6 +35,7 @@ struct AttnParams {
   int32_t H_kv;
   int32_t num_tiles;  // upper bound on the number of BM-row query tiles
   int32_t head_dim;   // real head_dim (read by the padded any-head_dim variant only)
+  int32_t small_cache;  // 32-bit copy offsets reach the whole cache (read by the short-query kernel)
   int64_t num_slots;
   int64_t q_token_bytes, q_head_bytes;
   int64_t o_token_bytes, o_head_bytes;
@@ -82,7 +83,8 @@ __device__ __forceinline__ bool locate_query_tile(const int32_t *cu_q, int B, in
 // list scheduling: the short blocks fill the gaps at the end instead of the long ones sticking out.
 __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const int32_t *cu_k, int B, int BM,
                                                       int rank, int &b_out, int &q_begin, int &q_len,
-                                                      int &tile_in_request, int &kv_begin, int &kv_len) {
+                                                      int &tile_in_request, int &kv_begin, int &kv_len,
+                                                      int *live_tiles = nullptr) {
   const int lane = threadIdx.x & 63;
   // four unconditional loads at a clamped index: one memory round trip (loads under a lane mask end up in
   // separate blocks, each with its own wait)
@@ -93,11 +95,14 @@ __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const
   const int kv = lane < B ? k1 - k0 : 0;
   const int tiles = len > 0 ? (len + BM - 1) / BM : 0;
   int before = 0;  // query tiles of the requests sorted in front of this lane's request
+  int all = 0;     // and of all requests
   for (int j = 0; j < B; ++j) {
     const int kv_j = __builtin_amdgcn_readlane(kv, j);
     const int tiles_j = __builtin_amdgcn_readlane(tiles, j);
     if (kv_j > kv || (kv_j == kv && j < lane)) before += tiles_j;
+    all += tiles_j;
   }
+  if (live_tiles) *live_tiles = all;
   const uint64_t hit = __builtin_amdgcn_ballot_w64(lane < B && rank >= before && rank < before + tiles);
   if (hit == 0) return false;
   const int src = __builtin_ctzll(hit);
@@ -153,6 +158,15 @@ inline int64_t attn_grid_blocks(const AttnParams &p) {
   }
   return ((int64_t)p.num_tiles * p.H + 7) / 8 * 8;  // the XCD remap needs a multiple of 8
 }
+
+// 32-bit copy offsets when the whole cache lies within 4 GiB of a head's base and the factors fit 24 bits
+inline bool small_cache(const AttnParams &p) {
+  return p.num_slots < (1 << 24) && p.kv_slot_bytes > 0 && p.kv_slot_bytes < (1 << 24) &&
+         p.num_slots * p.kv_slot_bytes + 4096 <= 0xffffffffLL;
+}
+
+// attn_short.hip: batches of short query blocks, head dims 64 and 128.
+int short_attention(const AttnParams &p, int mode, int dtype, hipStream_t stream);
 
 // Key range of tile t: the shared range [0, shared_len) comes first in tiles of BN
 // (query-side mode only, otherwise shared_len = 0), then [shared_len, kv_len).

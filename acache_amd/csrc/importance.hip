@@ -359,13 +359,6 @@ __device__ __forceinline__ void load_rows_lds(vec16 (&f)[D / 32], const char *ti
   for (int ks = 0; ks < D / 32; ++ks) f[ks] = *(const vec16 *)(tile + G::offset(16 * t + li, 4 * ks + lg));
 }
 
-// Make the compiler finish a register-resident fragment's loads here.  Left alone it waits where the fragment is
-// first used, inside the streaming loop, with a count that knows nothing of the LDS copies in flight there: a
-// wait for "everything I issued" then also drains the copy of the next tile, every step.
-__device__ __forceinline__ void settle(const vec16 &v) {
-  asm volatile("" ::"v"(v.w[0]), "v"(v.w[1]), "v"(v.w[2]), "v"(v.w[3]));
-}
-
 // One workgroup per (request, head, 256 mask rows): wave w keeps rows 64*w .. 64*w + 63 in registers, the
 // affix keys stream through LDS 32 at a time.  Same arithmetic and the same statistic as importance_stats_kernel.
 template <int DTYPE, int D>

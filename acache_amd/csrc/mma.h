@@ -35,6 +35,13 @@ template <> struct Mma<ACACHE_F16> {
   }
 };
 
+// Make the compiler finish a register-resident fragment's loads here.  Left alone it waits where the fragment is
+// first used, inside the streaming loop, with a count that knows nothing of the LDS copies in flight there: a
+// wait for "everything I issued" then also drains the copy of the next tile, every step.
+__device__ __forceinline__ void settle(const vec16 &v) {
+  asm volatile("" ::"v"(v.w[0]), "v"(v.w[1]), "v"(v.w[2]), "v"(v.w[3]));
+}
+
 // Rotate the (lo, hi) 16-byte chunk pair of one row: elements d0..d0+7 and
 // d0+half..d0+half+7, half = head_dim / 2.  sign = +1: x*cos + rot_half(x)*sin (key side);
 // sign = -1: x*cos - rot_half(x)*sin (query side).  Rounded once to DTYPE.

@@ -1,0 +1,103 @@
+"""Attention of a few requests with short query blocks (at most 32 rows on average, one (request, head) per CU at most):
+every relocation mode against the CPU oracle, at the edges of the 32-key chunks, of a wave's register-held slots (4096
+keys) and of the 32-row query tiles (more tiles than requests run in a second turn).  Bound: 2e-2, that of the other
+attention tests (rounding of probabilities and outputs to 16 bits)."""
+import pytest
+import torch
+
+from acache_amd import ops
+from oracle import acache_oracle as O
+
+pytestmark = pytest.mark.gpu
+A, START = 40, 9      # shared rows (slots 0 .. A-1) and, in the relocation modes, private keys in front of them
+
+
+def _case(q_lens, tails, H, Hkv, D, dtype, mode, seed, holes=False):
+    g = torch.Generator().manual_seed(seed)
+    reads, nxt = [], A
+    for i, tail in enumerate(tails):
+        if tail < 0:
+            reads.append([])                                     # no keys at all
+            continue
+        a0 = START + i if mode != "plain" else 0
+        mine = list(range(nxt, nxt + a0 + tail))
+        nxt += a0 + tail
+        shared = list(range(A)) if mode != "plain" else []
+        reads.append(mine[:a0] + shared + mine[a0:] if mode == "key" else shared + mine)
+    S = 16 * (nxt // 16 + 2)
+    slots = torch.tensor(sum(reads, []), dtype=torch.int32)
+    if holes:
+        slots[5::11] = -1                                        # absent rows
+        slots[7::13] = S + 3
+    cu = lambda lens: torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    t = [(torch.randn(sum(q_lens), H, D, generator=g) / D ** 0.25).to(dtype),
+         (torch.randn(S, Hkv, D, generator=g) / D ** 0.25).to(dtype), torch.randn(S, Hkv, D, generator=g).to(dtype),
+         cu(q_lens), cu([len(r) for r in reads]), slots]
+    kw = {}
+    if mode != "plain":
+        cos, sin = O.rope_table(4400, D, 5e5)
+        kw = dict(shared_prefix_len=A, rope_cos=cos, rope_sin=sin,
+                  affix_shifts=torch.tensor([START + i for i in range(len(tails))], dtype=torch.int32))
+        if mode == "query":
+            kw["shared_kv_lens"] = torch.tensor([A if n >= 0 else 0 for n in tails], dtype=torch.int32)
+    return t, kw
+
+
+def _device_call(t, kw, device, plan=None):
+    q, kc, vc, cu_q, cu_k, slots = (x.to(device) for x in t)
+    shape = (kc.shape[0] // 16, 16, *kc.shape[1:])
+    kw = {k: v.to(device) if torch.is_tensor(v) else v for k, v in kw.items()}
+    return ops.acache_attention(q, kc.view(shape), vc.view(shape), cu_q, cu_k, slots, plan=plan, **kw).cpu()
+
+
+def _check(t, kw, device):
+    got = _device_call(t, kw, device)
+    want = O.acache_attention(*t, **kw)
+    assert torch.isfinite(got.float()).all()
+    assert (got.float() - want.float()).abs().max().item() <= 2e-2
+    return got
+
+
+@pytest.mark.parametrize("mode", ["plain", "key", "query"])
+@pytest.mark.parametrize("H,Hkv,D,dtype", [(4, 4, 128, torch.bfloat16), (7, 1, 128, torch.float16),
+                                           (6, 3, 64, torch.bfloat16), (8, 8, 64, torch.float16)])
+def test_edges_against_the_oracle(device, mode, H, Hkv, D, dtype):
+    _check(*_case([1, 16, 17, 32, 31], [1, 31, 33, 257, 223], H, Hkv, D, dtype, mode, 1), device)
+    _check(*_case([40, 33, 20], [300, 90, 64], H, Hkv, D, dtype, mode, 2), device)      # five tiles, three requests
+    _check(*_case([8, 0, 32, 4], [70, 20, -1, 0 if mode != "plain" else 1], H, Hkv, D, dtype, mode, 3), device)
+
+
+@pytest.mark.parametrize("mode", ["plain", "key", "query"])
+def test_slots_are_refilled_and_absent_rows_are_zero(device, mode):
+    _check(*_case([32], [4241], 2, 1, 128, torch.bfloat16, mode, 4), device)
+    if mode == "plain":
+        t, kw = _case([20, 32], [150, 77], 2, 2, 128, torch.bfloat16, mode, 5, holes=True)
+        present = (t[5] >= 0) & (t[5] < t[1].shape[0])
+        zero = t[1].shape[0] - 1                                 # what an absent row reads as
+        t2 = [t[0], t[1].clone(), t[2].clone(), t[3], t[4], torch.where(present, t[5], zero).to(torch.int32)]
+        t2[1][zero], t2[2][zero] = 0, 0
+        assert (_device_call(t, kw, device).float() - O.acache_attention(*t2).float()).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("mode", ["plain", "query"])
+def test_more_requests_than_one_ballot_holds(device, mode):
+    n = 70
+    _check(*_case([(5 * i) % 33 for i in range(n)], [(37 * i) % 130 + 1 for i in range(n)], 2, 2, 64, torch.bfloat16, mode,
+                  6), device)
+
+
+def test_plan_and_slot_pitch_do_not_change_the_bits(device):
+    t, kw = _case([32, 7], [190, 61], 8, 8, 128, torch.bfloat16, "plain", 7)
+    got = _check(t, kw, device)
+    plan = ops.attention_plan(t[3], t[4], 8, 8, device, slots_per_xcd=2)
+    assert torch.equal(_device_call(t, kw, device, plan), got)
+    # slots 16 MiB apart: 64-bit copy addresses
+    few = torch.arange(24, dtype=torch.int32).repeat(2)
+    cu_k = torch.tensor([0, 24, 48], dtype=torch.int32)
+    q, kc, vc = t[0].to(device), t[1][:24].to(device), t[2][:24].to(device)
+    wide = [torch.zeros(24 << 23, dtype=torch.bfloat16, device=device).as_strided((24, 8, 128), (1 << 23, 128, 1))
+            for _ in range(2)]
+    wide[0].copy_(kc)
+    wide[1].copy_(vc)
+    args = (t[3].to(device), cu_k.to(device), few.to(device))
+    assert torch.equal(ops.acache_attention(q, *wide, *args), ops.acache_attention(q, kc, vc, *args))
