@@ -322,6 +322,16 @@ int acache_block_table_slots(
     void *stream);
 
 /*
+ * The same slot map from the requests' lengths, with both prefix sums (one launch):
+ *   cu_k[b + 1] = seqlens[0] + ... + seqlens[b],  cu_q[b + 1] = (b + 1) * q_len,  cu_q[0] = cu_k[0] = 0.
+ * Slots past total_k are not written.
+ */
+int acache_decode_layout(
+    int32_t *cu_q, int32_t *cu_k, int32_t *out_slots, const int32_t *seqlens,
+    const int32_t *block_tables, int32_t B, int32_t q_len, int32_t max_blocks,
+    int32_t block_size, int64_t total_k, void *stream);
+
+/*
  * Slot layout of a batch of requests that reuse a shared affix (device-side form of
  * Sequence.finalize_slot_mapping, nano-vdllm/sequence.py:169-202, which the reference
  * evaluates per request in Python before prepare_caching_acache,
