@@ -390,10 +390,13 @@ __global__ __launch_bounds__(256, RAGGED ? 1 : 2) void varlen_attn_kernel(AttnPa
 // One query tile of one (request, head): the NW waves (4 in every instantiation; the tile geometry below is
 // written in terms of NW so that it stays in one place) take WQ = 16 * NQ16 query rows each, starting at row
 // q_tile0 of the request, and stream the request's key tiles [t_begin, t_end) through the LDS ring.
-template <int DTYPE, int D, int NQ16, int MODE, int NW = 4, bool SMALL = false, int KSPLIT = 1>
+// PAIR (with KSPLIT = 2): the two wave pairs hold the same 32 rows of two query heads, `head` and the next one, of
+// which the second exists if `heads` is 2.
+template <int DTYPE, int D, int NQ16, int MODE, int NW = 4, bool SMALL = false, int KSPLIT = 1, bool PAIR = false>
 __device__ __forceinline__ void attn_dma_part(const AttnParams &p, char *lds_k0, char *lds_v0, char *lds_k1,
-                                              char *lds_v1, float *lds_rope, int b, int q_begin, int q_len, int q_tile0,
-                                              int head, int kvh, int kv_begin, int kv_len, int t_begin, int t_end) {
+                                              char *lds_v1, float *lds_rope, int b, int q_begin, int q_len_all, int q_tile0,
+                                              int head0, int kvh, int kv_begin, int kv_len, int t_begin, int t_end,
+                                              int heads = 1) {
   constexpr int BN = 64;
   constexpr int WQ = 16 * NQ16;
   constexpr int KS = D / 32;
@@ -428,13 +431,18 @@ __device__ __forceinline__ void attn_dma_part(const AttnParams &p, char *lds_k0,
   const int lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int kp = KSPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave % KSPLIT);  // which part of a tile's keys
-  const int q_wave0 = q_tile0 + (wave / KSPLIT) * WQ;
+  static_assert(!PAIR || (KSPLIT == 2 && NW == 4), "two heads, two waves each");
+  const int which = PAIR ? __builtin_amdgcn_readfirstlane(wave / KSPLIT) : 0;
+  const int head = head0 + (which < heads ? which : 0);
+  const int q_len = which < heads ? q_len_all : 0;       // a wave without a head has no rows
+  const int q_wave0 = q_tile0 + (PAIR ? 0 : (wave / KSPLIT) * WQ);
   int nq_valid = (q_len - q_wave0 + 15) / 16;
   nq_valid = nq_valid < 0 ? 0 : (nq_valid > NQ16 ? NQ16 : nq_valid);
   char *out_base = p.out + (int64_t)q_begin * p.o_token_bytes + (int64_t)head * p.o_head_bytes;
 
   if (kv_len <= 0) {
-    for (int r = tid / CH; r < NW / KSPLIT * WQ; r += THREADS / CH) {
+    for (int r = (PAIR ? tid % (64 * KSPLIT) : tid) / CH; r < (PAIR ? 1 : NW / KSPLIT) * WQ;
+         r += (PAIR ? 64 * KSPLIT : THREADS) / CH) {
       const int qr = q_tile0 + r;
       if (qr < q_len) store16(out_base + (int64_t)qr * p.o_token_bytes + (tid % CH) * 16, vec16{{0, 0, 0, 0}});
     }
@@ -950,6 +958,53 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void varlen_attn_unit_ker
                                                 q_tile0, head, kvh, kv_begin, kv_len, 0, kt);
 }
 
+// Grouped-query batches of short query blocks: a unit is the 32-row query tile of two heads of a group, so the K/V tiles
+// that the whole group reads pass through half as many LDS rings.  Rows, operands and the order of the sums are those of
+// the key split in varlen_attn_unit_kernel: a query block of at most 64 rows has the same bits in either.
+// Measured (bf16, 28 heads over 4 KV heads, 24 requests of 32 queries and about 1 300 keys, one head / two heads per
+// unit): 43.9 / 32.5 us, relocated on the query side 62.4 / 42.6 us.
+template <int DTYPE, int D, int MODE, bool SMALL>
+__global__ __launch_bounds__(256, 2) void varlen_attn_pair_kernel(AttnParams p) {
+  constexpr int TILE_BYTES = 64 * D * 2;
+  __shared__ __attribute__((aligned(1024))) char lds[4 * TILE_BYTES + (MODE == MODE_KEY_SIDE ? 2 * D * 4 : 0)];
+  const int group = p.H / p.H_kv;
+  int rank, kvh, slice, b = 0, q_begin = 0, q_len = 0, tile = 0, kv_begin = 0, kv_len = 0;
+  if (!block_to_tile_slice(p, (group + 1) / 2, rank, kvh, slice)) return;
+  if (p.B <= 64) {
+    if (!locate_query_tile_lpt(p.cu_q, p.cu_k, p.B, 32, rank, b, q_begin, q_len, tile, kv_begin, kv_len)) return;
+  } else {
+    if (!locate_query_tile(p.cu_q, p.B, 32, rank, b, q_begin, q_len, tile)) return;
+    kv_begin = p.cu_k[b];
+    kv_len = p.cu_k[b + 1] - kv_begin;
+  }
+  const int first = 2 * slice;                // heads of the group; an odd group's last unit has one
+  // (rows past the tile belong to the next unit)
+  const int q_stop = q_len < tile * 32 + 32 ? q_len : tile * 32 + 32;
+  attn_dma_part<DTYPE, D, 2, MODE, 4, SMALL, 2, true>(
+      p, lds, lds + TILE_BYTES, lds + 2 * TILE_BYTES, lds + 3 * TILE_BYTES, reinterpret_cast<float *>(lds + 4 * TILE_BYTES),
+      b, q_begin, q_stop, tile * 32, kvh * group + first, kvh, kv_begin, kv_len, 0, sk_key_tiles<MODE>(p, b, kv_len),
+      first + 1 < group ? 2 : 1);
+}
+
+template <int DTYPE, int D>
+static int launch_pairs(const AttnParams &p0, int mode, int64_t total_q, hipStream_t stream) {
+  AttnParams p = p0;
+  p.num_tiles = (int32_t)((total_q + 31) / 32) + p.B;
+  const int64_t blocks = attn_grid_blocks(p, (p.H / p.H_kv + 1) / 2);
+  if (blocks > 0x7fffffffLL) return fail(ACACHE_E_SHAPE, "varlen_attn: grid too large");
+  const bool small = small_cache(p);
+  const dim3 grid((unsigned)blocks), block(256);
+  if (mode == MODE_QUERY_SIDE)
+    hipLaunchKernelGGL((varlen_attn_pair_kernel<DTYPE, D, MODE_QUERY_SIDE, false>), grid, block, 0, stream, p);
+  else if (mode == MODE_KEY_SIDE)
+    hipLaunchKernelGGL((varlen_attn_pair_kernel<DTYPE, D, MODE_KEY_SIDE, false>), grid, block, 0, stream, p);
+  else if (small)
+    hipLaunchKernelGGL((varlen_attn_pair_kernel<DTYPE, D, MODE_PLAIN, true>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((varlen_attn_pair_kernel<DTYPE, D, MODE_PLAIN, false>), grid, block, 0, stream, p);
+  return launch_status("varlen_attn_pair_kernel");
+}
+
 template <int DTYPE, int D, int NQ16>
 static int launch_attn(const AttnParams &p0, int mode, int64_t total_q, int64_t plan_blocks, hipStream_t stream) {
   AttnParams p = p0;
@@ -1059,6 +1114,13 @@ extern "C" int acache_varlen_attn_planned(
   if (D == 128 || D == 64) {
     p.num_tiles = B;
     if (total_q <= 32 * (int64_t)B && attn_grid_blocks(p) <= 256) return short_attention(p, mode, dtype, st);
+    // More units than the two workgroup slots of every CU: heads of a group two by two, which saves a round.  (Up to
+    // there a unit per head is faster, since half as many waves hide less latency: 16 Dream requests 33.6 us against
+    // 40.2 in pairs, 24 Dream requests 62.4 against 42.6.
+    // At head dim 64 a CU holds more units and there is no round to save: 24 requests of 32 / 8 heads 22.2 against 23.9.)
+    if (D == 128 && total_q <= 32 * (int64_t)B && H > H_kv && attn_grid_blocks(p) > 512)
+      return dtype == ACACHE_BF16 ? launch_pairs<ACACHE_BF16, 128>(p, mode, total_q, st)
+                                  : launch_pairs<ACACHE_F16, 128>(p, mode, total_q, st);
   }
 #define ACACHE_ATTN(DT, DD) \
   if (dtype == DT && D == DD) return launch_attn<DT, DD, 2>(p, mode, total_q, plan_blocks, st);

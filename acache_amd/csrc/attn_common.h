@@ -124,10 +124,11 @@ __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const
 //     order, so each of them gets the same mix of long and short tiles;
 //   otherwise heads are outermost over one linear index.
 // The grid must hold attn_grid_blocks(p) blocks.  Returns false for a block without work.
-__device__ __forceinline__ bool block_to_tile_head(const AttnParams &p, int &tile, int &kvh, int &hg) {
+// `group` is the number of units per KV head and query tile: the query heads of the KV head, or fewer for a kernel whose
+// units take several of them.
+__device__ __forceinline__ bool block_to_tile_slice(const AttnParams &p, int group, int &tile, int &kvh, int &hg) {
   const int per_xcd = gridDim.x >> 3;
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-  const int group = p.H / p.H_kv;
   if (p.H_kv % 8 == 0) {
     const int heads_per_xcd = (p.H_kv >> 3) * group;
     tile = idx / heads_per_xcd;
@@ -143,7 +144,7 @@ __device__ __forceinline__ bool block_to_tile_head(const AttnParams &p, int &til
     hg = idx % group;
   } else {
     const int w = xcd * per_xcd + idx;
-    if (w >= p.num_tiles * p.H) return false;
+    if (w >= p.num_tiles * group * p.H_kv) return false;
     hg = w % group;
     tile = (w / group) % p.num_tiles;
     kvh = w / (group * p.num_tiles);
@@ -151,13 +152,18 @@ __device__ __forceinline__ bool block_to_tile_head(const AttnParams &p, int &til
   return true;
 }
 
-inline int64_t attn_grid_blocks(const AttnParams &p) {
+__device__ __forceinline__ bool block_to_tile_head(const AttnParams &p, int &tile, int &kvh, int &hg) {
+  return block_to_tile_slice(p, p.H / p.H_kv, tile, kvh, hg);
+}
+
+inline int64_t attn_grid_blocks(const AttnParams &p, int group) {
   if (p.H_kv < 8 && 8 % p.H_kv == 0) {
     const int xcds_per_head = 8 / p.H_kv;
-    return 8 * (((int64_t)p.num_tiles + xcds_per_head - 1) / xcds_per_head) * (p.H / p.H_kv);
+    return 8 * (((int64_t)p.num_tiles + xcds_per_head - 1) / xcds_per_head) * group;
   }
-  return ((int64_t)p.num_tiles * p.H + 7) / 8 * 8;  // the XCD remap needs a multiple of 8
+  return ((int64_t)p.num_tiles * group * p.H_kv + 7) / 8 * 8;  // the XCD remap needs a multiple of 8
 }
+inline int64_t attn_grid_blocks(const AttnParams &p) { return attn_grid_blocks(p, p.H / p.H_kv); }
 
 // 32-bit copy offsets when the whole cache lies within 4 GiB of a head's base and the factors fit 24 bits
 inline bool small_cache(const AttnParams &p) {

@@ -86,6 +86,23 @@ def test_more_requests_than_one_ballot_holds(device, mode):
                   6), device)
 
 
+@pytest.mark.parametrize("mode", ["plain", "key", "query"])
+@pytest.mark.parametrize("B,H,Hkv,D,dtype", [(19, 28, 4, 128, torch.bfloat16), (18, 32, 8, 128, torch.float16),
+                                             (44, 12, 3, 128, torch.float16), (70, 10, 2, 128, torch.bfloat16)])
+def test_two_heads_of_a_group_per_unit(device, mode, B, H, Hkv, D, dtype):
+    """Grouped-query batches beyond two units per CU: odd and even groups, all three ways KV heads meet XCDs, requests
+    without queries, without keys and with more than one query tile."""
+    q_lens = [(7 * i) % 33 for i in range(B)]
+    q_lens[3], q_lens[4], q_lens[5] = 0, 70, 33
+    tails = [(29 * i) % 140 + 1 for i in range(B)]
+    tails[6] = -1
+    t, kw = _case(q_lens, tails, H, Hkv, D, dtype, mode, B)
+    assert sum(q_lens) <= 32 * B
+    got = _check(t, kw, device)
+    plan = ops.attention_plan(t[3], t[4], H, Hkv, device)
+    assert torch.equal(_device_call(t, kw, device, plan), got)
+
+
 def test_plan_and_slot_pitch_do_not_change_the_bits(device):
     t, kw = _case([32, 7], [190, 61], 8, 8, 128, torch.bfloat16, "plain", 7)
     got = _check(t, kw, device)
