@@ -884,12 +884,14 @@ extern "C" int64_t acache_affix_importance_workspace_bytes(int64_t total_mask_ro
 constexpr int kNotFused = -1000;
 constexpr int kFusedWorkgroups = 256;  // one per CU: eight waves of 256 registers fill it
 
-static int launch_fused(ImportanceParams p, int32_t dtype, int32_t D, dim3 reduce_grid, int64_t workspace_bytes,
-                        hipStream_t s) {
+static int launch_fused(ImportanceParams p, int32_t dtype, int32_t D, dim3 reduce_grid, hipStream_t s) {
   if ((D != 128 && D != 64) || p.A > 1280) return kNotFused;
+  const int64_t workspace_bytes =
+      acache_affix_importance_workspace_bytes(p.total_mask_rows, p.B, p.H, p.H_kv, D, p.A, p.shifts != nullptr);
   // Work items are (request, chunk of its mask rows); `groups` workgroups per head take them in turn.  The chunk is
   // the multiple of 16 rows with the shortest busiest workgroup, an item's own cost (staging, partial sums) being
-  // worth about 16 rows; the partial sums of all chunks have to fit the workspace.
+  // worth about 16 rows; the partial sums of all chunks have to fit the workspace that every caller has (never the
+  // one that was handed in: the order of the sums, and so the bits, would depend on its size).
   int groups = kFusedWorkgroups / p.H;
   groups = groups < 1 ? 1 : groups;
   const int blocks = ((p.A + kFusedWaves - 1) / kFusedWaves + 15) / 16;  // 16-key blocks of the waves with most keys
@@ -993,7 +995,7 @@ static int importance_launch(
   const dim3 grid1s((unsigned)((int64_t)B * row_groups_staged), (unsigned)H);
   const dim3 grid2s((unsigned)((affix_len + 4 * kKeysPerStep - 1) / (4 * kKeysPerStep)), (unsigned)H, (unsigned)B);
   // One pass where a head's keys fit the registers (and LDS) of one workgroup.
-  const int fused_rc = launch_fused(p, dtype, D, grid3, workspace_bytes, s);
+  const int fused_rc = launch_fused(p, dtype, D, grid3, s);
   if (fused_rc != kNotFused) return fused_rc;
 #define ACACHE_CASE(DT, HD)                                                                       \
   if (dtype == DT && D == HD) {                                                                   \

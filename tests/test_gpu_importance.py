@@ -110,3 +110,16 @@ def test_argument_errors(device):
         ops.affix_importance(imp, q, kc, rows, cu, 8, 2, affix_shifts=torch.zeros(1, dtype=torch.int32, device=device))
     with pytest.raises(AssertionError):
         ops.affix_importance(imp, q, kc, rows, cu, 8, 2, workspace=torch.empty(8, dtype=torch.uint8, device=device))
+
+
+@pytest.mark.parametrize("D,A,rows", [(128, 1280, 17), (64, 1200, 64), (128, 1200, 128), (128, 1000, 256)])
+def test_bits_do_not_depend_on_the_size_of_the_workspace(device, D, A, rows):
+    """A workspace of exactly the size asked for, a larger one and the library's own scratch: the same order of sums."""
+    imp, _, (q, kc, idx, cu, args) = _case(device, 32, 32, D, A=A, mask_counts=[rows], shifts=[3], seed=rows)
+    need = ops.affix_importance_workspace_bytes(rows, 1, 32, 32, D, A, True)
+    for workspace in (torch.empty(need, dtype=torch.uint8, device=device),
+                      torch.empty(4 * need + 4096, dtype=torch.uint8, device=device), "builtin"):
+        again = torch.zeros_like(imp)
+        ops.affix_importance(again, q.to(device), kc.to(device), idx.to(device), cu.to(device), A, rows, workspace=workspace,
+                             **args)
+        assert torch.equal(again, imp)
