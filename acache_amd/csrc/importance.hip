@@ -599,10 +599,11 @@ __global__ __launch_bounds__(256) void importance_colsum_lds_kernel(ImportancePa
 // its launch are gone too.  Key blocks past the eighth of a wave sit in LDS in fragment order (NBL of them), because
 // operands, scores, column sums and the query fragment have to share the 256 registers.
 //
-// LLaDA probe (16 requests x 256 rows x 1000 keys x 32 heads, relocated), all launches of the call and the zeroing
-// of the sums: 120 -> 65 us; 300 / 600 / 768 / 1200 keys: 70 / 93 / 100 / 140 -> 40 / 49 / 54 / 92 us; one request:
-// 58 -> 24 us.  Of the fused launch's 60 us 40 are the scoring loop (1.25 us per 16-row tile: 512 matrix-pipe cycles
-// and 170 vector instructions per wave, two waves per SIMD), 9 the keys on their way into registers, 5 the rotation.
+// LLaDA heads, 256 rows a request, relocated, both launches of the call, two passes / this form: 16 requests with 300 /
+// 600 / 1000 / 1100 / 1200 keys 68 / 90 / 120 / 134 / 139 -> 41 / 52 / 68 / 79 / 88 us; one request of 300 / 1000 keys
+// 33 / 55 -> 13 / 20 us.  Most of it is the scoring loop (1.25 us per 16-row tile: 512 matrix-pipe cycles and 170 vector
+// instructions per wave, two waves per SIMD), then the keys on their way into registers and the rotation.  Sums of a
+// whole chunk of up to 256 rows instead of 64 took 64 us at 1000 keys, but their order followed the batch.
 // Measured and not taken: the two waves of a SIMD at different priorities (no change); scoring a wave's keys in two
 // halves with references of their own, the first half's exponentials between the matrix instructions of the second
 // (66.5 -> 68.5 us).
@@ -610,7 +611,34 @@ constexpr int kFusedWaves = 8;
 constexpr int kFusedThreads = 64 * kFusedWaves;
 // Query rows staged at a time: two buffers of them share the 160 KiB of LDS with the key blocks.
 constexpr int fused_stage_rows(int head_dim, int lds_key_blocks) {
-  return lds_key_blocks == 0 ? 256 : (lds_key_blocks == 2 || head_dim == 64 ? 128 : 96);
+  return lds_key_blocks == 0 ? 256 : (lds_key_blocks == 2 || head_dim == 64 ? 128 : 64);
+}
+// Query rows of a request whose column sums are added up in registers before they are stored.  Rows are counted from the
+// request's first one and the stored sums are added in order, so a request's importance does not depend on the batch it is
+// scored in, whichever rows share a workgroup.
+constexpr int kSumRows = 64;
+// Sums 0 .. ceil(rows / kSumRows) - 1 of request b start at this one: a bound on what the requests in front of it need
+// that every workgroup can compute, at most total_mask_rows / kSumRows + B sums in all.
+__device__ __forceinline__ int first_sum(int m0, int b) { return m0 / kSumRows + b; }
+
+// Column sums over the 16 lanes of a row, each lane left with the N / 16 sums N / 16 * (lane & 15) + j: every step adds one
+// half of the values to the partner's and hands the other half over (partners differ in the step's bit and in all lower
+// ones), 2.8 instructions a value instead of the five and a store of a few lanes that row_sum16 takes for each.
+template <int HALF, int CTRL, int N>
+__device__ __forceinline__ void spread_step(float (&v)[N], bool upper) {
+#pragma unroll
+  for (int j = 0; j < HALF; ++j) {
+    const float keep = upper ? v[j + HALF] : v[j], give = upper ? v[j] : v[j + HALF];
+    v[j] = keep + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), CTRL, 0xf, 0xf, true));
+  }
+}
+template <int N>
+__device__ __forceinline__ void spread_row_sums(float (&v)[N], int li) {
+  static_assert(N % 16 == 0, "the halves stay whole");
+  spread_step<N / 2, 0x140>(v, (li & 8) != 0);   // lane 15 - li of the row
+  spread_step<N / 4, 0x141>(v, (li & 4) != 0);   // lane 7 - li of the half row
+  spread_step<N / 8, 0x1b>(v, (li & 2) != 0);    // lane 3 - li of the quad
+  spread_step<N / 16, 0xb1>(v, (li & 1) != 0);   // lane 1 - li of the pair
 }
 
 // Maximum / sum over the four lanes that share lane & 15 (the lane groups of one query column), in every lane.
@@ -630,6 +658,7 @@ __global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(Importa
   constexpr int TR = NB <= 5 ? 2 : 1;            // 16-row tiles per step: two where the registers allow
   constexpr bool AHEAD = NB <= 6;                // query fragments of the next step loaded during this one, likewise
   constexpr int STAGE_ROWS = fused_stage_rows(D, NBL);   // query rows staged at a time; chunk_rows is at most this
+  static_assert(kSumRows % (16 * TR) == 0 && STAGE_ROWS % kSumRows == 0, "whole steps per sum, whole sums per item");
   constexpr int PAIRS = D / 16;                  // (d, d + D/2) chunk pairs per row
   constexpr int CHUNKS = D / 8;                  // 16-byte chunks per row
   constexpr int COPY_ROWS = 64 / CHUNKS;         // rows per wave copy
@@ -658,12 +687,13 @@ __global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(Importa
   // One item = (request, chunk of its mask rows).  Its rows go from q to LDS by the copy engine while the item before
   // is scored: indices first (fetch), the copies once those have arrived (issue), the rotation in LDS when the item's
   // turn has come.  Copy j of a wave covers COPY_ROWS rows; the swizzle is applied on the global side.
-  struct Item { int m0, rows, shift; };
+  struct Item { int m0, rows, shift, sum; };
   auto item_of = [&](int item) __attribute__((always_inline)) {
-    Item it{0, 0, 0};
+    Item it{0, 0, 0, 0};
     if (item < p.B * chunks) {
-      const int b = item / chunks, first = (item - b * chunks) * chunk_rows;
+      const int b = item % p.B, first = item / p.B * chunk_rows;  // chunk by chunk: a request's last one is the short one
       request_rows(p, b, it.m0, it.rows);
+      it.sum = first_sum(it.m0, b) + first / kSumRows;
       it.m0 += first;
       it.rows -= first;
       it.rows = it.rows > chunk_rows ? chunk_rows : (it.rows < 0 ? 0 : it.rows);
@@ -756,106 +786,126 @@ __global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(Importa
       __syncthreads();
     }
     issue(next, stage_buf ^ 1);
-    float *const dst = p.partial + ((int64_t)item * p.H + h) * p.A;
+    float *dst = p.partial + ((int64_t)now.sum * p.H + h) * p.A;
 
-    float col[NB][4] = {};
     vec16 qf[TR][KS];
     if (AHEAD) {
 #pragma unroll
       for (int u = 0; u < TR; ++u) load_rows_lds<D>(qf[u], q_rows, u, li, lg);
     }
-    for (int t = 0; t < tiles; t += TR) {
-      const int buf = (t / TR) & 1;
-      f32x4 sc[TR][NB];
-      if (!AHEAD) {
+    for (int t0 = 0; t0 < tiles; t0 += kSumRows / 16) {
+      const int t_stop = t0 + kSumRows / 16 < tiles ? t0 + kSumRows / 16 : tiles;
+      float col[NB][4] = {};
+      for (int t = t0; t < t_stop; t += TR) {
+        const int buf = (t / TR) & 1;
+        f32x4 sc[TR][NB];
+        if (!AHEAD) {
 #pragma unroll
-        for (int u = 0; u < TR; ++u) load_rows_lds<D>(qf[u], q_rows, t + u, li, lg);
-      }
-#pragma unroll
-      for (int u = 0; u < TR; ++u)
-#pragma unroll
-        for (int nt = 0; nt < NB; ++nt) sc[u][nt] = nt == NB - 1 ? absent : f32x4{0, 0, 0, 0};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int nt = 0; nt < NB; ++nt) {
-          const vec16 k = nt < NBR ? kf[nt < NBR ? nt : 0][ks] : load16(k_mine + ((nt - NBR) * KS + ks) * 1024);
-#pragma unroll
-          for (int u = 0; u < TR; ++u) sc[u][nt] = M::run(k, qf[u][ks], sc[u][nt]);
+          for (int u = 0; u < TR; ++u) load_rows_lds<D>(qf[u], q_rows, t + u, li, lg);
         }
-      if (AHEAD) {  // the next tiles' rows (past the last: rows that exist in LDS, never used)
 #pragma unroll
-        for (int u = 0; u < TR; ++u) load_rows_lds<D>(qf[u], q_rows, (t + TR + u) % (STAGE_ROWS / 16), li, lg);
-      }
-      float ref[TR];  // this wave's maximum per row; a wave without keys has -inf and probabilities of 0
+        for (int u = 0; u < TR; ++u)
 #pragma unroll
-      for (int u = 0; u < TR; ++u) {
-        float mx = -INFINITY;
+          for (int nt = 0; nt < NB; ++nt) sc[u][nt] = nt == NB - 1 ? absent : f32x4{0, 0, 0, 0};
 #pragma unroll
-        for (int nt = 0; nt < NB; ++nt)
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[u][nt][i]);
-        mx = across_groups(mx, [](float x, float y) { return fmaxf(x, y); }) * c;
-        ref[u] = mx;
-        mx = mx == -INFINITY ? 0.0f : mx;
-        float add[4] = {};
+          for (int nt = 0; nt < NB; ++nt) {
+            const vec16 k = nt < NBR ? kf[nt < NBR ? nt : 0][ks] : load16(k_mine + ((nt - NBR) * KS + ks) * 1024);
 #pragma unroll
-        for (int nt = 0; nt < NB; ++nt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            sc[u][nt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[u][nt][i], c, -mx));
-            add[i] += sc[u][nt][i];
+            for (int u = 0; u < TR; ++u) sc[u][nt] = M::run(k, qf[u][ks], sc[u][nt]);
           }
-        const float sum = across_groups((add[0] + add[1]) + (add[2] + add[3]), [](float x, float y) { return x + y; });
-        if (lg == 0) { row_max[buf][16 * u + li][wave] = ref[u]; row_sum[buf][16 * u + li][wave] = sum; }
+        if (AHEAD) {  // the next tiles' rows (past the last: rows that exist in LDS, never used)
+#pragma unroll
+          for (int u = 0; u < TR; ++u) load_rows_lds<D>(qf[u], q_rows, (t + TR + u) % (STAGE_ROWS / 16), li, lg);
+        }
+        float ref[TR];  // this wave's maximum per row; a wave without keys has -inf and probabilities of 0
+#pragma unroll
+        for (int u = 0; u < TR; ++u) {
+          float mx = -INFINITY;
+#pragma unroll
+          for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[u][nt][i]);
+          mx = across_groups(mx, [](float x, float y) { return fmaxf(x, y); }) * c;
+          ref[u] = mx;
+          mx = mx == -INFINITY ? 0.0f : mx;
+          float add[4] = {};
+#pragma unroll
+          for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              sc[u][nt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[u][nt][i], c, -mx));
+              add[i] += sc[u][nt][i];
+            }
+          const float sum = across_groups((add[0] + add[1]) + (add[2] + add[3]), [](float x, float y) { return x + y; });
+          if (lg == 0) { row_max[buf][16 * u + li][wave] = ref[u]; row_sum[buf][16 * u + li][wave] = sum; }
+        }
+        __syncthreads();  // the other buffer is free: everybody has read it before arriving here
+        // lane group lg merges waves 2 lg and 2 lg + 1, the groups meet in registers
+#pragma unroll
+        for (int u = 0; u < TR; ++u) {
+          const float2 m2 = *(const float2 *)&row_max[buf][16 * u + li][2 * lg];
+          const float2 s2 = *(const float2 *)&row_sum[buf][16 * u + li][2 * lg];
+          const float m = across_groups(fmaxf(m2.x, m2.y), [](float x, float y) { return fmaxf(x, y); });
+          const float total = across_groups(s2.x * __builtin_amdgcn_exp2f(m2.x - m) + s2.y * __builtin_amdgcn_exp2f(m2.y - m),
+                                            [](float x, float y) { return x + y; });
+          const float f = row_weight[stage_buf][16 * (t + u) + li] * (__builtin_amdgcn_exp2f(ref[u] - m) * __builtin_amdgcn_rcpf(total));
+#pragma unroll
+          for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) col[nt][i] = __builtin_fmaf(sc[u][nt][i], f, col[nt][i]);
+        }
       }
-      __syncthreads();  // the other buffer is free: everybody has read it before arriving here
-      // lane group lg merges waves 2 lg and 2 lg + 1, the groups meet in registers
+      constexpr int OWN = (NB + 3) / 4;  // sums a lane stores: key 16 * (n / 4) + 4 * lg + n % 4 for n = OWN * li + j
+      float sums[16 * OWN];
 #pragma unroll
-      for (int u = 0; u < TR; ++u) {
-        const float2 m2 = *(const float2 *)&row_max[buf][16 * u + li][2 * lg];
-        const float2 s2 = *(const float2 *)&row_sum[buf][16 * u + li][2 * lg];
-        const float m = across_groups(fmaxf(m2.x, m2.y), [](float x, float y) { return fmaxf(x, y); });
-        const float total = across_groups(s2.x * __builtin_amdgcn_exp2f(m2.x - m) + s2.y * __builtin_amdgcn_exp2f(m2.y - m),
-                                          [](float x, float y) { return x + y; });
-        const float f = row_weight[stage_buf][16 * (t + u) + li] * (__builtin_amdgcn_exp2f(ref[u] - m) * __builtin_amdgcn_rcpf(total));
+      for (int n = 0; n < 16 * OWN; ++n) sums[n] = n < 4 * NB ? col[n < 4 * NB ? n / 4 : 0][n % 4] : 0.0f;
+      int own = lane;  // opaque: what follows is computed here, not kept in registers across the tiles
+      asm volatile("" : "+v"(own));
+      spread_row_sums(sums, own & 15);
 #pragma unroll
-        for (int nt = 0; nt < NB; ++nt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) col[nt][i] = __builtin_fmaf(sc[u][nt][i], f, col[nt][i]);
+      for (int j = 0; j < OWN; ++j) {
+        const int n = OWN * (own & 15) + j, a = 16 * (n / 4) + 4 * (own >> 4) + n % 4;
+        if (a < n_keys) dst[a_wave + a] = sums[j];
       }
+      dst += (int64_t)p.H * p.A;
     }
-    int left = li == 0 ? n_keys - 4 * lg : 0;  // keys this lane stores, counted from its first
-    asm volatile("" : "+v"(left));
-#pragma unroll
-    for (int nt = 0; nt < NB; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float v = row_sum16(col[nt][i]);
-        if (16 * nt + i < left) dst[a_wave + 4 * lg + 16 * nt + i] = v;
-      }
   }
 }
 
-// importance[b, a] += sum over the row chunks and heads of partial[b, chunk, h, a], in a fixed order: four lanes
-// take every fourth partial row each (their loads all in flight together), then the four shares are added in
-// lane order.
-__global__ __launch_bounds__(256) void importance_reduce_kernel(ImportanceParams p, int rows) {
-  __shared__ float share[4][64];
+// importance[b, a] += sum over the row sums of request b and the heads of partial[sum, h, a], in a fixed order: PARTS
+// lanes take every PARTS-th partial row each (their loads all in flight together), then the shares are added in lane
+// order.  ROW_SUMS: one sum per kSumRows rows (the one-pass form), otherwise one per request.  The chain of a lane's loads
+// is what the launch takes: sixteen lanes in the one-pass form (four: 0.5 to 1 us more a call for one or two requests).
+template <int PARTS, bool ROW_SUMS>
+__global__ __launch_bounds__(64 * PARTS) void importance_reduce_kernel(ImportanceParams p) {
+  __shared__ float share[PARTS][64];
   const int a = blockIdx.x * 64 + (threadIdx.x & 63);
   const int part = threadIdx.x >> 6;
   const int b = blockIdx.y;
   float acc = 0.0f;
+  int first = b, sums = 1;
+  if (ROW_SUMS) {
+    int m0, n_rows;
+    request_rows(p, b, m0, n_rows);
+    first = first_sum(m0, b);
+    sums = (n_rows + kSumRows - 1) / kSumRows;
+  }
+  const int rows = sums * p.H;
   if (a < p.A) {
-    const float *src = p.partial + (int64_t)b * rows * p.A + a;
+    const float *src = p.partial + (int64_t)first * p.H * p.A + a;
 #pragma unroll 8
-    for (int r = part; r < rows; r += 4) acc += src[(int64_t)r * p.A];
+    for (int r = part; r < rows; r += PARTS) acc += src[(int64_t)r * p.A];
   }
   share[part][threadIdx.x & 63] = acc;
   __syncthreads();
   if (part == 0 && a < p.A) {
-    const int j = threadIdx.x;
-    p.importance[(int64_t)b * p.imp_stride + a] += ((share[0][j] + share[1][j]) + share[2][j]) + share[3][j];
+    float *dst = p.importance + (int64_t)b * p.imp_stride + a;
+    float total = share[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < PARTS; ++w) total += share[w][threadIdx.x];
+    *dst += total;
   }
 }
 
@@ -886,26 +936,25 @@ constexpr int kFusedWorkgroups = 256;  // one per CU: eight waves of 256 registe
 
 static int launch_fused(ImportanceParams p, int32_t dtype, int32_t D, dim3 reduce_grid, hipStream_t s) {
   if ((D != 128 && D != 64) || p.A > 1280) return kNotFused;
-  const int64_t workspace_bytes =
-      acache_affix_importance_workspace_bytes(p.total_mask_rows, p.B, p.H, p.H_kv, D, p.A, p.shifts != nullptr);
   // Work items are (request, chunk of its mask rows); `groups` workgroups per head take them in turn.  The chunk is
-  // the multiple of 16 rows with the shortest busiest workgroup, an item's own cost (staging, partial sums) being
-  // worth about 16 rows; the partial sums of all chunks have to fit the workspace that every caller has (never the
-  // one that was handed in: the order of the sums, and so the bits, would depend on its size).
+  // the multiple of the rows per sum with the shortest busiest workgroup, an item's own cost (staging, partial sums)
+  // being worth about 16 rows.
   int groups = kFusedWorkgroups / p.H;
   groups = groups < 1 ? 1 : groups;
   const int blocks = ((p.A + kFusedWaves - 1) / kFusedWaves + 15) / 16;  // 16-key blocks of the waves with most keys
   const int stage_rows = fused_stage_rows(D, blocks > 8 ? blocks - 7 : 0);
+  // The partial sums (total_mask_rows / kSumRows + B of them at most, per head) fit what the other form takes for its
+  // statistics, partial sums and packed queries: a row's share of a sum is no more than its statistic and query.
+  static_assert(1280 * 4 / kSumRows <= 4 + 2 * 64, "partial sums fit the workspace");
   int chunk_rows = 0, chunks = 0;
   int64_t best = INT64_MAX;
-  for (int rows = 16; rows <= stage_rows; rows += 16) {
-    const int64_t n = (p.max_mask_rows + rows - 1) / rows;
-    if (n * p.B * p.H * p.A * (int64_t)sizeof(float) > workspace_bytes) continue;
-    const int used = n == 1 && p.max_mask_rows < rows ? (p.max_mask_rows + 15) / 16 * 16 : rows;
+  for (int rows = kSumRows; rows <= stage_rows; rows += kSumRows) {
+    const int64_t n = (p.max_mask_rows + (int64_t)rows - 1) / rows;
+    const int64_t used = (p.max_mask_rows + 16 * n - 1) / (16 * n) * 16;  // on average: a request's last chunk is shorter
     const int64_t span = (n * p.B + groups - 1) / groups * (used + 16);
     if (span < best) { best = span; chunk_rows = rows; chunks = (int)n; }
   }
-  if (chunk_rows == 0 || (int64_t)chunks * p.B > 0x7fffffffLL / 2) return kNotFused;
+  if ((int64_t)chunks * p.B > 0x7fffffffLL / 2) return kNotFused;
   if ((int64_t)groups > (int64_t)chunks * p.B) groups = chunks * p.B;
   p.partial = (float *)p.stats;  // the whole workspace: this form needs neither row statistics nor packed queries
   const dim3 grid((unsigned)(p.H * groups));
@@ -914,7 +963,7 @@ static int launch_fused(ImportanceParams p, int32_t dtype, int32_t D, dim3 reduc
     hipLaunchKernelGGL((importance_fused_kernel<DT, HD, NBR, NBL>), grid, dim3(kFusedThreads), 0, s, p, chunk_rows, chunks, groups); \
     const int rc = launch_status("importance_fused_kernel");                                                  \
     if (rc) return rc;                                                                                        \
-    hipLaunchKernelGGL(importance_reduce_kernel, reduce_grid, dim3(256), 0, s, p, chunks * p.H);              \
+    hipLaunchKernelGGL((importance_reduce_kernel<16, true>), reduce_grid, dim3(1024), 0, s, p);               \
     return launch_status("importance_reduce_kernel");                                                         \
   }
 #define ACACHE_FUSED_SIZES(DT, HD) \
@@ -1017,7 +1066,7 @@ static int importance_launch(
       const int rc2 = launch_status("importance_colsum_kernel");                                  \
       if (rc2) return rc2;                                                                        \
     }                                                                                             \
-    hipLaunchKernelGGL(importance_reduce_kernel, grid3, dim3(256), 0, s, p, p.H);                 \
+    hipLaunchKernelGGL((importance_reduce_kernel<4, false>), grid3, dim3(256), 0, s, p);          \
     return launch_status("importance_reduce_kernel");                                             \
   }
 #define ACACHE_DIMS(DT)                                                                             \

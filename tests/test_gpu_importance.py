@@ -123,3 +123,18 @@ def test_bits_do_not_depend_on_the_size_of_the_workspace(device, D, A, rows):
         ops.affix_importance(again, q.to(device), kc.to(device), idx.to(device), cu.to(device), A, rows, workspace=workspace,
                              **args)
         assert torch.equal(again, imp)
+
+
+@pytest.mark.parametrize("H,Hkv,D,A,batch", [(32, 32, 128, 1000, [256] * 15), (32, 32, 128, 1200, [224] + [7, 256] * 3),
+                                             (28, 4, 128, 300, [130, 0] + [64] * 20), (32, 8, 64, 1100, [200, 256, 65, 1])])
+def test_a_request_has_the_same_bits_alone_and_in_a_batch(device, H, Hkv, D, A, batch):
+    """Rows are summed in groups counted from the request's first row, whichever requests share the call."""
+    shifts = [(11 * i) % 60 for i in range(len(batch))]
+    imp, _, (q, kc, rows, cu, args) = _case(device, H, Hkv, D, A=A, mask_counts=batch, shifts=shifts, seed=A)
+    at = cu.tolist()
+    for first, last in ((0, 1), (1, 3), (len(batch) - 1, len(batch))):
+        part = torch.zeros(last - first, A + 3, device=device)
+        some = dict(args, affix_shifts=args["affix_shifts"][first:last])
+        ops.affix_importance(part, q.to(device), kc.to(device), rows[at[first]:at[last]].to(device),
+                             (cu[first:last + 1] - cu[first]).to(device), A, max(1, max(batch[first:last])), **some)
+        assert torch.equal(part, imp[first:last])
