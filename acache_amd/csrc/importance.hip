@@ -669,7 +669,7 @@ __global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(Importa
   __shared__ __attribute__((aligned(1024))) char q_stage[2][STAGE_ROWS * D * 2];
   __shared__ __attribute__((aligned(1024))) char k_rows[NBL ? kFusedWaves * NBL * KS * 1024 : 16];
   __shared__ __attribute__((aligned(16))) float row_max[2][16 * TR][kFusedWaves], row_sum[2][16 * TR][kFusedWaves];
-  __shared__ float row_weight[2][STAGE_ROWS];    // 1, or 0 for a row that is absent
+  __shared__ float row_present[2][STAGE_ROWS];   // 1, or 0 for a row that is absent
   __shared__ __attribute__((aligned(16))) float rope[2][2 * D];  // cos and sin row of the request's shift
 
   const int tid = threadIdx.x;
@@ -724,7 +724,7 @@ __global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(Importa
                                 : (const char *)kZeroRow + ((lane % CHUNKS) << 4);
       if (first < (it.rows + 16 * TR - 1) / (16 * TR) * (16 * TR)) {  // wave-uniform: rows that some tile reads
         lds_dma16(src, q_stage[buf] + first * D * 2);
-        if (lane % CHUNKS == 0) row_weight[buf][r] = present ? 1.0f : 0.0f;
+        if (lane % CHUNKS == 0) row_present[buf][r] = present ? 1.0f : 0.0f;
       }
     }
   };
@@ -850,7 +850,17 @@ __global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(Importa
           const float m = across_groups(fmaxf(m2.x, m2.y), [](float x, float y) { return fmaxf(x, y); });
           const float total = across_groups(s2.x * __builtin_amdgcn_exp2f(m2.x - m) + s2.y * __builtin_amdgcn_exp2f(m2.y - m),
                                             [](float x, float y) { return x + y; });
-          const float f = row_weight[stage_buf][16 * (t + u) + li] * (__builtin_amdgcn_exp2f(ref[u] - m) * __builtin_amdgcn_rcpf(total));
+          float f = __builtin_amdgcn_exp2f(ref[u] - m) * __builtin_amdgcn_rcpf(total);
+          // An absent row is a zero query: against an infinite key its scores are not numbers, and a factor of 0 would not
+          // keep them out.
+          const bool present = row_present[stage_buf][16 * (t + u) + li] != 0.0f;
+          if (__builtin_amdgcn_ballot_w64(!present) != 0) {
+            f = present ? f : 0.0f;
+#pragma unroll
+            for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) sc[u][nt][i] = present ? sc[u][nt][i] : 0.0f;
+          }
 #pragma unroll
           for (int nt = 0; nt < NB; ++nt)
 #pragma unroll

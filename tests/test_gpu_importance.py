@@ -138,3 +138,24 @@ def test_a_request_has_the_same_bits_alone_and_in_a_batch(device, H, Hkv, D, A, 
         ops.affix_importance(part, q.to(device), kc.to(device), rows[at[first]:at[last]].to(device),
                              (cu[first:last + 1] - cu[first]).to(device), A, max(1, max(batch[first:last])), **some)
         assert torch.equal(part, imp[first:last])
+
+
+@pytest.mark.parametrize("D,A", [(128, 90), (128, 700), (128, 1200), (64, 1100)])
+def test_infinite_key_and_absent_rows(device, D, A):
+    """A key with an infinite element that every live query scores at -inf weighs nothing; absent rows and the rows that fill
+    up the last tile are zero queries, whose scores against it are no numbers, and must not reach any sum."""
+    g = torch.Generator().manual_seed(A)
+    H, n = 4, 20
+    q = (torch.randn(40, H, D, generator=g) / D ** 0.25).to(torch.bfloat16)
+    kc = (torch.randn(A, H, D, generator=g) / D ** 0.25).to(torch.bfloat16)
+    q[..., 5] = q[..., 5].abs() + 0.5
+    kc[17, :, 5] = float("-inf")
+    rows = torch.arange(n, dtype=torch.int32)
+    rows[[3, 11]] = torch.tensor([-1, 400], dtype=torch.int32)
+    got = torch.zeros(1, A, device=device)
+    ops.affix_importance(got, q.to(device), kc.to(device), rows.to(device), torch.tensor([0, n], dtype=torch.int32, device=device),
+                         A, n)
+    live = [r for r in range(n) if r not in (3, 11)]
+    s = torch.einsum("rhd,ahd->rha", q[live].float(), kc.float()) * D ** -0.5
+    want = torch.softmax(s, -1).sum((0, 1))
+    assert want[17] == 0 and torch.allclose(got.cpu()[0], want, rtol=2e-3, atol=1e-4)
