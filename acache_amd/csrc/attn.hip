@@ -639,6 +639,9 @@ __device__ __forceinline__ void attn_dma_part(const AttnParams &p, char *lds_k0,
       }
     };
     copy_point(0);
+    // A wave whose part of the tile holds no key leaves its state as it is: a first tile without keys would move the
+    // reference to 0, where it would stay above scores far below 0 (copies go out at point 0 with a key split).
+    if (KSPLIT == 2 && MASKED && n_valid <= kp * (BN / KSPLIT)) return;
     __builtin_amdgcn_s_setprio(1);
     scores(qf);
     // Issue order of this region: K fragments are read four fragments (eight matrix
@@ -821,7 +824,7 @@ __device__ __forceinline__ void attn_dma_part(const AttnParams &p, char *lds_k0,
   // ---- key split: the odd wave of a pair hands its partial state to the even one ---------------
   // Both waves hold the same queries in the same lanes, so the merge is lane-local.  The odd wave parks O (fp32,
   // in register order: exactly one ring buffer) in its own output-staging buffer and (reference, denominator)
-  // at the end of its partner's; a wave that never saw a key (requests of at most 32 keys) reports -inf.
+  // at the end of its partner's; a wave that never saw a key still has the reference -inf and weighs 0.
   if constexpr (KSPLIT == 2) {
     static_assert(NQ16 * DT * 64 * 16 <= TILE_BYTES, "a wave's partial O must fit one ring buffer");
     f32x4 *xo = reinterpret_cast<f32x4 *>(lds_k0 + (wave | 1) * TILE_BYTES);
@@ -833,7 +836,7 @@ __device__ __forceinline__ void attn_dma_part(const AttnParams &p, char *lds_k0,
       for (int qt = 0; qt < NQ16; ++qt) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) xo[(qt * DT + dt) * 64 + lane] = o_acc[qt][dt];
-        xml[(2 * qt) * 64 + lane] = kv_len > BN / KSPLIT ? m_run[qt] : -INFINITY;
+        xml[(2 * qt) * 64 + lane] = m_run[qt];
         xml[(2 * qt + 1) * 64 + lane] = l_acc[qt][0];
       }
     }

@@ -118,3 +118,28 @@ def test_plan_and_slot_pitch_do_not_change_the_bits(device):
     wide[1].copy_(vc)
     args = (t[3].to(device), cu_k.to(device), few.to(device))
     assert torch.equal(ops.acache_attention(q, *wide, *args), ops.acache_attention(q, kc, vc, *args))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("logit", [-20.0, -100.0])
+@pytest.mark.parametrize("shared", [1, 31, 32, 33])
+@pytest.mark.parametrize("H,Hkv,q_lens", [(4, 2, [40, 64]), (4, 2, [16, 64]), (28, 4, [32] * 19), (4, 2, [32, 32])])
+def test_few_shared_keys_and_scores_far_below_zero(device, H, Hkv, q_lens, shared, logit, dtype):
+    """Query-side relocation whose shared range ends inside the first half of its tile: the waves that take the second half
+    of a tile's keys have none there, and later keys that all score near `logit`.  32 and 64 rows with the key split of
+    a per-head unit, of two heads per unit, and wave-private chunks.  A softmax does not know such an offset: 2e-2 as above."""
+    D, g = 128, torch.Generator().manual_seed(shared)
+    level = (-logit / D ** 0.5) ** 0.5
+    kv = [shared + 70 + i for i in range(len(q_lens))]
+    S = shared + sum(kv)
+    q = (level + 0.3 * torch.randn(sum(q_lens), H, D, generator=g)).to(dtype)
+    kc = (-level + 0.3 * torch.randn(S + 16 - S % 16, Hkv, D, generator=g)).to(dtype)
+    vc = torch.randn(kc.shape, generator=g).to(dtype)
+    own = iter(range(shared, S))
+    slots = torch.tensor([s for n in kv for s in list(range(shared)) + [next(own) for _ in range(n - shared)]], dtype=torch.int32)
+    cu = lambda lens: torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    cos, sin = O.rope_table(64, D, 5e5)
+    B = len(q_lens)
+    _check([q, kc, vc, cu(q_lens), cu(kv), slots],
+           dict(shared_prefix_len=shared, rope_cos=cos, rope_sin=sin, affix_shifts=torch.zeros(B, dtype=torch.int32),
+                shared_kv_lens=torch.full((B,), shared, dtype=torch.int32)), device)
