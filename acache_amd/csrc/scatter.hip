@@ -95,7 +95,9 @@ __global__ __launch_bounds__(256) void decode_layout_kernel(int32_t *cu_q, int32
   if (blockIdx.x == 0 && tid == 0) {
     if (b == 0) cu_q[0] = cu_k[0] = 0;
     cu_q[b + 1] = (b + 1) * q_len;
-    cu_k[b + 1] = start + len;
+    // never past the slot map, which the readers of cu_k index without another check
+    const int64_t end = (int64_t)start + len;
+    cu_k[b + 1] = (int32_t)(end < 0 ? 0 : (end > total_k ? total_k : end));
   }
   for (int n = blockIdx.x * 256 + tid; n < len; n += gridDim.x * 256) {
     if (start + n < 0 || start + n >= total_k) break;  // lengths that sum to more than the caller said

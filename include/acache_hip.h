@@ -324,7 +324,7 @@ int acache_block_table_slots(
 /*
  * The same slot map from the requests' lengths, with both prefix sums (one launch):
  *   cu_k[b + 1] = seqlens[0] + ... + seqlens[b],  cu_q[b + 1] = (b + 1) * q_len,  cu_q[0] = cu_k[0] = 0.
- * Slots past total_k are not written.
+ * Lengths that sum to more than total_k are cut there: slots past it are not written and cu_k does not exceed it.
  */
 int acache_decode_layout(
     int32_t *cu_q, int32_t *cu_k, int32_t *out_slots, const int32_t *seqlens,

@@ -40,6 +40,14 @@ def test_equals_scan_and_slot_map(device, B, longest, bs):
         assert cut[total - 1:].tolist() == [-9] * 6
 
 
+def test_lengths_beyond_the_slot_map_are_cut(device):
+    """No reader of cu_k gets past the slots that exist, whatever the lengths on the device say."""
+    lens = torch.tensor([5, 9, 3, 4], dtype=torch.int32)
+    tables = torch.arange(8, dtype=torch.int32).view(4, 2)
+    for total, want in ((21, [0, 5, 14, 17, 21]), (14, [0, 5, 14, 14, 14]), (8, [0, 5, 8, 8, 8]), (0, [0, 0, 0, 0, 0])):
+        assert _layout(lens, tables, 2, 8, total, device)[1].tolist() == want
+
+
 @pytest.mark.parametrize("known", [True, False])
 def test_batched_decode_attention_equals_the_ragged_call(device, known):
     g = torch.Generator(device=device).manual_seed(3)
