@@ -747,20 +747,28 @@ def baseline_decode_attention(
     if softmax_scale is None:
         softmax_scale = head_dim ** -0.5
     seqlens = _i32(seqlens, "seqlens")
-    assert seqlens.numel() == batch
-    if total_k is None:
-        total_k = int(seqlens.sum().item())
-    tables = _i32(block_tables, "block_tables")
-    assert tables.dim() == 2 and tables.shape[0] >= batch
-    cu_q = torch.empty(batch + 1, dtype=torch.int32, device=q.device)
-    cu_k = torch.empty(batch + 1, dtype=torch.int32, device=q.device)
-    slots = torch.empty(int(total_k), dtype=torch.int32, device=q.device)
-    lib = _lib.load()
-    with torch.cuda.device(q.device):
-        rc = lib.acache_decode_layout(
-            _ptr(cu_q), _ptr(cu_k), _ptr(slots), _ptr(seqlens), _ptr(tables), batch, query_len, tables.shape[1],
-            k_cache.shape[1], int(total_k), _stream(q))
-    _lib.check(rc, "decode_layout")
+    if seqlens.numel() == batch and 0 < batch <= 65535 and query_len > 0 and block_tables.dim() == 2:
+        if total_k is None:
+            total_k = int(seqlens.sum().item())
+        seqlens, tables = seqlens.to(q.device), _i32(block_tables, "block_tables").to(q.device)
+        if tables.shape[0] < batch:  # requests without a row have no blocks
+            tables = torch.nn.functional.pad(tables, (0, 0, 0, batch - tables.shape[0]), value=-1)
+        cu_q = torch.empty(batch + 1, dtype=torch.int32, device=q.device)
+        cu_k = torch.empty(batch + 1, dtype=torch.int32, device=q.device)
+        slots = torch.empty(int(total_k), dtype=torch.int32, device=q.device)
+        lib = _lib.load()
+        with torch.cuda.device(q.device):
+            rc = lib.acache_decode_layout(
+                _ptr(cu_q), _ptr(cu_k), _ptr(slots), _ptr(seqlens), _ptr(tables), batch, query_len, tables.shape[1],
+                k_cache.shape[1], int(total_k), _stream(q))
+        _lib.check(rc, "decode_layout")
+    else:  # nothing to lay out, more requests than one launch covers, or lengths that broadcast
+        cu_k = torch.zeros(batch + 1, dtype=torch.int32, device=q.device)
+        cu_k[1:] = torch.cumsum(seqlens, 0)
+        if total_k is None:
+            total_k = int(cu_k[-1].item())
+        cu_q = torch.arange(0, (batch + 1) * query_len, query_len, dtype=torch.int32, device=q.device)
+        slots = block_table_slots(block_tables, cu_k, k_cache.shape[1], total_k)
     q3 = q.reshape(batch * query_len, num_heads, head_dim)
     out = _varlen_attn(q3, k_cache, v_cache, cu_q, cu_k, slots, softmax_scale, 0, None, None, None, None)
     return out.view(batch, query_len, num_heads, head_dim)

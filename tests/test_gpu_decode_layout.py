@@ -60,3 +60,23 @@ def test_batched_decode_attention_equals_the_ragged_call(device, known):
     cu = lambda lens: torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=device)
     want = ops.baseline_ragged_attention(q.flatten(0, 1), k, v, cu([32] * 3), cu(seqlens), tables)
     assert torch.equal(got.flatten(0, 1), want)
+
+
+def test_calls_that_the_layout_launch_does_not_cover(device):
+    """A table without rows for trailing requests that have no keys, or with more rows than requests; one length for a batch
+    (a prefix sum that broadcasts: the first request has the keys); no requests; no query rows."""
+    g = torch.Generator(device=device).manual_seed(4)
+    q = torch.randn(3, 4, 4, 128, generator=g, device=device).to(torch.bfloat16)
+    k, v = (torch.randn(8, 16, 4, 128, generator=g, device=device).to(torch.bfloat16) for _ in range(2))
+    tables = torch.tensor([[5, 2], [0, -1], [7, 1], [3, 4]], dtype=torch.int32, device=device)
+    lens = lambda *n: torch.tensor(n, device=device)
+    full = ops.baseline_decode_attention(q, k, v, lens(20, 9, 0), tables[:3])
+    assert torch.equal(ops.baseline_decode_attention(q, k, v, lens(20, 9, 0), tables[:2]), full)
+    assert torch.equal(ops.baseline_decode_attention(q, k, v, lens(20, 9, 0), tables), full)
+    assert torch.equal(full[0], ops.baseline_decode_attention(q[:1], k, v, lens(20), tables[:1])[0])
+    assert not full[2].any()
+    one = ops.baseline_decode_attention(q, k, v, lens(20), tables[:3])
+    assert torch.equal(one[0], full[0]) and not one[1:].any()
+    assert ops.baseline_decode_attention(q[:0], k, v, lens()[:0], tables[:0]).shape == (0, 4, 4, 128)
+    with pytest.raises(RuntimeError):
+        ops.baseline_decode_attention(q[:, :0], k, v, lens(20, 9, 0), tables[:3])
