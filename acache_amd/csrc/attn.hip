@@ -1058,6 +1058,46 @@ static int launch_attn_any_head_dim(const AttnParams &p0, int mode, int64_t tota
   return launch_status("varlen_attn_kernel (any head_dim)");
 }
 
+// Which batches of short query blocks (32 rows per request on average at most) leave the per-head units of launch_attn.
+// Their plan, if any, is not needed.  The lengths are on the device: the host knows totals only.
+
+// Wave-private key chunks (attn_short.hip), a unit of 32 query rows per CU; sets p.num_tiles to the tiles of its grid.
+// Measured as time against the per-head units (bf16, blocks of 1, 16 and 32 rows, 1 to 8 LLaDA and Dream requests and 4 to
+// 128 requests of 8 and 2 heads, private keys and three quarters shared; up to 128 (request, KV head) streams):
+//   keys per request       200           512           768           1100          2000
+//   D 128, plain           1.01 to 1.25  0.93 to 1.14  0.86 to 1.06  0.79 to 0.96  0.73 to 0.90
+//   D 128, key side        1.08 to 1.33  0.95 to 1.09  0.86 to 0.97  0.78 to 0.93  0.73 to 0.86
+//   D 128, query side      1.06 to 1.23  0.94 to 1.04  0.84 to 0.93  0.77 to 0.86  0.57 to 0.74
+//   D 64                   0.92 to 1.15  0.83 to 0.99  0.77 to 0.89  0.68 to 0.78  0.53 to 0.72
+// (the eight waves' set-up and merge against a chain of short tiles).  More streams than that are bound by memory where the
+// keys are private: plain 0.87 to 1.18 and key side 0.84 to 1.04 at 1100 keys, but query side 0.78 to 0.87.
+// A request of more than 32 rows is several units.  They all fit the CUs if even the worst lengths do (two LLaDA requests
+// of 33 and 31 rows and 1300 keys: 24.5 us in per-head units, 30.3 with units in two turns, 18.8 in one).  Beyond that the
+// grid has a unit per request and head, further ones wait (8 Dream requests of 33 and 31 rows: 25.1 / 32.1 us), and the
+// batch has to look like blocks of one length, which is what refinement steps are.
+static bool takes_short_kernel(AttnParams &p, int mode, int64_t total_q, int64_t total_k) {
+  const int64_t B = p.B;
+  if ((p.head_dim != 128 && p.head_dim != 64) || total_q > 32 * B) return false;
+  if (total_k < B * (p.head_dim == 64 ? 512 : mode == MODE_PLAIN ? 1024 : 768)) return false;
+  if (p.head_dim == 128 && mode != MODE_QUERY_SIDE && B * p.H_kv > 128) return false;
+  p.num_tiles = (int32_t)((total_q + 31 * B) / 32);
+  if (attn_grid_blocks(p) <= 256) return true;
+  p.num_tiles = p.B;
+  return total_q % B == 0 && attn_grid_blocks(p) <= 256;
+}
+
+// Two heads of a group per unit: where a unit per head is more than the two workgroup slots of every CU, which saves a
+// round.  (Up to there a unit per head is faster, since half as many waves hide less latency: 16 Dream requests 33.6 us
+// against 40.2 in pairs, 24 Dream requests 62.4 against 42.6.  Blocks of 1 to 32 rows, 40 to 1300 keys, groups of 2 to 7:
+// 0.61 to 1.0 times the per-head units, 0.79 on average.  A long request among short ones is cut into 32-row tiles instead
+// of 128-row ones, 1.05 to 1.23 times, so the batch has to look like blocks of one length.
+// At head dim 64 a CU holds more units and there is no round to save: 24 requests of 32 / 8 heads 22.2 against 23.9.)
+static bool takes_pair_kernel(AttnParams &p, int64_t total_q) {
+  if (p.head_dim != 128 || total_q > 32 * (int64_t)p.B || total_q % p.B != 0 || p.H == p.H_kv) return false;
+  p.num_tiles = p.B;
+  return attn_grid_blocks(p) > 512;
+}
+
 }  // namespace acache
 
 using namespace acache;
@@ -1110,21 +1150,10 @@ extern "C" int acache_varlen_attn_planned(
   const int mode = query_side ? MODE_QUERY_SIDE : (relocate ? MODE_KEY_SIDE : MODE_PLAIN);
   hipStream_t st = (hipStream_t)stream;
   p.small_cache = 0;
-  // Short query blocks, few of them: at most 32 query rows per request on average (with the lengths on the device the
-  // average is what the host knows) and no more (request, head) units per XCD than it has CUs, since a unit fills one.
-  // Their plan, if any, is not needed.  Measured (bf16, 32-row blocks, against the kernels below): 1 to 8 LLaDA
-  // requests 1.15 to 1.5 times as fast, 9 Dream requests (35 units on some XCDs) 0.7 times, 16 LLaDA requests the same.
-  if (D == 128 || D == 64) {
-    p.num_tiles = B;
-    if (total_q <= 32 * (int64_t)B && attn_grid_blocks(p) <= 256) return short_attention(p, mode, dtype, st);
-    // More units than the two workgroup slots of every CU: heads of a group two by two, which saves a round.  (Up to
-    // there a unit per head is faster, since half as many waves hide less latency: 16 Dream requests 33.6 us against
-    // 40.2 in pairs, 24 Dream requests 62.4 against 42.6.
-    // At head dim 64 a CU holds more units and there is no round to save: 24 requests of 32 / 8 heads 22.2 against 23.9.)
-    if (D == 128 && total_q <= 32 * (int64_t)B && H > H_kv && attn_grid_blocks(p) > 512)
-      return dtype == ACACHE_BF16 ? launch_pairs<ACACHE_BF16, 128>(p, mode, total_q, st)
-                                  : launch_pairs<ACACHE_F16, 128>(p, mode, total_q, st);
-  }
+  if (takes_short_kernel(p, mode, total_q, total_k)) return short_attention(p, mode, dtype, st);
+  if (takes_pair_kernel(p, total_q))
+    return dtype == ACACHE_BF16 ? launch_pairs<ACACHE_BF16, 128>(p, mode, total_q, st)
+                                : launch_pairs<ACACHE_F16, 128>(p, mode, total_q, st);
 #define ACACHE_ATTN(DT, DD) \
   if (dtype == DT && D == DD) return launch_attn<DT, DD, 2>(p, mode, total_q, plan_blocks, st);
   ACACHE_ATTN(ACACHE_BF16, 128)

@@ -343,8 +343,7 @@ __global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) float lds_rope[MODE == MODE_KEY_SIDE ? 2 * D : 4];
   int rank, kvh, hg, b = 0, q_begin = 0, q_len = 0, tile_in_request = 0, kv_begin = 0, kv_len = 0;
   if (!block_to_tile_head(p, rank, kvh, hg)) return;
-  // The grid holds one unit per (request, head), which is all of them when every request has at most 32 rows; the
-  // others follow in a second turn.  (A grid for the worst case would be half empty blocks, each waiting for a CU.)
+  // The grid holds num_tiles units per head: all of them, or one per request, and the others follow in a second turn.
   if (p.B <= 64) {
     int live = rank + 1;
     for (; rank < live; rank += p.num_tiles) {
