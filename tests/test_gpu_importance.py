@@ -11,7 +11,8 @@ from oracle import acache_oracle as O
 pytestmark = pytest.mark.gpu
 
 
-def _case(device, H, Hkv, D, A, mask_counts, shifts, slot0=0, dtype=torch.bfloat16, seed=0):
+def _case(device, H, Hkv, D, A, mask_counts, shifts, slot0=0, dtype=torch.bfloat16, seed=0, absent_every=0):
+    """`absent_every`: every so many mask rows lie outside q and count as no query."""
     g = torch.Generator().manual_seed(seed)
     S = slot0 + A + 7
     cos, sin = O.rope_table(max(shifts) + 2 if shifts else 4, D, 5e5)
@@ -21,7 +22,12 @@ def _case(device, H, Hkv, D, A, mask_counts, shifts, slot0=0, dtype=torch.bfloat
     rows = torch.randperm(Tq, generator=g)[:sum(mask_counts)].sort().values.to(torch.int32)
     cu = torch.tensor([0] + torch.tensor(mask_counts).cumsum(0).tolist(), dtype=torch.int32)
     sh = torch.tensor(shifts, dtype=torch.int32) if shifts else None
-    want = O.affix_importance(q, kc, rows, cu, A, affix_shifts=sh, cos=cos, sin=sin, affix_slot0=slot0)
+    live = torch.ones(len(rows), dtype=torch.bool)
+    if absent_every:
+        live[absent_every // 2::absent_every] = False
+    kept = torch.cat([torch.zeros(1, dtype=torch.int64), live.cumsum(0)])[cu.long()].to(torch.int32)
+    want = O.affix_importance(q, kc, rows[live], kept, A, affix_shifts=sh, cos=cos, sin=sin, affix_slot0=slot0)
+    rows[~live] = torch.tensor([-1, Tq, 1 << 30], dtype=torch.int32).repeat(len(rows))[:int((~live).sum())]
     imp = torch.zeros(len(mask_counts), A + 3, dtype=torch.float32, device=device)
     args = dict(affix_shifts=None if sh is None else sh.to(device), rope_cos=cos.to(device) if shifts else None,
                 rope_sin=sin.to(device) if shifts else None, affix_slot0=slot0)
@@ -40,12 +46,23 @@ def test_importance_matches_oracle(device, H, Hkv, D):
 
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("A,masks", [(1, [3, 1]), (7, [16, 0, 2]), (16 * 8, [17]), (16 * 8 + 1, [33, 300, 1]),
-                                     (16 * 8 * 5 + 3, [40]), (1024, [31, 65]), (1025, [20]), (1152, [9, 130]),
+                                     (16 * 8 * 5 + 3, [40]), (1024, [31, 65]), (1025, [20]), (1152, [9, 63, 64, 65, 130]),
                                      (1153, [97]), (1280, [16]), (1281, [16])])
 def test_affix_lengths_on_both_sides_of_the_key_block_counts(device, D, A, masks):
-    """One to eight 16-key blocks per wave in registers, two or three more in LDS, beyond that two passes; row counts
-    on both sides of a 16-row tile and of the staged rows."""
+    """One to eight 16-key blocks per wave in registers, or seven there and two or three in LDS, beyond that two passes; row
+    counts on both sides of a 16-row tile and of the 64 rows of a sum."""
     _case(device, 2, 1, D, A=A, mask_counts=masks, shifts=[(7 * i) % 50 for i in range(len(masks))], slot0=3, seed=A)
+
+
+@pytest.mark.parametrize("D,A,dtype", [(128, 400, torch.float16), (128, 600, torch.bfloat16), (128, 800, torch.bfloat16),
+                                       (128, 1000, torch.float16), (128, 1100, torch.bfloat16), (128, 1200, torch.bfloat16),
+                                       (64, 450, torch.bfloat16), (64, 1000, torch.bfloat16), (64, 1250, torch.float16)])
+@pytest.mark.parametrize("counts", [[256, 0, 1, 65, 130, 16, 256, 33, 200], [40, 64, 64, 17, 0, 50]])
+def test_workgroups_that_take_several_requests(device, D, A, dtype, counts):
+    """64 heads leave four workgroups per head: two and three turns each, with the next request's queries on their way while
+    one is scored, requests with and without a shift behind one another, empty ones, and absent rows in every turn."""
+    shifts = [0 if i % 3 == 1 else 5 + 9 * i for i in range(len(counts))]
+    _case(device, 64, 8, D, A=A, mask_counts=counts, shifts=shifts, slot0=2, dtype=dtype, seed=A, absent_every=37)
 
 
 def test_llada_shape_and_accumulation_over_layers(device):
