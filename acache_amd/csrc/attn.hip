@@ -14,7 +14,8 @@
 //   rescale factor are per-lane scalars; the softmax denominator is one more
 //   MFMA row block (V^T rows of ones).
 //
-// Two kernels (batches of a few short query blocks go to attn_short.hip):
+// Two kernels (batches of a few short query blocks go to attn_short.hip, grouped-query batches of many to
+// varlen_attn_pair_kernel below):
 //   varlen_attn_unit_kernel (head_dim 64 and 128, all three relocation modes): K/V rows are copied
 //     global -> LDS directly through the slot map into a two-deep ring, swizzled by permuting the
 //     global side of the copy; V stays row-major and is read with the LDS transpose read.  Scores are
@@ -1070,7 +1071,8 @@ static int launch_attn_any_head_dim(const AttnParams &p0, int mode, int64_t tota
 //   D 128, query side      1.06 to 1.23  0.94 to 1.04  0.84 to 0.93  0.77 to 0.86  0.57 to 0.74
 //   D 64                   0.92 to 1.15  0.83 to 0.99  0.77 to 0.89  0.68 to 0.78  0.53 to 0.72
 // (the eight waves' set-up and merge against a chain of short tiles).  More streams than that are bound by memory where the
-// keys are private: plain 0.87 to 1.18 and key side 0.84 to 1.04 at 1100 keys, but query side 0.78 to 0.87.
+// keys are private: plain 0.87 to 1.18 and key side 0.84 to 1.04 at 1100 keys, but query side 0.78 to 0.87.  (Plain and key
+// side share their lines: a key-side call has the bits of a plain one over a materialised copy.)
 // A request of more than 32 rows is several units.  They all fit the CUs if even the worst lengths do (two LLaDA requests
 // of 33 and 31 rows and 1300 keys: 24.5 us in per-head units, 30.3 with units in two turns, 18.8 in one).  Beyond that the
 // grid has a unit per request and head, further ones wait (8 Dream requests of 33 and 31 rows: 25.1 / 32.1 us), and the
@@ -1078,7 +1080,7 @@ static int launch_attn_any_head_dim(const AttnParams &p0, int mode, int64_t tota
 static bool takes_short_kernel(AttnParams &p, int mode, int64_t total_q, int64_t total_k) {
   const int64_t B = p.B;
   if ((p.head_dim != 128 && p.head_dim != 64) || total_q > 32 * B) return false;
-  if (total_k < B * (p.head_dim == 64 ? 512 : mode == MODE_PLAIN ? 1024 : 768)) return false;
+  if (total_k < B * (p.head_dim == 64 ? 512 : mode == MODE_QUERY_SIDE ? 768 : 1024)) return false;
   if (p.head_dim == 128 && mode != MODE_QUERY_SIDE && B * p.H_kv > 128) return false;
   p.num_tiles = (int32_t)((total_q + 31 * B) / 32);
   if (attn_grid_blocks(p) <= 256) return true;

@@ -151,6 +151,27 @@ def test_plan_and_slot_pitch_do_not_change_the_bits(device):
         assert torch.equal(ops.acache_attention(q, *wide, *args), ops.acache_attention(q, kc, vc, *args))
 
 
+@pytest.mark.parametrize("D,keys", [(128, 700), (128, 900), (128, 1100), (64, 400), (64, 600)])
+@pytest.mark.parametrize("H,Hkv,B", [(4, 4, 3), (28, 4, 7), (16, 16, 8), (16, 16, 9)])
+def test_key_side_equals_a_materialised_copy(device, D, keys, H, Hkv, B):
+    """On both sides of every line of the dispatch, plain attention over a relocated copy takes the form that key-side
+    relocation takes: the same bits.  All requests have their shared rows at the same position."""
+    g, S = torch.Generator(device=device).manual_seed(keys), A + 16 * (keys // 16 + 1)
+    q = torch.randn(32 * B, H, D, generator=g, device=device).to(torch.bfloat16)
+    kc, vc = (torch.randn(1, S + A + 8, Hkv, D, generator=g, device=device).to(torch.bfloat16) for _ in range(2))
+    own = torch.randperm(S - A)[:keys - A] + A
+    at = torch.cat([own[:START], torch.arange(A), own[START:]])
+    cu = lambda n: torch.arange(0, n * B + 1, n, dtype=torch.int32, device=device)
+    call = lambda slots, **kw: ops.acache_attention(q, kc[0], vc[0], cu(32), cu(keys),
+                                                    slots.to(torch.int32).repeat(B).to(device), **kw)
+    cos, sin = (t.to(device) for t in O.rope_table(64, D, 5e5))
+    key_side = call(at, shared_prefix_len=A, rope_cos=cos, rope_sin=sin,
+                    affix_shifts=torch.full((B,), START, dtype=torch.int32, device=device))
+    ops.materialize_relocated_affix(kc, vc, cos, sin, S, A, START)
+    at[START:START + A] = torch.arange(S, S + A)
+    assert torch.equal(call(at), key_side)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("logit", [-20.0, -100.0])
 @pytest.mark.parametrize("shared", [1, 31, 32, 33])
