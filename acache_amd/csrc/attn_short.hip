@@ -15,11 +15,12 @@
 // waves, one barrier per half: 25 us for one request.  Four such waves and two workgroups per CU, for more units than
 // CUs: 16 LLaDA requests 51 us, against 48 of the two-deep ring in attn.hip.)
 //
-// Measured (bf16, D = 128, 32 query rows per request, microseconds per call, before (varlen_attn_unit_kernel) / now):
-//   LLaDA heads, 1 200 to 1 400 keys: 1 request 19.5 / 16.1, 2: 22.1 / 17.4, 4: 23.0 / 19.9, 8: 33.0 / 27.7; relocated on
-//   the query side 2: 32.3 / 21.3, 4: 32.8 / 24.0, 8: 41.2 / 31.2.  Dream heads, 4 requests: 19.3 / 16.8, relocated 28.9 /
-//   20.7.  Of the 15.3 us of the one-request kernel 2.5 are launch and tile lookup, 2.4 the first chunk's two memory round
-//   trips, 7.7 the chunks (590 KB of keys and values into one CU, at most 110 GB/s) and 2.8 the merge and the stores.
+// Measured (bf16, D = 128, 32 query rows and about 1 300 keys per request, three quarters of them shared, microseconds per
+// call, varlen_attn_unit_kernel / this kernel):
+//   LLaDA heads, plain 1 request 18.4 / 16.0, 4: 22.6 / 19.1; query side 1: 23.6 / 19.0, 4: 30.8 / 21.6, 8: 33.5 / 24.3;
+//   key side 1: 29.4 / 24.0.  Dream heads, plain 1: 18.6 / 16.3, 8: 19.5 / 17.5; query side 8: 25.6 / 20.6; key side 8:
+//   31.1 / 27.0.  One LLaDA request keeps 32 CUs busy with 590 KB of keys and values each, which takes 5.4 us by copies
+//   alone (110 GB/s into one CU).
 #include "attn_common.h"
 
 namespace acache {

@@ -596,8 +596,8 @@ __global__ __launch_bounds__(256) void importance_colsum_lds_kernel(ImportancePa
 // per tile, and add the normalised probabilities to per-lane column sums.  The keys are read once per workgroup,
 // which takes the rows of several requests in turn (one workgroup per CU); the queries go straight from q to LDS by
 // the copy engine while the item before is scored, and are counter-rotated there, so the packed copy in memory and
-// its launch are gone too.  Key blocks past the eighth of a wave sit in LDS in fragment order (NBL of them), because
-// operands, scores, column sums and the query fragment have to share the 256 registers.
+// its launch are gone too.  A wave with nine or ten key blocks keeps seven in registers and NBL of them, two or three, in
+// LDS in fragment order, because operands, scores, column sums and the query fragment share the 256 registers.
 //
 // LLaDA heads, 256 rows a request, relocated, both launches of the call, two passes / this form: 16 requests with 300 /
 // 600 / 1000 / 1100 / 1200 keys 68 / 90 / 120 / 134 / 139 -> 41 / 52 / 68 / 79 / 88 us; one request of 300 / 1000 keys
@@ -936,7 +936,8 @@ extern "C" int64_t acache_affix_importance_workspace_bytes(int64_t total_mask_ro
                                                            int32_t relocated) {
   if (total_mask_rows < 0 || B < 0 || H < 0 || H_kv < 0 || D < 0 || affix_len < 0) return 0;
   (void)H_kv;
-  (void)relocated;  // the packed copy of the mask queries (2-byte elements) is made with and without relocation
+  (void)relocated;  // the two-pass form makes its packed copy of the mask queries (2-byte elements) either way
+  // (one size for both forms: the one-pass form's partial sums take less than this)
   return stats_bytes(total_mask_rows, H) + partial_bytes(B, H, affix_len) + total_mask_rows * H * D * 2;
 }
 

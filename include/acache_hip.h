@@ -190,8 +190,11 @@ int acache_rope_qk_scatter(
  * [0, total_q) is an absent query and adds nothing.  workspace:
  * device scratch of at least acache_affix_importance_workspace_bytes(total_mask_rows, B, H,
  * H_kv, D, affix_len, relocated = affix_shifts != NULL) bytes (row statistics, per-head
- * partial sums and the packed, counter-rotated copy of the mask queries,
- * passed between the launches), 16-byte aligned, owned by the caller.  max_mask_rows: an upper bound on
+ * partial sums and the packed, counter-rotated copy of the mask queries, passed between
+ * the launches; affixes of up to 1280 keys at D 64 and 128 take partial sums only, which
+ * need less), 16-byte aligned, owned by the caller; a larger one does not change the result.
+ * The sums added for a request depend on its own rows, keys and shift, not on the other
+ * requests of the call.  max_mask_rows: an upper bound on
  * the mask rows of one request; a request whose cu_mask entries claim more rows than that, or more than
  * total_mask_rows leaves room for, is scored on the rows that fit (cu_mask is device memory the host does
  * not read).  D: a multiple of 16 up to 256; dtype bf16 or f16.
