@@ -748,18 +748,22 @@ def baseline_decode_attention(
         softmax_scale = head_dim ** -0.5
     seqlens = _i32(seqlens, "seqlens")
     if seqlens.numel() == batch and 0 < batch <= 65535 and query_len > 0 and block_tables.dim() == 2:
+        device = q.device
         if total_k is None:
             total_k = int(seqlens.sum().item())
-        seqlens, tables = seqlens.to(q.device), _i32(block_tables, "block_tables").to(q.device)
-        if tables.shape[0] < batch:  # requests without a row have no blocks
-            tables = torch.nn.functional.pad(tables, (0, 0, 0, batch - tables.shape[0]), value=-1)
-        cu_q = torch.empty(batch + 1, dtype=torch.int32, device=q.device)
-        cu_k = torch.empty(batch + 1, dtype=torch.int32, device=q.device)
-        slots = torch.empty(int(total_k), dtype=torch.int32, device=q.device)
+        tables = _i32(block_tables, "block_tables")
+        rows, max_blocks = tables.shape
+        if rows < batch:  # requests without a row have no blocks
+            tables = torch.nn.functional.pad(tables, (0, 0, 0, batch - rows), value=-1)
+        if seqlens.device != device or tables.device != device:
+            seqlens, tables = seqlens.to(device), tables.to(device)
+        cu_q = torch.empty(batch + 1, dtype=torch.int32, device=device)
+        cu_k = torch.empty_like(cu_q)
+        slots = torch.empty(int(total_k), dtype=torch.int32, device=device)
         lib = _lib.load()
-        with torch.cuda.device(q.device):
+        with torch.cuda.device(device):
             rc = lib.acache_decode_layout(
-                _ptr(cu_q), _ptr(cu_k), _ptr(slots), _ptr(seqlens), _ptr(tables), batch, query_len, tables.shape[1],
+                _ptr(cu_q), _ptr(cu_k), _ptr(slots), _ptr(seqlens), _ptr(tables), batch, query_len, max_blocks,
                 k_cache.shape[1], int(total_k), _stream(q))
         _lib.check(rc, "decode_layout")
     else:  # nothing to lay out, more requests than one launch covers, or lengths that broadcast
