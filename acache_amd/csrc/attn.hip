@@ -14,8 +14,8 @@
 //   rescale factor are per-lane scalars; the softmax denominator is one more
 //   MFMA row block (V^T rows of ones).
 //
-// Two kernels (batches of a few short query blocks go to attn_short.hip, grouped-query batches of many to
-// varlen_attn_pair_kernel below):
+// Two kernels (batches of a few short query blocks go to attn_short.hip, grouped-query batches of more to attn_group.hip
+// or varlen_attn_pair_kernel below):
 //   varlen_attn_unit_kernel (head_dim 64 and 128, all three relocation modes): K/V rows are copied
 //     global -> LDS directly through the slot map into a two-deep ring, swizzled by permuting the
 //     global side of the copy; V stays row-major and is read with the LDS transpose read.  Scores are
@@ -1088,6 +1088,43 @@ static bool takes_short_kernel(AttnParams &p, int mode, int64_t total_q, int64_t
   return total_q % B == 0 && attn_grid_blocks(p) <= 256;
 }
 
+// Several heads of a group per unit of eight waves (attn_group.hip), one unit per CU; sets p.num_tiles.  Returns the heads, 0
+// for the other kernels.  Time against those (the per-head units, or pairs of heads in four waves beyond two units per CU),
+// bf16, 32 / 8, 28 / 4, 14 / 2 and 8 / 2 heads, ragged keys, blocks of 8 and 32 rows:
+//   keys per request             60            150           300           600           1100          2000
+//   2 heads, up to 256 units (more of one head)
+//     plain                      0.88 to 1.18  0.82 to 1.09  0.80 to 1.03  0.85 to 1.03  0.85 to 1.03  0.85 to 0.94
+//     key side                   0.84 to 1.08  0.80 to 0.94  0.77 to 0.85  0.73 to 0.81  0.70 to 0.76  0.70 to 0.75
+//     query side                 0.78 to 0.91  0.81 to 0.94  0.78 to 0.90  0.78 to 0.87  0.72 to 0.82  0.63 to 0.72
+//   4 heads, 193 to 256 units
+//     plain                      0.78 to 0.92  0.77 to 0.90  0.82 to 0.94  0.88 to 0.99  0.97 to 1.03  0.93 to 1.06
+//     key side                   0.72 to 0.82  0.71 to 0.77  0.75 to 0.82  0.79 to 0.83  0.82 to 0.86  0.88 to 0.90
+//     query side                 0.66 to 0.74  0.72 to 0.78  0.74 to 0.81  0.81 to 0.88  0.85 to 0.93  0.84 to 0.88
+//   4 heads, 385 to 512 units
+//     plain                      0.78 to 0.83  0.80 to 0.86  0.84 to 0.90  0.89 to 0.94  0.86 to 0.99  0.83 to 1.03
+//     key side                   0.72 to 0.73  0.73 to 0.74  0.75          0.79 to 0.82  0.82 to 0.84  0.86 to 0.87
+//     query side                 0.67 to 0.70  0.73          0.75 to 0.76  0.81 to 0.83  0.84 to 0.86  0.85 to 0.88
+// Two heads take one turn of the CUs, four up to two, where the last leaves at most a quarter of the CUs idle (with more
+// idle: plain 0.83 to 1.15, query side 0.75 to 1.04).  A batch that fits 256 units of one
+// head stays with those.  Plain and key side share their lines: a key-side call has the bits of a plain one over a
+// materialised copy.  All 32-row tiles get a unit where the worst lengths of such a batch fit the grid; beyond that it has
+// to look like blocks of one length, as for the kernel above.
+static int heads_per_group_unit(AttnParams &p, int mode, int64_t total_q, int64_t total_k) {
+  const int64_t B = p.B;
+  const int group = p.H / p.H_kv;
+  if (p.head_dim != 128 || group < 2 || total_q > 32 * B) return 0;
+  const bool query_side = mode == MODE_QUERY_SIDE;
+  p.num_tiles = (int32_t)((total_q + 31 * B) / 32);
+  if (attn_grid_blocks(p, (group + 1) / 2) > 256) {
+    if (total_q % B != 0) return 0;
+    p.num_tiles = p.B;
+  }
+  if (attn_grid_blocks(p) <= 256) return 0;
+  if (attn_grid_blocks(p, (group + 1) / 2) <= 256) return query_side || total_k >= 256 * B ? 2 : 0;
+  const int64_t units = attn_grid_blocks(p, (group + 3) / 4), idle = (512 - units) % 256;
+  return units <= 512 && (query_side ? idle <= 64 : idle < 64 && total_k <= 1536 * B) ? 4 : 0;
+}
+
 // Two heads of a group per unit: where a unit per head is more than the two workgroup slots of every CU, which saves a
 // round.  (Up to there a unit per head is faster, since half as many waves hide less latency: 16 Dream requests 33.6 us
 // against 40.2 in pairs, 24 Dream requests 62.4 against 42.6.  Blocks of 1 to 32 rows, 40 to 1300 keys, groups of 2 to 7:
@@ -1153,6 +1190,7 @@ extern "C" int acache_varlen_attn_planned(
   hipStream_t st = (hipStream_t)stream;
   p.small_cache = 0;
   if (takes_short_kernel(p, mode, total_q, total_k)) return short_attention(p, mode, dtype, st);
+  if (const int heads = heads_per_group_unit(p, mode, total_q, total_k)) return group_attention(p, heads, mode, dtype, st);
   if (takes_pair_kernel(p, total_q))
     return dtype == ACACHE_BF16 ? launch_pairs<ACACHE_BF16, 128>(p, mode, total_q, st)
                                 : launch_pairs<ACACHE_F16, 128>(p, mode, total_q, st);

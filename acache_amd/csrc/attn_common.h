@@ -123,6 +123,65 @@ __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const
   return true;
 }
 
+// The unit of a kernel whose blocks all run at once (attn_short.hip, attn_group.hip: the order does not matter), with
+// what its set-up needs of the request.
+struct ShortUnit {
+  int b, q_begin, q_len, tile, kv_begin, kv_len;
+  int shared_len, shift;  // clamped; 0 in the modes that have none
+};
+
+// Query tile `rank` (BM rows) in batch order.  For up to 64 requests everything is loaded in one round trip, one request
+// per lane, and a batch of one tile per request, which is what blocks of one length are, needs no prefix sum: 0.3 us
+// from the loads to the unit, where ranking one request by its keys takes 0.9 and sixteen 1.6.
+template <int MODE>
+__device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, int rank, ShortUnit &u) {
+  const int lane = threadIdx.x & 63;
+  int shared = 0, shift = 0;
+  if (p.B <= 64) {
+    const int l = lane < p.B ? lane : p.B - 1;
+    const int q0 = p.cu_q[l], q1 = p.cu_q[l + 1], k0 = p.cu_k[l], k1 = p.cu_k[l + 1];
+    if (MODE == MODE_QUERY_SIDE) shared = p.shared_kv_lens[l];
+    if (MODE != MODE_PLAIN) shift = p.affix_shifts[l];
+    const int tiles = lane < p.B && q1 > q0 ? (q1 - q0 + BM - 1) / BM : 0;
+    int src = rank;
+    u.tile = 0;
+    if (__builtin_amdgcn_ballot_w64(lane < p.B && tiles != 1) == 0) {
+      if (rank >= p.B) return false;
+    } else {
+      int incl = tiles;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(incl, d);
+        if (lane >= d) incl += up;
+      }
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(incl > rank);
+      if (hit == 0) return false;
+      src = __builtin_ctzll(hit);
+      u.tile = rank - (__builtin_amdgcn_readlane(incl, src) - __builtin_amdgcn_readlane(tiles, src));
+    }
+    u.b = src;
+    u.q_begin = __builtin_amdgcn_readlane(q0, src);
+    u.q_len = __builtin_amdgcn_readlane(q1, src) - u.q_begin;
+    u.kv_begin = __builtin_amdgcn_readlane(k0, src);
+    u.kv_len = __builtin_amdgcn_readlane(k1, src) - u.kv_begin;
+    if (MODE == MODE_QUERY_SIDE) shared = __builtin_amdgcn_readlane(shared, src);
+    if (MODE != MODE_PLAIN) shift = __builtin_amdgcn_readlane(shift, src);
+  } else {
+    if (!locate_query_tile(p.cu_q, p.B, BM, rank, u.b, u.q_begin, u.q_len, u.tile)) return false;
+    u.b = __builtin_amdgcn_readfirstlane(u.b);
+    u.q_begin = __builtin_amdgcn_readfirstlane(u.q_begin);
+    u.q_len = __builtin_amdgcn_readfirstlane(u.q_len);
+    u.tile = __builtin_amdgcn_readfirstlane(u.tile);
+    u.kv_begin = p.cu_k[u.b];
+    u.kv_len = p.cu_k[u.b + 1] - u.kv_begin;
+    if (MODE == MODE_QUERY_SIDE) shared = p.shared_kv_lens[u.b];
+    if (MODE != MODE_PLAIN) shift = p.affix_shifts[u.b];
+  }
+  u.shared_len = shared < 0 ? 0 : (shared > u.kv_len ? u.kv_len : shared);
+  u.shift = shift < 0 || shift >= p.rope_rows ? 0 : shift;
+  return true;
+}
+
 // Block -> (query tile rank, KV head, head inside its group) for the kernels that stream K/V per (tile, head).
 // Consecutive block indices go to different XCDs (index mod 8), each with its own L2, so every XCD is given a
 // contiguous range of KV heads: all query tiles that read a head's K/V find it in the same L2.
@@ -182,6 +241,9 @@ inline bool small_cache(const AttnParams &p) {
 // attn_short.hip: batches of short query blocks, head dims 64 and 128.
 int short_attention(const AttnParams &p, int mode, int dtype, hipStream_t stream);
 
+// attn_group.hip: grouped-query batches of short query blocks, head dim 128.
+int group_attention(const AttnParams &p, int heads_per_unit, int mode, int dtype, hipStream_t stream);
+
 // Key range of tile t: the shared range [0, shared_len) comes first in tiles of BN
 // (query-side mode only, otherwise shared_len = 0), then [shared_len, kv_len).
 struct TileRange {
@@ -230,6 +292,15 @@ __device__ __forceinline__ const char *uniform_ptr(const char *p) {
 // The copy with the source given as a wave-uniform base plus a 32-bit byte offset per lane.
 __device__ __forceinline__ void lds_dma16_off(const char *base, uint32_t offset, uint32_t lds_offset) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "{m0}"(lds_offset) : "memory");
+}
+
+// threadIdx.x behind an opaque zero: what is derived from it is computed where it stands.  Left to itself the compiler
+// moves lane constants to the front of the kernel and keeps them in scratch until they are needed; reading them back waits
+// for every copy in flight.
+__device__ __forceinline__ int opaque_tid() {
+  int zero;
+  asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
+  return threadIdx.x + zero;
 }
 
 // Online-softmax update of one key tile, in two steps shared by both attention kernels so that
