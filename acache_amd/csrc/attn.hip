@@ -1063,16 +1063,17 @@ static int launch_attn_any_head_dim(const AttnParams &p0, int mode, int64_t tota
 // Their plan, if any, is not needed.  The lengths are on the device: the host knows totals only.
 
 // Wave-private key chunks (attn_short.hip), a unit of 32 query rows per CU; sets p.num_tiles to the tiles of its grid.
-// Measured as time against the per-head units (bf16, blocks of 1, 16 and 32 rows, 1 to 8 LLaDA and Dream requests and 4 to
-// 128 requests of 8 and 2 heads, private keys and three quarters shared; up to 128 (request, KV head) streams):
-//   keys per request       200           512           768           1100          2000
-//   D 128, plain           1.01 to 1.25  0.93 to 1.14  0.86 to 1.06  0.79 to 0.96  0.73 to 0.90
-//   D 128, key side        1.08 to 1.33  0.95 to 1.09  0.86 to 0.97  0.78 to 0.93  0.73 to 0.86
-//   D 128, query side      1.06 to 1.23  0.94 to 1.04  0.84 to 0.93  0.77 to 0.86  0.57 to 0.74
-//   D 64                   0.92 to 1.15  0.83 to 0.99  0.77 to 0.89  0.68 to 0.78  0.53 to 0.72
-// (the eight waves' set-up and merge against a chain of short tiles).  More streams than that are bound by memory where the
-// keys are private: plain 0.87 to 1.18 and key side 0.84 to 1.04 at 1100 keys, but query side 0.78 to 0.87.  (Plain and key
-// side share their lines: a key-side call has the bits of a plain one over a materialised copy.)
+// Measured as time against the per-head units (bf16, 1 to 32 requests of 32 / 32, 28 / 4, 16 / 16 and 8 / 2 heads, ragged
+// keys, blocks of 8 and 32 rows, every key private or most of them shared):
+//   keys per request       100           200           300           400           600           1000          2000
+//   D 128, plain           1.01 to 1.22  1.00 to 1.14  0.89 to 1.08  0.86 to 1.02  0.84 to 1.00  0.76 to 0.95  0.67 to 0.99
+//   D 128, key side        1.00 to 1.18  0.94 to 1.05  0.91 to 1.03  0.84 to 0.91  0.78 to 0.83  0.70 to 0.76  0.62 to 0.79
+//   D 128, query side      0.90 to 0.99  0.84 to 0.94  0.78 to 0.86  0.78 to 0.81  0.73 to 0.78  0.56 to 0.66  0.48 to 0.66
+//   D 64, plain            1.15 to 1.21  1.04 to 1.14  0.98 to 1.07  0.96 to 1.04  0.84 to 0.96  0.71 to 0.95  0.61 to 0.99
+//   D 64, key side         1.06 to 1.10  0.92 to 0.99  0.85 to 0.93  0.80 to 0.88  0.76 to 0.82  0.68 to 0.74  0.60 to 0.65
+//   D 64, query side       0.94 to 1.00  0.87 to 0.96  0.81 to 0.89  0.79 to 0.88  0.75 to 0.79  0.63 to 0.69  0.47 to 0.60
+// (the eight waves' set-up and merge against a chain of short tiles).  Plain and key side share their lines: a key-side call
+// has the bits of a plain one over a materialised copy.
 // A request of more than 32 rows is several units.  They all fit the CUs if even the worst lengths do (two LLaDA requests
 // of 33 and 31 rows and 1300 keys: 24.5 us in per-head units, 30.3 with units in two turns, 18.8 in one).  Beyond that the
 // grid has a unit per request and head, further ones wait (8 Dream requests of 33 and 31 rows: 25.1 / 32.1 us), and the
@@ -1080,8 +1081,7 @@ static int launch_attn_any_head_dim(const AttnParams &p0, int mode, int64_t tota
 static bool takes_short_kernel(AttnParams &p, int mode, int64_t total_q, int64_t total_k) {
   const int64_t B = p.B;
   if ((p.head_dim != 128 && p.head_dim != 64) || total_q > 32 * B) return false;
-  if (total_k < B * (p.head_dim == 64 ? 512 : mode == MODE_QUERY_SIDE ? 768 : 1024)) return false;
-  if (p.head_dim == 128 && mode != MODE_QUERY_SIDE && B * p.H_kv > 128) return false;
+  if (total_k < B * (mode == MODE_QUERY_SIDE ? 256 : p.head_dim == 64 ? 512 : 400)) return false;
   p.num_tiles = (int32_t)((total_q + 31 * B) / 32);
   if (attn_grid_blocks(p) <= 256) return true;
   p.num_tiles = p.B;
@@ -1114,12 +1114,14 @@ static int heads_per_group_unit(AttnParams &p, int mode, int64_t total_q, int64_
   const int group = p.H / p.H_kv;
   if (p.head_dim != 128 || group < 2 || total_q > 32 * B) return 0;
   const bool query_side = mode == MODE_QUERY_SIDE;
-  p.num_tiles = (int32_t)((total_q + 31 * B) / 32);
+  const int32_t worst = (int32_t)((total_q + 31 * B) / 32);
+  p.num_tiles = total_q % B == 0 ? p.B : worst;
+  if (attn_grid_blocks(p) <= 256) return 0;
+  p.num_tiles = worst;
   if (attn_grid_blocks(p, (group + 1) / 2) > 256) {
     if (total_q % B != 0) return 0;
     p.num_tiles = p.B;
   }
-  if (attn_grid_blocks(p) <= 256) return 0;
   if (attn_grid_blocks(p, (group + 1) / 2) <= 256) return query_side || total_k >= 256 * B ? 2 : 0;
   const int64_t units = attn_grid_blocks(p, (group + 3) / 4), idle = (512 - units) % 256;
   return units <= 512 && (query_side ? idle <= 64 : idle < 64 && total_k <= 1536 * B) ? 4 : 0;

@@ -123,6 +123,15 @@ __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const
   return true;
 }
 
+// threadIdx.x behind an opaque zero: what is derived from it is computed where it stands.  Left to itself the compiler
+// moves lane constants to the front of the kernel and keeps them in scratch until they are needed; reading them back waits
+// for every copy in flight.
+__device__ __forceinline__ int opaque_tid() {
+  int zero;
+  asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
+  return threadIdx.x + zero;
+}
+
 // The unit of a kernel whose blocks all run at once (attn_short.hip, attn_group.hip: the order does not matter), with
 // what its set-up needs of the request.
 struct ShortUnit {
@@ -135,7 +144,7 @@ struct ShortUnit {
 // from the loads to the unit, where ranking one request by its keys takes 0.9 and sixteen 1.6.
 template <int MODE>
 __device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, int rank, ShortUnit &u) {
-  const int lane = threadIdx.x & 63;
+  const int lane = opaque_tid() & 63;
   int shared = 0, shift = 0;
   if (p.B <= 64) {
     const int l = lane < p.B ? lane : p.B - 1;
@@ -292,15 +301,6 @@ __device__ __forceinline__ const char *uniform_ptr(const char *p) {
 // The copy with the source given as a wave-uniform base plus a 32-bit byte offset per lane.
 __device__ __forceinline__ void lds_dma16_off(const char *base, uint32_t offset, uint32_t lds_offset) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "{m0}"(lds_offset) : "memory");
-}
-
-// threadIdx.x behind an opaque zero: what is derived from it is computed where it stands.  Left to itself the compiler
-// moves lane constants to the front of the kernel and keeps them in scratch until they are needed; reading them back waits
-// for every copy in flight.
-__device__ __forceinline__ int opaque_tid() {
-  int zero;
-  asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
-  return threadIdx.x + zero;
 }
 
 // Online-softmax update of one key tile, in two steps shared by both attention kernels so that

@@ -15,12 +15,16 @@
 // waves, one barrier per half: 25 us for one request.  Four such waves and two workgroups per CU, for more units than
 // CUs: 16 LLaDA requests 51 us, against 48 of the two-deep ring in attn.hip.)
 //
-// Measured (bf16, D = 128, 32 query rows and about 1 300 keys per request, three quarters of them shared, microseconds per
-// call, varlen_attn_unit_kernel / this kernel):
-//   LLaDA heads, plain 1 request 18.4 / 16.0, 4: 22.6 / 19.1; query side 1: 23.6 / 19.0, 4: 30.8 / 21.6, 8: 33.5 / 24.3;
-//   key side 1: 29.4 / 24.0.  Dream heads, plain 1: 18.6 / 16.3, 8: 19.5 / 17.5; query side 8: 25.6 / 20.6; key side 8:
-//   31.1 / 27.0.  One LLaDA request keeps 32 CUs busy with 590 KB of keys and values each, which takes 5.4 us by copies
-//   alone (110 GB/s into one CU).
+// The set-up is three dependent round trips (lengths; slots, queries, table rows; keys), as in attn_group.hip: the queries
+// go through LDS once per unit and are relocated there once.  With every wave reading the 32 rows for itself behind a
+// lookup of one request at a time it was 5.0 us of one request's 14.9.
+//
+// Measured (bf16, D = 128, 32 query rows and about 1 300 keys per request, three quarters of them shared in the relocation
+// modes, microseconds per call, varlen_attn_unit_kernel / this kernel with a set-up per wave / now):
+//   32 / 32 heads, plain 1 request 18.4 / 16.3 / 14.7, 4: 22.6 / 23.0 / 20.2; query side 1: 23.6 / 19.0 / 15.5, 4: 30.8 /
+//   23.6 / 19.3, 8: 33.5 / 26.1 / 21.1; key side 1: 29.4 / 24.5 / 21.1.  28 / 4 heads, plain 1: 18.6 / 16.7 / 14.9, 8: 19.5 /
+//   19.5 / 16.9; query side 8: 25.6 / 22.1 / 17.7; key side 8: 31.1 / 28.8 / 23.6.  One request of 32 heads
+//   keeps 32 CUs busy with 590 KB of keys and values each, which takes 5.4 us by copies alone (110 GB/s into one CU).
 #include "attn_common.h"
 
 namespace acache {
@@ -33,9 +37,8 @@ __device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmc
 
 // One unit: 32 query rows (query tile `tile_in_request` of request b) of one head.
 template <int DTYPE, int D, int MODE>
-__device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, float *stats, float *lds_rope, int kvh,
-                                                int hg, int b, int q_begin, int q_len, int tile_in_request,
-                                                int kv_begin, int kv_len) {
+__device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, char *lds_q, float *stats, float *lds_rope,
+                                                int kvh, int head, const ShortUnit &u) {
   constexpr int QROWS = 32, NQ16 = 2;         // query rows of a unit
   constexpr int BN = 32;                      // keys per chunk
   constexpr int KS = D / 32, DT = D / 16;
@@ -50,60 +53,23 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-  const int group = p.H / p.H_kv;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = opaque_tid(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
-  const int head = kvh * group + hg;
-  const int q_row0 = tile_in_request * QROWS;
-  char *const out_base = p.out + (int64_t)q_begin * p.o_token_bytes + (int64_t)head * p.o_head_bytes;
+  const int kv_begin = u.kv_begin, kv_len = u.kv_len, shared_len = u.shared_len, shift = u.shift;
+  const int q_row0 = u.q_begin + u.tile * QROWS;
+  const int rows = u.q_len - u.tile * QROWS < QROWS ? u.q_len - u.tile * QROWS : QROWS;
+  char *const out_base = p.out + (int64_t)q_row0 * p.o_token_bytes + (int64_t)head * p.o_head_bytes;
 
   if (kv_len <= 0) {  // no keys: defined output (zeros)
-    for (int r = tid / CH; r < QROWS; r += 64 * NW / CH)
-      if (q_row0 + r < q_len)
-        store16(out_base + (int64_t)(q_row0 + r) * p.o_token_bytes + (tid % CH) * 16, vec16{{0, 0, 0, 0}});
+    for (int r = tid / CH; r < rows; r += 64 * NW / CH)
+      store16(out_base + (int64_t)r * p.o_token_bytes + (tid % CH) * 16, vec16{{0, 0, 0, 0}});
     return;
   }
 
-  int shared_len = 0, shift = 0;
-  if (MODE == MODE_QUERY_SIDE) {
-    shared_len = p.shared_kv_lens[b];
-    shared_len = __builtin_amdgcn_readfirstlane(shared_len < 0 ? 0 : (shared_len > kv_len ? kv_len : shared_len));
-  }
-  if (MODE != MODE_PLAIN) {
-    shift = p.affix_shifts[b];
-    if (shift < 0 || shift >= p.rope_rows) shift = 0;
-  }
   // chunks: the shared range first (query-side mode), then the rest
   const int chunks_a = (shared_len + BN - 1) / BN;
   const int n_chunks = chunks_a + (kv_len - shared_len + BN - 1) / BN;
-
-  // Query fragments.  Query-side mode scores the shared keys against the counter-rotated q', the others against q; a
-  // wave holds one of the two and reads q again when its shared chunks are done.
-  vec16 qf[NQ16][KS];
-  const char *const q_base = p.q + (int64_t)q_begin * p.q_token_bytes + (int64_t)head * p.q_head_bytes;
-  auto load_q = [&](bool rotated) __attribute__((always_inline)) {
-#pragma unroll
-    for (int qt = 0; qt < NQ16; ++qt) {
-      // (rows past the end repeat the last one and are not stored: a load under a lane mask is a block of its own)
-      const int qr = q_row0 + qt * 16 + li < q_len ? q_row0 + qt * 16 + li : q_len - 1;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        qf[qt][ks] = load16(q_base + (int64_t)qr * p.q_token_bytes + (32 * ks + 8 * lg) * 2);
-      if (MODE == MODE_QUERY_SIDE && rotated && shift != 0) {
-        const float *cr = p.cos_tab + (int64_t)shift * D, *sr = p.sin_tab + (int64_t)shift * D;
-#pragma unroll
-        for (int ks = 0; ks < KS / 2; ++ks)
-          rotate_pair<DTYPE, D>(qf[qt][ks], qf[qt][ks + KS / 2], cr, sr, 32 * ks + 8 * lg, -1.0f);
-      }
-    }
-  };
-  auto settle_q = [&]() __attribute__((always_inline)) {  // (waited for here, not inside the loop)
-#pragma unroll
-    for (int qt = 0; qt < NQ16; ++qt)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) settle(qf[qt][ks]);
-  };
 
   // ---- copies -------------------------------------------------------------------------------------------------
   // Lane l of slots[j] holds the slot of row l % 32 of the wave's chunk 2 j + l / 32, counted from the last refill.
@@ -170,32 +136,12 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
     }
   };
 
-  // ---- fragment addresses ---------------------------------------------------------------------------------------
   typedef __attribute__((address_space(3))) const char *LdsBytes;
-  LdsBytes k_frag[KS], v_frag[DT];
-  {
-    const LdsBytes mine = (LdsBytes)lds + wave * WAVE_BYTES;
-    const int k_swz = (li / RW) % CH;
-    const int v_row = 4 * lg + (li >> 2), v_swz = (v_row / RW) % (CH / 2);
-    const int v_off = v_row * ROW_BYTES + (((li & 3) >> 1) << 4) + ((li & 1) << 3);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) k_frag[ks] = mine + (li * ROW_BYTES + (((4 * ks + lg) ^ k_swz) << 4));
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) v_frag[dt] = mine + (BUF_BYTES + v_off + (((dt ^ v_swz) & (CH / 2 - 1)) << 5));
-  }
-
   // Key-side relocation: the shared rows of a chunk are rotated in LDS once they have landed, with the arithmetic of
   // the stand-alone relocation kernel.  Lane -> row lane / 2, half of its (d, d + D/2) pairs.
-  if (MODE == MODE_KEY_SIDE) {
-    if (tid < 2 * D / 4) {
-      const float *src = (tid < D / 4 ? p.cos_tab : p.sin_tab) + (int64_t)shift * D + (tid % (D / 4)) * 4;
-      store16(lds_rope + tid * 4, load16(src));
-    }
-    __syncthreads();
-  }
   auto rotate_shared_rows = [&](int chunk, int sl) __attribute__((always_inline)) {
     constexpr int PAIRS = CH / 2;
-    const int row = lane / 2;
+    const int lane = opaque_tid() & 63, row = lane / 2;
     const int delta = chunk * BN + row - sl, ad = delta < 0 ? -delta : delta;
     if (sl >= 0 && sl < p.shared_prefix_len && delta != 0 && ad < p.rope_rows) {
       char *bytes = lds + wave * WAVE_BYTES + row * ROW_BYTES;
@@ -228,22 +174,91 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
   const uint32_t one2 = M::pack2(1.0f, 1.0f);
   const vec16 ones{{one2, one2, one2, one2}};
 
-  if (wave < n_chunks) {
-    load_slots(0);                            // slots, queries and then the first chunk: two memory round trips
-    load_q(MODE == MODE_QUERY_SIDE && wave < chunks_a);
-    take_slots(0);
-    copy_chunk(kc_base, k_piece, k_dst);
-    copy_chunk(vc_base, v_piece, k_dst + BUF_BYTES);
-    settle_q();
+  // ---- set-up: slots, queries and cos / sin rows in one round trip, the first chunks in the next ---------------------
+  // The query rows lie in LDS like a chunk of keys, next to the counter-rotated q' in query-side mode, which scores the
+  // shared keys against q' and the others against q: a wave holds one of the two and reads q when its shared chunks are done.
+  // (Plain mode at head dim 64: half as many bytes and no rotation, so every wave reads the rows for itself, 0.4 us less of a
+  // call of 8 us.)
+  constexpr bool STAGE_Q = D == 128 || MODE != MODE_PLAIN;
+  vec16 qf[NQ16][KS];
+  load_slots(0);
+  if (!STAGE_Q) {
+#pragma unroll
+    for (int qt = 0; qt < NQ16; ++qt) {
+      const int row = qt * 16 + li < rows ? qt * 16 + li : rows - 1;
+      const char *src = p.q + (int64_t)(q_row0 + row) * p.q_token_bytes + (int64_t)head * p.q_head_bytes;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) qf[qt][ks] = load16(src + (32 * ks + 8 * lg) * 2);
+    }
+  } else if (wave < QROWS / RPI) {
+    // (rows past the end repeat the last one and are not stored)
+    const int row = wave * RPI + dma_row;
+    const char *src = p.q + (int64_t)(q_row0 + (row < rows ? row : rows - 1)) * p.q_token_bytes + (int64_t)head * p.q_head_bytes +
+                      ((dma_piece ^ ((row / RW) % CH)) << 4);
+    lds_dma16_at(src, __builtin_amdgcn_readfirstlane(lds_offset_of(lds_q) + (uint32_t)(wave * RPI * ROW_BYTES)));
   }
+  if (MODE != MODE_PLAIN && wave == 0) {  // (at head dim 64 both rows twice)
+    const float *row = (lane / (D / 4) % 2 == 0 ? p.cos_tab : p.sin_tab) + (int64_t)shift * D;
+    lds_dma16_at(reinterpret_cast<const char *>(row) + (lane % (D / 4)) * 16, __builtin_amdgcn_readfirstlane(lds_offset_of((const char *)lds_rope)));
+  }
+  take_slots(0);
+  copy_chunk(kc_base, k_piece, k_dst);      // (a wave without a chunk copies zero rows)
+  copy_chunk(vc_base, v_piece, k_dst + BUF_BYTES);
+  if (STAGE_Q) {
+    wait_copies<2 * NI>();                  // queries and table rows have landed
+    __syncthreads();
+  }
+  auto read_q = [&](const char *from) __attribute__((always_inline)) {
+    const int swz = (li / RW) % CH;
+#pragma unroll
+    for (int qt = 0; qt < NQ16; ++qt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const u32x4 raw = *(__attribute__((address_space(3))) const u32x4 *)((LdsBytes)from + ((qt * 16 + li) * ROW_BYTES + (((4 * ks + lg) ^ swz) << 4)));
+        qf[qt][ks] = vec16{{raw.x, raw.y, raw.z, raw.w}};
+      }
+  };
+  if (MODE == MODE_QUERY_SIDE && shift != 0) {
+    constexpr int PAIRS = CH / 2;
+    if (tid < QROWS * PAIRS) {
+      const int row = tid / PAIRS, pair = tid % PAIRS, f = (row / RW) % CH;
+      const char *src = lds_q + row * ROW_BYTES;
+      char *dst = lds_q + QROWS * ROW_BYTES + row * ROW_BYTES;
+      vec16 lo = load16(src + ((pair ^ f) << 4)), hi = load16(src + (((pair + PAIRS) ^ f) << 4));
+      rotate_pair<DTYPE, D>(lo, hi, lds_rope, lds_rope + D, pair * 8, -1.0f);
+      store16(dst + ((pair ^ f) << 4), lo);
+      store16(dst + (((pair + PAIRS) ^ f) << 4), hi);
+    }
+    __syncthreads();
+  }
+  if (STAGE_Q) {
+    read_q(MODE == MODE_QUERY_SIDE && shift != 0 && wave < chunks_a ? lds_q + QROWS * ROW_BYTES : lds_q);
+  } else {
+#pragma unroll
+    for (int qt = 0; qt < NQ16; ++qt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) settle(qf[qt][ks]);  // (waited for here, not inside the loop)
+  }
+
+  // ---- fragment addresses ---------------------------------------------------------------------------------------
+  LdsBytes k_frag[KS], v_frag[DT];
+  {
+    const int lane = opaque_tid() & 63, li = lane & 15, lg = lane >> 4;
+    const LdsBytes mine = (LdsBytes)lds + wave * WAVE_BYTES;
+    const int k_swz = (li / RW) % CH;
+    const int v_row = 4 * lg + (li >> 2), v_swz = (v_row / RW) % (CH / 2);
+    const int v_off = v_row * ROW_BYTES + (((li & 3) >> 1) << 4) + ((li & 1) << 3);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) k_frag[ks] = mine + (li * ROW_BYTES + (((4 * ks + lg) ^ k_swz) << 4));
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) v_frag[dt] = mine + (BUF_BYTES + v_off + (((dt ^ v_swz) & (CH / 2 - 1)) << 5));
+  }
+
   int turn = 0;
   for (int chunk = wave; chunk < n_chunks; chunk += NW) {
     const TileRange r = tile_range_of(chunk, chunks_a, shared_len, kv_len, BN);
     const bool more = chunk + NW < n_chunks;
-    if (MODE == MODE_QUERY_SIDE && chunk >= chunks_a && chunk - NW < chunks_a && turn > 0) {
-      load_q(false);
-      settle_q();
-    }
+    if (MODE == MODE_QUERY_SIDE && chunk >= chunks_a && chunk - NW < chunks_a && turn > 0) read_q(lds_q);
     const int rot_now = rot_slot;
     if (more) take_slots(++turn);
 
@@ -310,8 +325,10 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
     }
   }
   __syncthreads();
-  for (int job = wave; job < NQ16 * DT; job += NW) {
-    const int qt = job / DT, dt = job % DT;
+  static_assert(NQ16 * DT % NW == 0, "the pairs are dealt evenly");
+#pragma unroll
+  for (int k = 0; k < NQ16 * DT / NW; ++k) {
+    const int job = wave + k * NW, qt = job / DT, dt = job % DT;
     float m[NW], top = -INFINITY, l = 0.0f;
     f32x4 o{0, 0, 0, 0};
 #pragma unroll
@@ -326,8 +343,8 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
       o += reinterpret_cast<const f32x4 *>(lds + w * WAVE_BYTES)[job * 64 + lane] * a;
     }
     const float inv = l > 0.0f ? 1.0f / l : 1.0f;
-    const int qr = q_row0 + qt * 16 + li;
-    if (qr < q_len) {
+    const int qr = qt * 16 + li;
+    if (qr < rows) {
       uint2 val;
       val.x = M::pack2(o[0] * inv, o[1] * inv);
       val.y = M::pack2(o[2] * inv, o[3] * inv);
@@ -338,30 +355,18 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
 
 template <int DTYPE, int D, int MODE>
 __global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
-  // the waves' buffers, their (reference, denominator) pairs, and in key-side mode the cos / sin rows of the shift
+  // the waves' buffers, the queries (and q'), the waves' (reference, denominator) pairs, the cos / sin rows of the shift
   __shared__ __attribute__((aligned(1024))) char lds[NW * 2 * 32 * D * 2];
+  __shared__ __attribute__((aligned(1024))) char lds_q[(MODE == MODE_QUERY_SIDE ? 2 : 1) * 32 * D * 2];
   __shared__ float stats[NW * 2 * 2 * 16];
-  __shared__ __attribute__((aligned(16))) float lds_rope[MODE == MODE_KEY_SIDE ? 2 * D : 4];
-  int rank, kvh, hg, b = 0, q_begin = 0, q_len = 0, tile_in_request = 0, kv_begin = 0, kv_len = 0;
+  __shared__ __attribute__((aligned(16))) float lds_rope[MODE == MODE_PLAIN ? 4 : 256];
+  int rank, kvh, hg;
   if (!block_to_tile_head(p, rank, kvh, hg)) return;
   // The grid holds num_tiles units per head: all of them, or one per request, and the others follow in a second turn.
-  if (p.B <= 64) {
-    int live = rank + 1;
-    for (; rank < live; rank += p.num_tiles) {
-      if (!locate_query_tile_lpt(p.cu_q, p.cu_k, p.B, 32, rank, b, q_begin, q_len, tile_in_request, kv_begin, kv_len, &live)) return;
-      short_attn_unit<DTYPE, D, MODE>(p, lds, stats, lds_rope, kvh, hg, b, q_begin, q_len, tile_in_request, kv_begin, kv_len);
-      __syncthreads();
-    }
-  } else {
-    for (; locate_query_tile(p.cu_q, p.B, 32, rank, b, q_begin, q_len, tile_in_request); rank += p.num_tiles) {
-      b = __builtin_amdgcn_readfirstlane(b);
-      kv_begin = p.cu_k[b];
-      short_attn_unit<DTYPE, D, MODE>(p, lds, stats, lds_rope, kvh, hg, b, __builtin_amdgcn_readfirstlane(q_begin),
-                                          __builtin_amdgcn_readfirstlane(q_len),
-                                          __builtin_amdgcn_readfirstlane(tile_in_request), kv_begin,
-                                          p.cu_k[b + 1] - kv_begin);
-      __syncthreads();
-    }
+  ShortUnit u;
+  for (; locate_short_unit<MODE>(p, 32, rank, u); rank += p.num_tiles) {
+    short_attn_unit<DTYPE, D, MODE>(p, lds, lds_q, stats, lds_rope, kvh, kvh * (p.H / p.H_kv) + hg, u);
+    __syncthreads();
   }
 }
 

@@ -101,3 +101,11 @@ def test_scores_far_below_zero(device, B, shared):
     _check([q, kc, vc, cu([32] * B), cu(kv), slots],
            dict(shared_prefix_len=shared, rope_cos=cos, rope_sin=sin, affix_shifts=torch.zeros(B, dtype=torch.int32),
                 shared_kv_lens=torch.full((B,), shared, dtype=torch.int32)), device)
+
+
+@pytest.mark.parametrize("mode", ["plain", "key", "query"])
+@pytest.mark.parametrize("H,Hkv,D,dtype", [(32, 32, 128, torch.bfloat16), (28, 4, 128, torch.float16), (16, 4, 64, torch.bfloat16)])
+@pytest.mark.parametrize("keys", [256, 400, 512])
+def test_one_head_per_unit_from_a_few_hundred_keys(device, mode, H, Hkv, D, dtype, keys):
+    """Batches of up to 256 units of one head take the wave-private form from 256, 400 or 512 keys on average."""
+    _check(*_case([32, 1, 17, 0, 33], [31, 97, -1, 64, 255], H, Hkv, D, dtype, mode, keys, keys_per_request=keys), device)
