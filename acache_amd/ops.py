@@ -20,6 +20,7 @@ from __future__ import annotations
 import os
 
 import math
+from contextlib import nullcontext
 from itertools import accumulate as _accumulate
 
 import torch
@@ -36,14 +37,23 @@ def _code(t: torch.Tensor) -> int:
         raise ValueError(f"unsupported dtype {t.dtype}; expected bfloat16, float16 or float32") from None
 
 
+# The host side of a launch.  A short call (the attention of one request: 13 to 15 us on the GPU) is bound by it, and
+# entering a device context and building a Stream object took 3.4 of its 16.5 us.
+_HERE = nullcontext()
+
+
+def _on(t: torch.Tensor):
+    """Context in which ``t``'s device is the current one: nothing to do where it already is."""
+    return _HERE if t.get_device() == torch.cuda.current_device() else torch.cuda.device(t.device)
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Handle of the stream that is current on ``t``'s device."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
-    if t is None or t.numel() == 0:
-        return None
-    return t.data_ptr()
+    return None if t is None else t.data_ptr() or None  # (0 for a tensor without elements)
 
 
 def _i32(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -104,7 +114,7 @@ def materialize_relocated_affix(
     cos, sin = _rope_f32(rope_cos), _rope_f32(rope_sin)
     assert cos.shape == sin.shape and cos.shape[1] == D
     lib = _lib.load()
-    with torch.cuda.device(k_cache.device):
+    with _on(k_cache):
         rc = lib.acache_materialize_relocated_affix(
             _ptr(k_cache), _ptr(v_cache), _ptr(cos), _ptr(sin),
             int(dst_slot), int(affix_len), int(affix_shift),
@@ -159,7 +169,7 @@ def relocate_rope_gather(
     assert out_k[0].is_contiguous() and out_v[0].is_contiguous()
     assert out_k.stride(0) == out_v.stride(0)
     lib = _lib.load()
-    with torch.cuda.device(k_cache.device):
+    with _on(k_cache):
         rc = lib.acache_relocate_rope_gather(
             _ptr(out_k), _ptr(out_v), _ptr(k_cache), _ptr(v_cache),
             _ptr(slots), _ptr(deltas), _ptr(cos), _ptr(sin),
@@ -191,7 +201,7 @@ def store_kvcache(
     num_slots = k_cache.numel() // D
     assert k_cache.is_contiguous() and v_cache.is_contiguous()
     lib = _lib.load()
-    with torch.cuda.device(key.device):
+    with _on(key):
         rc = lib.acache_kv_scatter(
             _ptr(k_cache), _ptr(v_cache), _ptr(key), _ptr(value), _ptr(slots),
             N, 1, num_heads, head_dim, _code(key), num_slots,
@@ -234,7 +244,7 @@ def rope_qk_scatter(
         slots = _i32(slot_mapping, "slot_mapping")
         num_slots = k_cache.numel() // (H_kv * D)
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _on(q):
         rc = lib.acache_rope_qk_scatter(
             _ptr(q), _ptr(k), _ptr(v) if slots is not None else None,
             _ptr(k_cache) if slots is not None else None, _ptr(v_cache) if slots is not None else None,
@@ -261,7 +271,7 @@ def argmax_confidence(logits: torch.Tensor, picks: torch.Tensor | None = None):
         assert picks_flat.numel() == R
         token = picks_flat
     lib = _lib.load()
-    with torch.cuda.device(logits.device):
+    with _on(logits):
         rc = lib.acache_argmax_confidence(
             _ptr(token) if picks is None else None, _ptr(conf), _ptr(flat), _ptr(picks_flat) if picks is not None else None,
             R, V, flat.stride(0) if R > 1 else max(V, flat.stride(0)), _code(flat), _stream(flat))
@@ -281,7 +291,7 @@ def commit_tokens(blocks: torch.Tensor, proposal: torch.Tensor, confidence: torc
     assert confidence.shape == blocks.shape and confidence.dtype == torch.float32 and confidence.is_contiguous()
     assert committed_rows.is_cuda and committed_rows.dtype == torch.int32 and committed_rows.numel() == 1
     lib = _lib.load()
-    with torch.cuda.device(blocks.device):
+    with _on(blocks):
         rc = lib.acache_commit_tokens(_ptr(blocks), _ptr(proposal), _ptr(confidence), _ptr(committed_rows),
                                       blocks.shape[0], blocks.shape[1], int(mask_id), float(threshold), _stream(blocks))
     _lib.check(rc, "commit_tokens")
@@ -294,7 +304,7 @@ def swiglu(gate_up: torch.Tensor, hidden: int) -> torch.Tensor:
     flat = gate_up.reshape(-1, 2 * hidden)
     out = torch.empty(flat.shape[0], hidden, dtype=gate_up.dtype, device=gate_up.device)
     lib = _lib.load()
-    with torch.cuda.device(gate_up.device):
+    with _on(gate_up):
         rc = lib.acache_swiglu(_ptr(out), _ptr(flat), flat.shape[0], hidden,
                                flat.stride(0) if flat.shape[0] > 1 else 2 * hidden, hidden, _code(flat), _stream(flat))
     _lib.check(rc, "swiglu")
@@ -318,7 +328,7 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tens
         total = torch.empty(M, d, dtype=x.dtype, device=x.device)
     stride = lambda t: t.stride(0) if M > 1 else d
     lib = _lib.load()
-    with torch.cuda.device(x.device):
+    with _on(x):
         rc = lib.acache_add_rms_norm(_ptr(total), _ptr(flat), _ptr(dl), _ptr(w), _ptr(y), M, d,
                                      d, stride(flat), stride(dl) if dl is not None else d, d, float(eps),
                                      _code(flat), _stream(flat))
@@ -377,7 +387,7 @@ def affix_importance(
     if isinstance(workspace, str):
         if workspace != "builtin":
             raise ValueError("workspace: a uint8 tensor, None or 'builtin'")
-        with torch.cuda.device(q.device):
+        with _on(q):
             rc = lib.acache_affix_importance_noalloc(*common, _stream(q))
         _lib.check(rc, "affix_importance_noalloc")
         return importance
@@ -385,7 +395,7 @@ def affix_importance(
     if workspace is None:
         workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=q.device)
     assert workspace.is_cuda and workspace.numel() * workspace.element_size() >= need
-    with torch.cuda.device(q.device):
+    with _on(q):
         rc = lib.acache_affix_importance(*common, _ptr(workspace), workspace.numel() * workspace.element_size(),
                                          _stream(q))
     _lib.check(rc, "affix_importance")
@@ -438,7 +448,7 @@ def build_slot_layout(lengths, affix_spans, anchors, block_tables: torch.Tensor,
     rpos = torch.empty(cu_rec[-1], dtype=torch.int32, device=device)
     rslot = torch.empty(cu_rec[-1], dtype=torch.int32, device=device)
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on(block_tables):
         rc = lib.acache_build_slot_layout(
             _ptr(read), _ptr(rpos) or read.data_ptr(), _ptr(rslot) or read.data_ptr(), _ptr(d_len), _ptr(d_rec),
             _ptr(d_start), _ptr(d_end), _ptr(d_anc), _ptr(d_anchors), _ptr(block_tables), B, block_tables.shape[1],
@@ -472,7 +482,7 @@ def kv_scatter_layers(
     slots = _i32(slot_mapping, "slot_mapping")
     assert slots.numel() == N
     lib = _lib.load()
-    with torch.cuda.device(key.device):
+    with _on(key):
         rc = lib.acache_kv_scatter(
             _ptr(k_cache), _ptr(v_cache), _ptr(key), _ptr(value), _ptr(slots),
             N, L, H, D, _code(key), S,
@@ -513,7 +523,7 @@ def topk_anchors(
         offsets = _i32(offsets, "offsets")
         assert offsets.numel() == B
     lib = _lib.load()
-    with torch.cuda.device(scores.device):
+    with _on(scores):
         rc = lib.acache_topk_anchors(
             _ptr(out), scores.data_ptr(), _ptr(cu_affix), _ptr(cu_k), _ptr(offsets),
             1 if largest else 0, B, out.element_size(), _stream(scores))
@@ -568,7 +578,7 @@ def block_table_slots(
     B, max_blocks = block_tables.shape
     out = torch.empty(int(total_k), dtype=torch.int32, device=block_tables.device)
     lib = _lib.load()
-    with torch.cuda.device(block_tables.device):
+    with _on(block_tables):
         rc = lib.acache_block_table_slots(
             _ptr(out), _ptr(block_tables), _ptr(cu_seqlens_k), B, max_blocks, int(block_size),
             int(total_k), _stream(block_tables))
@@ -612,7 +622,6 @@ def _varlen_attn(q, k_cache, v_cache, cu_q, cu_k, slots, scale, shared_prefix_le
     Hkv = k_cache.shape[-2]
     assert k_cache.shape[-1] == D and v_cache.shape == k_cache.shape
     assert v_cache.stride() == k_cache.stride() and v_cache.dtype == k_cache.dtype == q.dtype
-    num_slots = k_cache.numel() // (Hkv * D) if k_cache.is_contiguous() else None
     if k_cache.dim() == 4:
         assert k_cache.stride(0) == k_cache.shape[1] * k_cache.stride(1), "cache blocks must be contiguous"
         slot_stride, head_stride = k_cache.stride(1), k_cache.stride(2)
@@ -632,7 +641,7 @@ def _varlen_attn(q, k_cache, v_cache, cu_q, cu_k, slots, scale, shared_prefix_le
         plan_blocks = plan.shape[0]
         if plan_blocks == 0:
             plan = None
-    with torch.cuda.device(q.device):
+    with _on(q):
         rc = lib.acache_varlen_attn_planned(
             _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(cu_q), _ptr(cu_k), _ptr(slots),
             float(scale), int(shared_prefix_len), _ptr(shared_kv_lens), _ptr(affix_shifts),
@@ -761,7 +770,7 @@ def baseline_decode_attention(
         cu_k = torch.empty_like(cu_q)
         slots = torch.empty(int(total_k), dtype=torch.int32, device=device)
         lib = _lib.load()
-        with torch.cuda.device(device):
+        with _on(q):
             rc = lib.acache_decode_layout(
                 _ptr(cu_q), _ptr(cu_k), _ptr(slots), _ptr(seqlens), _ptr(tables), batch, query_len, max_blocks,
                 k_cache.shape[1], int(total_k), _stream(q))
