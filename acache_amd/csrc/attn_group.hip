@@ -220,7 +220,7 @@ __device__ __forceinline__ void group_attn_unit(const AttnParams &p, char *lds, 
       const char *src = lds_q + row * ROW_BYTES;
       char *dst = lds + q_rot_at(row / QROWS) + (row % QROWS) * ROW_BYTES;
       vec16 lo = load16(src + ((pair ^ f) << 4)), hi = load16(src + (((pair + PAIRS) ^ f) << 4));
-      rotate_pair<DTYPE, D>(lo, hi, lds_rope, lds_rope + D, pair * 8, -1.0f);
+      rotate_pair_half_fast<DTYPE>(lo, hi, lds_rope, lds_rope + D, pair * 8, D / 2, -1.0f);
       store16(dst + ((pair ^ f) << 4), lo);
       store16(dst + (((pair + PAIRS) ^ f) << 4), hi);
     }

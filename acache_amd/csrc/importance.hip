@@ -780,7 +780,7 @@ __global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(Importa
 #pragma nounroll
       for (int r = tid / PAIRS; r < now.rows; r += kFusedThreads / PAIRS) {
         vec16 lo = load16(q_rows + G::offset(r, ch)), hi = load16(q_rows + G::offset(r, ch + PAIRS));
-        rotate_pair_half<DTYPE>(lo, hi, cs, sn, 0, 8, -1.0f);
+        rotate_pair_half_fast<DTYPE>(lo, hi, cs, sn, 0, 8, -1.0f);  // (188 -> 100 instructions a turn of this loop)
         store16(q_rows + G::offset(r, ch), lo);
         store16(q_rows + G::offset(r, ch + PAIRS), hi);
       }
