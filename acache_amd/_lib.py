@@ -60,6 +60,10 @@ SIGNATURES = {
         c_int32, c_void_p]),
     "acache_decode_layout": (c_int32, [
         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int64, c_void_p]),
+    "acache_decode_attn": (c_int32, [
+        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int32, c_int32, c_int64,
+        c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int64,
+        c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p]),
     "acache_varlen_attn": (c_int32, [
         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
         c_float,

@@ -7,7 +7,10 @@
 
 namespace acache {
 
-enum { MODE_PLAIN = 0, MODE_KEY_SIDE = 1, MODE_QUERY_SIDE = 2 };
+// MODE_PAGED: plain attention of equal query blocks whose keys are given by lengths and block tables (the short-block
+// kernels only); everything else reads prefix sums and a slot map.
+enum { MODE_PLAIN = 0, MODE_KEY_SIDE = 1, MODE_QUERY_SIDE = 2, MODE_PAGED = 3 };
+constexpr bool relocates(int mode) { return mode == MODE_KEY_SIDE || mode == MODE_QUERY_SIDE; }
 
 // Source of absent rows for the global->LDS copies: a key past the end of its
 // range, or one whose slot lies outside the cache, is fetched from here, so the
@@ -35,6 +38,14 @@ struct AttnParams {
   int32_t H_kv;
   int32_t num_tiles;  // upper bound on the number of BM-row query tiles
   int32_t head_dim;   // real head_dim (read by the padded any-head_dim variant only)
+  // MODE_PAGED: up to 64 requests of q_block query rows and seqlens[b] keys, no more than total_k in all; key n of request b
+  // lies in block tables[b * max_blocks + (n >> block_shift)], absent where that is negative or past max_blocks
+  const int32_t *seqlens;
+  const int32_t *tables;
+  int64_t total_k;
+  int32_t max_blocks;
+  int32_t block_shift;
+  int32_t q_block;
   int32_t small_cache;  // 32-bit copy offsets reach the whole cache (read by the short-query kernel)
   int64_t num_slots;
   int64_t q_token_bytes, q_head_bytes;
@@ -146,11 +157,34 @@ template <int MODE>
 __device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, int rank, ShortUnit &u) {
   const int lane = opaque_tid() & 63;
   int shared = 0, shift = 0;
+  if (MODE == MODE_PAGED) {
+    const int tiles = (p.q_block + BM - 1) / BM;
+    u.b = rank / tiles;
+    u.tile = rank - u.b * tiles;
+    if (u.b >= p.B) return false;
+    const int len = lane < p.B ? p.seqlens[lane] : 0;
+    int before = lane < u.b ? len : 0;        // keys of the requests in front: the caller's total bounds them all
+    before += __builtin_amdgcn_update_dpp(0, before, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+    before += __builtin_amdgcn_update_dpp(0, before, 0x112, 0xf, 0xf, false);
+    before += __builtin_amdgcn_update_dpp(0, before, 0x114, 0xf, 0xf, false);
+    before += __builtin_amdgcn_update_dpp(0, before, 0x118, 0xf, 0xf, false);
+    int start = 0;
+#pragma unroll
+    for (int row = 0; row < 4; ++row) start += __builtin_amdgcn_readlane(before, 16 * row + 15);
+    const int64_t end = (int64_t)start + __builtin_amdgcn_readlane(len, u.b);
+    const int64_t from = start < 0 ? 0 : (start > p.total_k ? p.total_k : start);
+    u.q_begin = u.b * p.q_block;
+    u.q_len = p.q_block;
+    u.kv_begin = 0;
+    u.kv_len = (int)((end < 0 ? 0 : (end > p.total_k ? p.total_k : end)) - from);
+    u.shared_len = u.shift = 0;
+    return true;
+  }
   if (p.B <= 64) {
     const int l = lane < p.B ? lane : p.B - 1;
     const int q0 = p.cu_q[l], q1 = p.cu_q[l + 1], k0 = p.cu_k[l], k1 = p.cu_k[l + 1];
     if (MODE == MODE_QUERY_SIDE) shared = p.shared_kv_lens[l];
-    if (MODE != MODE_PLAIN) shift = p.affix_shifts[l];
+    if (relocates(MODE)) shift = p.affix_shifts[l];
     const int tiles = lane < p.B && q1 > q0 ? (q1 - q0 + BM - 1) / BM : 0;
     int src = rank;
     u.tile = 0;
@@ -174,7 +208,7 @@ __device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, i
     u.kv_begin = __builtin_amdgcn_readlane(k0, src);
     u.kv_len = __builtin_amdgcn_readlane(k1, src) - u.kv_begin;
     if (MODE == MODE_QUERY_SIDE) shared = __builtin_amdgcn_readlane(shared, src);
-    if (MODE != MODE_PLAIN) shift = __builtin_amdgcn_readlane(shift, src);
+    if (relocates(MODE)) shift = __builtin_amdgcn_readlane(shift, src);
   } else {
     if (!locate_query_tile(p.cu_q, p.B, BM, rank, u.b, u.q_begin, u.q_len, u.tile)) return false;
     u.b = __builtin_amdgcn_readfirstlane(u.b);
@@ -184,11 +218,20 @@ __device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, i
     u.kv_begin = p.cu_k[u.b];
     u.kv_len = p.cu_k[u.b + 1] - u.kv_begin;
     if (MODE == MODE_QUERY_SIDE) shared = p.shared_kv_lens[u.b];
-    if (MODE != MODE_PLAIN) shift = p.affix_shifts[u.b];
+    if (relocates(MODE)) shift = p.affix_shifts[u.b];
   }
   u.shared_len = shared < 0 ? 0 : (shared > u.kv_len ? u.kv_len : shared);
   u.shift = shift < 0 || shift >= p.rope_rows ? 0 : shift;
   return true;
+}
+
+// MODE_PAGED: the table entry of key n (a chunk of 32 keys lies in one block), and the slot of a key from it.
+__device__ __forceinline__ int table_entry(const AttnParams &p, int b, int n) {
+  const int block = n >> p.block_shift;
+  return block < p.max_blocks ? p.tables[(int64_t)b * p.max_blocks + block] : -1;
+}
+__device__ __forceinline__ int slot_of_entry(const AttnParams &p, int entry, int n) {
+  return entry < 0 ? -1 : (int)((uint32_t)entry << p.block_shift) + (n & ((1 << p.block_shift) - 1));
 }
 
 // Block -> (query tile rank, KV head, head inside its group) for the kernels that stream K/V per (tile, head).

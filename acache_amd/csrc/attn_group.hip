@@ -1,4 +1,5 @@
-// Varlen attention for grouped-query batches of short query blocks: head dim 128, all three relocation modes.
+// Varlen attention for grouped-query batches of short query blocks: head dim 128, all three relocation modes and block
+// tables.
 //
 // What bounds it: with a unit per query head (varlen_attn_unit_kernel) the heads of a group copy every key tile into LDS
 // once each, and 32 rows are so little work per key that a unit spends its time in the chain copy -> scores -> softmax ->
@@ -76,6 +77,10 @@ __device__ __forceinline__ void group_attn_unit(const AttnParams &p, char *lds, 
   const char *const slot_base = reinterpret_cast<const char *>(p.slot_map + kv_begin);
   auto load_slots = [&](int round) __attribute__((always_inline)) {
     const TileRange r = tile_range_of(round * W + stream, chunks_a, shared_len, kv_len, BN);
+    if (MODE == MODE_PAGED) {                 // one table entry for the chunk; take_slots makes the slots of it
+      slot_next[0] = r.n0 < r.n_end ? table_entry(p, u.b, r.n0) : -1;
+      return;
+    }
     const int rot_row = which * RPW + lane / (64 / RPW);
     if (r.n0 + BN <= r.n_end) {               // (wave-uniform) a scalar base, one offset per lane, immediates
       const char *const base = slot_base + (int64_t)r.n0 * 4;
@@ -97,11 +102,13 @@ __device__ __forceinline__ void group_attn_unit(const AttnParams &p, char *lds, 
     }
   };
   bool all_present = false;
-  auto take_slots = [&]() __attribute__((always_inline)) {
+  auto take_slots = [&](int round) __attribute__((always_inline)) {
     bool ok = true;
+    const int first = (round * W + stream) * BN + dma_row;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      slot[i] = slot_next[i];
+      if (MODE == MODE_PAGED) slot[i] = first + i * RPI < kv_len ? slot_of_entry(p, slot_next[0], first + i * RPI) : -1;
+      else slot[i] = slot_next[i];
       asm volatile("" : "+v"(slot[i]));       // (waited for here, in front of the next copies)
       ok &= (uint32_t)slot[i] < slot_limit;
     }
@@ -189,11 +196,11 @@ __device__ __forceinline__ void group_attn_unit(const AttnParams &p, char *lds, 
   }
   if (lane == 0) landed[wave] = 0;
   static_assert(2 * D * 4 == 64 * 16, "cos and sin row are one copy instruction");
-  if (MODE != MODE_PLAIN && wave == 0) {
+  if (relocates(MODE) && wave == 0) {
     const float *row = (lane < 32 ? p.cos_tab : p.sin_tab) + (int64_t)shift * D;
     lds_dma16_at(reinterpret_cast<const char *>(row) + (lane % 32) * 16, __builtin_amdgcn_readfirstlane(lds_offset_of((const char *)lds_rope)));
   }
-  take_slots();
+  take_slots(0);
   copy_round(my_dst);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI) : "memory");  // queries and table rows have landed
   __syncthreads();
@@ -274,7 +281,7 @@ __device__ __forceinline__ void group_attn_unit(const AttnParams &p, char *lds, 
         kf[nt][ks] = vec16{{raw.x, raw.y, raw.z, raw.w}};
       }
     if (more) {
-      take_slots();
+      take_slots(round + 1);
       if (round + 2 < rounds) load_slots(round + 2);
       copy_round(my_dst + THERE);
     }
@@ -370,7 +377,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 1) void group_attn_kernel(AttnPar
   char *const lds_q = lds + RING;
   __shared__ int landed[GROUP_WAVES];
   __shared__ float stats[GROUP_WAVES * 2 * 2 * 16];
-  __shared__ __attribute__((aligned(16))) float lds_rope[MODE == MODE_PLAIN ? 4 : 2 * D];
+  __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 2 * D : 4];
   const int group = p.H / p.H_kv;
   int rank, kvh, slice;
   if (!block_to_tile_slice(p, (group + HU - 1) / HU, rank, kvh, slice)) return;
@@ -398,7 +405,8 @@ int group_attention(const AttnParams &p, int heads_per_unit, int mode, int dtype
 #define ACACHE_GROUP_ALL(DT, HU)            \
   ACACHE_GROUP_MODE(DT, HU, MODE_PLAIN)     \
   ACACHE_GROUP_MODE(DT, HU, MODE_KEY_SIDE)  \
-  ACACHE_GROUP_MODE(DT, HU, MODE_QUERY_SIDE)
+  ACACHE_GROUP_MODE(DT, HU, MODE_QUERY_SIDE) \
+  ACACHE_GROUP_MODE(DT, HU, MODE_PAGED)
   ACACHE_GROUP_ALL(ACACHE_BF16, 2)
   ACACHE_GROUP_ALL(ACACHE_F16, 2)
   ACACHE_GROUP_ALL(ACACHE_BF16, 4)

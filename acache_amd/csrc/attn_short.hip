@@ -1,5 +1,5 @@
 // Varlen attention for batches of short query blocks (refinement steps: the 32 tokens of a generation block against
-// a thousand cached keys), head dims 64 and 128, all three relocation modes.
+// a thousand cached keys), head dims 64 and 128, all three relocation modes and block tables.
 //
 // What bounds it: 32 query rows are so little matrix work per key that a workgroup whose waves share every key tile
 // spends its time in the chain copy -> barrier -> LDS read -> scores -> softmax -> LDS read -> output, one tile after
@@ -79,6 +79,10 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
 #pragma unroll
     for (int j = 0; j < SLOT_REGS; ++j) {
       const TileRange r = tile_range_of(wave + (turn + 2 * j + (lane >> 5)) * NW, chunks_a, shared_len, kv_len, BN);
+      if (MODE == MODE_PAGED) {               // one table entry for the chunk; take_slots makes the slots of it
+        slots[j] = r.n0 < r.n_end ? table_entry(p, u.b, r.n0) : -1;
+        continue;
+      }
       const int n = r.n0 + (lane & 31);
       const int s = p.slot_map[kv_begin + (n < kv_len ? n : kv_len - 1)];
       slots[j] = n < r.n_end ? s : -1;
@@ -116,6 +120,10 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       slot[i] = __shfl(slots[0], (turn % 2) * 32 + i * RPI + dma_row);
+      if (MODE == MODE_PAGED) {
+        const int n = (wave + turn * NW) * BN + i * RPI + dma_row;
+        slot[i] = n < kv_len ? slot_of_entry(p, slot[i], n) : -1;
+      }
       ok &= (uint32_t)slot[i] < slot_limit;
     }
     if (MODE == MODE_KEY_SIDE) rot_slot = __shfl(slots[0], (turn % 2) * 32 + lane / 2);
@@ -179,7 +187,7 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
   // shared keys against q' and the others against q: a wave holds one of the two and reads q when its shared chunks are done.
   // (Plain mode at head dim 64: half as many bytes and no rotation, so every wave reads the rows for itself, 0.4 us less of a
   // call of 8 us.)
-  constexpr bool STAGE_Q = D == 128 || MODE != MODE_PLAIN;
+  constexpr bool STAGE_Q = D == 128 || relocates(MODE);
   vec16 qf[NQ16][KS];
   load_slots(0);
   if (!STAGE_Q) {
@@ -197,7 +205,7 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
                       ((dma_piece ^ ((row / RW) % CH)) << 4);
     lds_dma16_at(src, __builtin_amdgcn_readfirstlane(lds_offset_of(lds_q) + (uint32_t)(wave * RPI * ROW_BYTES)));
   }
-  if (MODE != MODE_PLAIN && wave == 0) {  // (at head dim 64 both rows twice)
+  if (relocates(MODE) && wave == 0) {  // (at head dim 64 both rows twice)
     const float *row = (lane / (D / 4) % 2 == 0 ? p.cos_tab : p.sin_tab) + (int64_t)shift * D;
     lds_dma16_at(reinterpret_cast<const char *>(row) + (lane % (D / 4)) * 16, __builtin_amdgcn_readfirstlane(lds_offset_of((const char *)lds_rope)));
   }
@@ -359,7 +367,7 @@ __global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(1024))) char lds[NW * 2 * 32 * D * 2];
   __shared__ __attribute__((aligned(1024))) char lds_q[(MODE == MODE_QUERY_SIDE ? 2 : 1) * 32 * D * 2];
   __shared__ float stats[NW * 2 * 2 * 16];
-  __shared__ __attribute__((aligned(16))) float lds_rope[MODE == MODE_PLAIN ? 4 : 256];
+  __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 256 : 4];
   int rank, kvh, hg;
   if (!block_to_tile_head(p, rank, kvh, hg)) return;
   // The grid holds num_tiles units per head: all of them, or one per request, and the others follow in a second turn.
@@ -385,7 +393,8 @@ int short_attention(const AttnParams &p, int mode, int dtype, hipStream_t stream
 #define ACACHE_SHORT_ALL(DT, DD)            \
   ACACHE_SHORT_MODE(DT, DD, MODE_PLAIN)     \
   ACACHE_SHORT_MODE(DT, DD, MODE_KEY_SIDE)  \
-  ACACHE_SHORT_MODE(DT, DD, MODE_QUERY_SIDE)
+  ACACHE_SHORT_MODE(DT, DD, MODE_QUERY_SIDE) \
+  ACACHE_SHORT_MODE(DT, DD, MODE_PAGED)
   ACACHE_SHORT_ALL(ACACHE_BF16, 128)
   ACACHE_SHORT_ALL(ACACHE_BF16, 64)
   ACACHE_SHORT_ALL(ACACHE_F16, 128)

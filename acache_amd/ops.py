@@ -616,20 +616,22 @@ def attention_plan(cu_seqlens_q, cu_seqlens_k, num_heads: int, num_kv_heads: int
     return plan.to(device, non_blocking=True)
 
 
+def _attn_cache(q, k_cache, v_cache):
+    """(slots, slot stride, head stride) of the caches that ``q`` (``[tokens, H, D]``) attends to."""
+    assert k_cache.shape[-1] == q.shape[-1] and v_cache.shape == k_cache.shape
+    assert v_cache.stride() == k_cache.stride() and v_cache.dtype == k_cache.dtype == q.dtype
+    if k_cache.dim() == 4:
+        assert k_cache.stride(0) == k_cache.shape[1] * k_cache.stride(1), "cache blocks must be contiguous"
+        return k_cache.shape[0] * k_cache.shape[1], k_cache.stride(1), k_cache.stride(2)
+    assert k_cache.dim() == 3
+    return k_cache.shape[0], k_cache.stride(0), k_cache.stride(1)
+
+
 def _varlen_attn(q, k_cache, v_cache, cu_q, cu_k, slots, scale, shared_prefix_len,
                  shared_kv_lens, affix_shifts, cos, sin, plan=None):
     total_q, H, D = q.shape
     Hkv = k_cache.shape[-2]
-    assert k_cache.shape[-1] == D and v_cache.shape == k_cache.shape
-    assert v_cache.stride() == k_cache.stride() and v_cache.dtype == k_cache.dtype == q.dtype
-    if k_cache.dim() == 4:
-        assert k_cache.stride(0) == k_cache.shape[1] * k_cache.stride(1), "cache blocks must be contiguous"
-        slot_stride, head_stride = k_cache.stride(1), k_cache.stride(2)
-        num_slots = k_cache.shape[0] * k_cache.shape[1]
-    else:
-        assert k_cache.dim() == 3
-        slot_stride, head_stride = k_cache.stride(0), k_cache.stride(1)
-        num_slots = k_cache.shape[0]
+    num_slots, slot_stride, head_stride = _attn_cache(q, k_cache, v_cache)
     out = torch.empty_like(q)
     B = cu_q.numel() - 1
     rope_rows = 0 if cos is None else cos.shape[0]
@@ -766,22 +768,27 @@ def baseline_decode_attention(
             tables = torch.nn.functional.pad(tables, (0, 0, 0, batch - rows), value=-1)
         if seqlens.device != device or tables.device != device:
             seqlens, tables = seqlens.to(device), tables.to(device)
-        cu_q = torch.empty(batch + 1, dtype=torch.int32, device=device)
-        cu_k = torch.empty_like(cu_q)
-        slots = torch.empty(int(total_k), dtype=torch.int32, device=device)
+        total_k = int(total_k)
+        q3 = q.reshape(batch * query_len, num_heads, head_dim)
+        num_slots, slot_stride, head_stride = _attn_cache(q3, k_cache, v_cache)
+        out = torch.empty_like(q3)
+        scratch = torch.empty(2 * (batch + 1) + total_k, dtype=torch.int32, device=device)
         lib = _lib.load()
         with _on(q):
-            rc = lib.acache_decode_layout(
-                _ptr(cu_q), _ptr(cu_k), _ptr(slots), _ptr(seqlens), _ptr(tables), batch, query_len, max_blocks,
-                k_cache.shape[1], int(total_k), _stream(q))
-        _lib.check(rc, "decode_layout")
-    else:  # nothing to lay out, more requests than one launch covers, or lengths that broadcast
-        cu_k = torch.zeros(batch + 1, dtype=torch.int32, device=q.device)
-        cu_k[1:] = torch.cumsum(seqlens, 0)
-        if total_k is None:
-            total_k = int(cu_k[-1].item())
-        cu_q = torch.arange(0, (batch + 1) * query_len, query_len, dtype=torch.int32, device=q.device)
-        slots = block_table_slots(block_tables, cu_k, k_cache.shape[1], total_k)
+            rc = lib.acache_decode_attn(
+                _ptr(out), _ptr(q3), _ptr(k_cache), _ptr(v_cache), _ptr(seqlens), _ptr(tables), _ptr(scratch),
+                float(softmax_scale), batch, query_len, total_k, max_blocks, k_cache.shape[1], num_heads,
+                k_cache.shape[-2], head_dim, _code(q), num_slots, q3.stride(0), q3.stride(1), out.stride(0), out.stride(1),
+                slot_stride, head_stride, _stream(q))
+        _lib.check(rc, "baseline_decode_attention")
+        return out.view(batch, query_len, num_heads, head_dim)
+    # nothing to lay out, more requests than one launch covers, or lengths that broadcast
+    cu_k = torch.zeros(batch + 1, dtype=torch.int32, device=q.device)
+    cu_k[1:] = torch.cumsum(seqlens, 0)
+    if total_k is None:
+        total_k = int(cu_k[-1].item())
+    cu_q = torch.arange(0, (batch + 1) * query_len, query_len, dtype=torch.int32, device=q.device)
+    slots = block_table_slots(block_tables, cu_k, k_cache.shape[1], total_k)
     q3 = q.reshape(batch * query_len, num_heads, head_dim)
     out = _varlen_attn(q3, k_cache, v_cache, cu_q, cu_k, slots, softmax_scale, 0, None, None, None, None)
     return out.view(batch, query_len, num_heads, head_dim)

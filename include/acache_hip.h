@@ -335,6 +335,21 @@ int acache_decode_layout(
     int32_t block_size, int64_t total_k, void *stream);
 
 /*
+ * Plain attention of B blocks of q_len query rows against the first seqlens[b] keys of each request's block table:
+ * acache_decode_layout followed by acache_varlen_attn, and one launch where the kernel the call takes reads lengths and
+ * tables itself (blocks of at most 32 rows on up to 64 requests, cache blocks of a power of two of at least 32 tokens).
+ * q: [B * q_len, H, D] by its strides (elements), block_tables: [B, max_blocks] (negative entries: absent keys), scratch:
+ * 2 * (B + 1) + total_k int32 that the launch in front of the other kernels fills.  Lengths that sum to more than total_k
+ * are cut there.  Block-table decode of the reference (nano-vdllm/model/acache_attention.py:585-640).
+ */
+int acache_decode_attn(
+    void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *seqlens,
+    const int32_t *block_tables, int32_t *scratch, float scale, int32_t B, int32_t q_len, int64_t total_k,
+    int32_t max_blocks, int32_t block_size, int32_t H, int32_t H_kv, int32_t D, int32_t dtype, int64_t num_slots,
+    int64_t q_token_stride, int64_t q_head_stride, int64_t out_token_stride, int64_t out_head_stride,
+    int64_t kv_slot_stride, int64_t kv_head_stride, void *stream);
+
+/*
  * Slot layout of a batch of requests that reuse a shared affix (device-side form of
  * Sequence.finalize_slot_mapping, nano-vdllm/sequence.py:169-202, which the reference
  * evaluates per request in Python before prepare_caching_acache,
