@@ -1212,7 +1212,7 @@ static int attention_call(
       return rc;
     }
   }
-  if (takes_short) return short_attention(p, short_mode, dtype, st);
+  if (takes_short) return short_attention(p, (total_q % B == 0 ? B : (int64_t)p.num_tiles) * H, short_mode, dtype, st);
   if (heads) return group_attention(p, heads, short_mode, dtype, st);
   if (takes_pair_kernel(p, total_q))
     return dtype == ACACHE_BF16 ? launch_pairs<ACACHE_BF16, 128>(p, mode, total_q, st)

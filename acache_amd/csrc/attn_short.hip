@@ -35,20 +35,24 @@ template <int N> __device__ __forceinline__ void wait_copies() { asm volatile("s
 // this wave's LDS reads have returned: their buffer may be filled again
 __device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// One unit: 32 query rows (query tile `tile_in_request` of request b) of one head.
-template <int DTYPE, int D, int MODE>
+// One unit: 32 query rows (query tile `tile_in_request` of request b) of one head, or its part `part` of FS: all scores, and
+// D / FS features of the values and of the output.
+template <int DTYPE, int D, int MODE, int FS>
 __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, char *lds_q, float *stats, float *lds_rope,
-                                                int kvh, int head, const ShortUnit &u) {
+                                                int kvh, int head, int part, const ShortUnit &u) {
   constexpr int QROWS = 32, NQ16 = 2;         // query rows of a unit
   constexpr int BN = 32;                      // keys per chunk
-  constexpr int KS = D / 32, DT = D / 16;
+  constexpr int KS = D / 32, DT = D / FS / 16;
   constexpr int ROW_BYTES = D * 2;
   constexpr int CH = ROW_BYTES / 16;          // 16-byte pieces per row
   constexpr int RW = 256 / ROW_BYTES;         // rows per 256-byte bank window
   constexpr int RPI = 64 / CH;                // rows per copy instruction
   constexpr int NI = BN / RPI;                // copy instructions per chunk and tensor
   constexpr int BUF_BYTES = BN * ROW_BYTES;
-  constexpr int WAVE_BYTES = 2 * BUF_BYTES;   // a wave's K buffer, then its V buffer
+  // the same of this part's values: D / FS features of a row
+  constexpr int V_ROW_BYTES = ROW_BYTES / FS, V_CH = CH / FS, V_RW = 256 / V_ROW_BYTES, V_RPI = 64 / V_CH, V_NI = BN / V_RPI;
+  static_assert(V_NI >= 1 && V_CH >= 4, "whole copy instructions");
+  constexpr int WAVE_BYTES = BUF_BYTES + BN * V_ROW_BYTES;  // a wave's K buffer, then its V buffer
   using M = Mma<DTYPE>;
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -59,11 +63,11 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
   const int kv_begin = u.kv_begin, kv_len = u.kv_len, shared_len = u.shared_len, shift = u.shift;
   const int q_row0 = u.q_begin + u.tile * QROWS;
   const int rows = u.q_len - u.tile * QROWS < QROWS ? u.q_len - u.tile * QROWS : QROWS;
-  char *const out_base = p.out + (int64_t)q_row0 * p.o_token_bytes + (int64_t)head * p.o_head_bytes;
+  char *const out_base = p.out + (int64_t)q_row0 * p.o_token_bytes + (int64_t)head * p.o_head_bytes + part * V_ROW_BYTES;
 
   if (kv_len <= 0) {  // no keys: defined output (zeros)
-    for (int r = tid / CH; r < rows; r += 64 * NW / CH)
-      store16(out_base + (int64_t)r * p.o_token_bytes + (tid % CH) * 16, vec16{{0, 0, 0, 0}});
+    for (int r = tid / V_CH; r < rows; r += 64 * NW / V_CH)
+      store16(out_base + (int64_t)r * p.o_token_bytes + (tid % V_CH) * 16, vec16{{0, 0, 0, 0}});
     return;
   }
 
@@ -94,18 +98,19 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
   };
   const int dma_row = lane / CH, dma_piece = lane % CH;
   const char *const kc_base = uniform_ptr(p.k_cache + (int64_t)kvh * p.kv_head_bytes);
-  const char *const vc_base = uniform_ptr(p.v_cache + (int64_t)kvh * p.kv_head_bytes);
+  const char *const vc_base = uniform_ptr(p.v_cache + (int64_t)kvh * p.kv_head_bytes + part * V_ROW_BYTES);
   // byte offset of this lane's (swizzled) piece inside its row of copy i: the layouts of attn_dma_part
   auto k_piece = [&](int i) __attribute__((always_inline)) {
     return (uint32_t)((dma_piece ^ (((i * RPI + dma_row) / RW) % CH)) << 4);
   };
+  const int v_dma_row = lane / V_CH, v_dma_piece = lane % V_CH;
   auto v_piece = [&](int i) __attribute__((always_inline)) {
-    return (uint32_t)((dma_piece ^ (2 * (((i * RPI + dma_row) / RW) % (CH / 2)))) << 4);
+    return (uint32_t)((v_dma_piece ^ (2 * (((i * V_RPI + v_dma_row) / V_RW) % (V_CH / 2)))) << 4);
   };
   const uint32_t slot_limit = p.num_slots > 0x7fffffffLL ? 0x7fffffffu : (uint32_t)p.num_slots;
   const uint32_t slot_pitch = (uint32_t)p.kv_slot_bytes;
   const uint32_t k_dst = __builtin_amdgcn_readfirstlane(lds_offset_of(lds) + (uint32_t)(wave * WAVE_BYTES));
-  int slot[NI];                               // this lane's slots in the chunk being copied; -1: absent
+  int slot[NI], v_slot[V_NI];                 // this lane's slots in the chunk being copied; -1: absent
   bool all_present = false;
   int rot_slot = -1;                          // key-side mode: slot of row lane / 2 of that chunk
   auto take_slots = [&](int turn) __attribute__((always_inline)) {
@@ -117,31 +122,42 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
       for (int j = 0; j + 1 < SLOT_REGS; ++j) slots[j] = slots[j + 1];
     }
     bool ok = true;
+    auto slot_of_row = [&](int row) __attribute__((always_inline)) {
+      int s = __shfl(slots[0], (turn % 2) * 32 + row);
+      if (MODE == MODE_PAGED) {
+        const int n = (wave + turn * NW) * BN + row;
+        s = n < kv_len ? slot_of_entry(p, s, n) : -1;
+      }
+      return s;
+    };
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      slot[i] = __shfl(slots[0], (turn % 2) * 32 + i * RPI + dma_row);
-      if (MODE == MODE_PAGED) {
-        const int n = (wave + turn * NW) * BN + i * RPI + dma_row;
-        slot[i] = n < kv_len ? slot_of_entry(p, slot[i], n) : -1;
-      }
+      slot[i] = slot_of_row(i * RPI + dma_row);
       ok &= (uint32_t)slot[i] < slot_limit;
     }
+#pragma unroll
+    for (int i = 0; i < V_NI; ++i) v_slot[i] = FS == 1 ? slot[FS == 1 ? i : 0] : slot_of_row(i * V_RPI + v_dma_row);
     if (MODE == MODE_KEY_SIDE) rot_slot = __shfl(slots[0], (turn % 2) * 32 + lane / 2);
     all_present = p.small_cache && __builtin_amdgcn_ballot_w64(!ok) == 0;
   };
-  auto copy_chunk = [&](const char *base, auto piece, uint32_t dst) __attribute__((always_inline)) {
+  auto copy_rows = [&]<int N>(const char *base, const int (&rows_slot)[N], int first, auto piece,
+                              uint32_t dst) __attribute__((always_inline)) {
     if (all_present) {  // wave-uniform base + 32-bit offsets
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
-        lds_dma16_off(base, __umul24((uint32_t)slot[i], slot_pitch) + piece(i), dst + i * RPI * ROW_BYTES);
+      for (int i = 0; i < N; ++i)
+        lds_dma16_off(base, __umul24((uint32_t)rows_slot[i], slot_pitch) + piece(i), dst + i * 1024);
     } else {            // absent rows come from the zero row
-      const char *zero = reinterpret_cast<const char *>(kZeroRow) + (dma_piece << 4);
+      const char *zero = reinterpret_cast<const char *>(kZeroRow) + (first << 4);
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const char *src = base + ((uint64_t)(uint32_t)slot[i] * slot_pitch + piece(i));
-        lds_dma16_at((uint32_t)slot[i] < slot_limit ? src : zero, dst + i * RPI * ROW_BYTES);
+      for (int i = 0; i < N; ++i) {
+        const char *src = base + ((uint64_t)(uint32_t)rows_slot[i] * slot_pitch + piece(i));
+        lds_dma16_at((uint32_t)rows_slot[i] < slot_limit ? src : zero, dst + i * 1024);
       }
     }
+  };
+  auto copy_keys = [&]() __attribute__((always_inline)) { copy_rows(kc_base, slot, dma_piece, k_piece, k_dst); };
+  auto copy_values = [&]() __attribute__((always_inline)) {
+    copy_rows(vc_base, v_slot, v_dma_piece, v_piece, k_dst + BUF_BYTES);
   };
 
   typedef __attribute__((address_space(3))) const char *LdsBytes;
@@ -210,10 +226,10 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
     lds_dma16_at(reinterpret_cast<const char *>(row) + (lane % (D / 4)) * 16, __builtin_amdgcn_readfirstlane(lds_offset_of((const char *)lds_rope)));
   }
   take_slots(0);
-  copy_chunk(kc_base, k_piece, k_dst);      // (a wave without a chunk copies zero rows)
-  copy_chunk(vc_base, v_piece, k_dst + BUF_BYTES);
+  copy_keys();                              // (a wave without a chunk copies zero rows)
+  copy_values();
   if (STAGE_Q) {
-    wait_copies<2 * NI>();                  // queries and table rows have landed
+    wait_copies<NI + V_NI>();               // queries and table rows have landed
     __syncthreads();
   }
   auto read_q = [&](const char *from) __attribute__((always_inline)) {
@@ -254,12 +270,12 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
     const int lane = opaque_tid() & 63, li = lane & 15, lg = lane >> 4;
     const LdsBytes mine = (LdsBytes)lds + wave * WAVE_BYTES;
     const int k_swz = (li / RW) % CH;
-    const int v_row = 4 * lg + (li >> 2), v_swz = (v_row / RW) % (CH / 2);
-    const int v_off = v_row * ROW_BYTES + (((li & 3) >> 1) << 4) + ((li & 1) << 3);
+    const int v_row = 4 * lg + (li >> 2), v_swz = (v_row / V_RW) % (V_CH / 2);
+    const int v_off = v_row * V_ROW_BYTES + (((li & 3) >> 1) << 4) + ((li & 1) << 3);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) k_frag[ks] = mine + (li * ROW_BYTES + (((4 * ks + lg) ^ k_swz) << 4));
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) v_frag[dt] = mine + (BUF_BYTES + v_off + (((dt ^ v_swz) & (CH / 2 - 1)) << 5));
+    for (int dt = 0; dt < DT; ++dt) v_frag[dt] = mine + (BUF_BYTES + v_off + (((dt ^ v_swz) & (V_CH / 2 - 1)) << 5));
   }
 
   int turn = 0;
@@ -270,7 +286,7 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
     const int rot_now = rot_slot;
     if (more) take_slots(++turn);
 
-    wait_copies<NI>();                        // the keys have landed (the values, issued behind them, may not have)
+    wait_copies<V_NI>();                      // the keys have landed (the values, issued behind them, may not have)
     if (MODE == MODE_KEY_SIDE) {
       rotate_shared_rows(chunk, rot_now);
       wait_lds_reads();
@@ -284,7 +300,7 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
         kf[nt][ks] = vec16{{raw.x, raw.y, raw.z, raw.w}};
       }
     wait_lds_reads();
-    if (more) copy_chunk(kc_base, k_piece, k_dst);
+    if (more) copy_keys();
     f32x4 s_acc[NQ16][2];
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt)
@@ -306,11 +322,11 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)v_frag[dt]));
-      const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(v_frag[dt] + 16 * ROW_BYTES)));
+      const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(v_frag[dt] + 16 * V_ROW_BYTES)));
       vf[dt] = vec16{{lo.x, lo.y, hi.x, hi.y}};
     }
     wait_lds_reads();
-    if (more) copy_chunk(vc_base, v_piece, k_dst + BUF_BYTES);
+    if (more) copy_values();
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -333,9 +349,10 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
     }
   }
   __syncthreads();
-  static_assert(NQ16 * DT % NW == 0, "the pairs are dealt evenly");
+  if (NQ16 * DT < NW && wave >= NQ16 * DT) return;
 #pragma unroll
-  for (int k = 0; k < NQ16 * DT / NW; ++k) {
+  for (int k = 0; k < (NQ16 * DT + NW - 1) / NW; ++k) {
+    static_assert(NQ16 * DT % NW == 0 || NQ16 * DT < NW, "the pairs are dealt evenly");
     const int job = wave + k * NW, qt = job / DT, dt = job % DT;
     float m[NW], top = -INFINITY, l = 0.0f;
     f32x4 o{0, 0, 0, 0};
@@ -361,35 +378,50 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
   }
 }
 
-template <int DTYPE, int D, int MODE>
+template <int DTYPE, int D, int MODE, int FS>
 __global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
   // the waves' buffers, the queries (and q'), the waves' (reference, denominator) pairs, the cos / sin rows of the shift
-  __shared__ __attribute__((aligned(1024))) char lds[NW * 2 * 32 * D * 2];
+  __shared__ __attribute__((aligned(1024))) char lds[NW * 32 * (D + D / FS) * 2];
   __shared__ __attribute__((aligned(1024))) char lds_q[(MODE == MODE_QUERY_SIDE ? 2 : 1) * 32 * D * 2];
   __shared__ float stats[NW * 2 * 2 * 16];
   __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 256 : 4];
-  int rank, kvh, hg;
-  if (!block_to_tile_head(p, rank, kvh, hg)) return;
+  int rank, kvh, slice;
+  if (!block_to_tile_slice(p, p.H / p.H_kv * FS, rank, kvh, slice)) return;
   // The grid holds num_tiles units per head: all of them, or one per request, and the others follow in a second turn.
   ShortUnit u;
   for (; locate_short_unit<MODE>(p, 32, rank, u); rank += p.num_tiles) {
-    short_attn_unit<DTYPE, D, MODE>(p, lds, lds_q, stats, lds_rope, kvh, kvh * (p.H / p.H_kv) + hg, u);
+    short_attn_unit<DTYPE, D, MODE, FS>(p, lds, lds_q, stats, lds_rope, kvh, kvh * (p.H / p.H_kv) + slice / FS, slice % FS, u);
     __syncthreads();
   }
 }
 
-template <int DTYPE, int D, int MODE>
+template <int DTYPE, int D, int MODE, int FS>
 static int launch_short(AttnParams p, hipStream_t stream) {
   p.small_cache = small_cache(p);
-  const int64_t blocks = attn_grid_blocks(p);
+  const int64_t blocks = attn_grid_blocks(p, p.H / p.H_kv * FS);
   if (blocks > 0x7fffffffLL) return fail(ACACHE_E_SHAPE, "varlen_attn: grid too large");
-  hipLaunchKernelGGL((short_attn_kernel<DTYPE, D, MODE>), dim3((unsigned)blocks), dim3(64 * NW), 0, stream, p);
+  hipLaunchKernelGGL((short_attn_kernel<DTYPE, D, MODE, FS>), dim3((unsigned)blocks), dim3(64 * NW), 0, stream, p);
   return launch_status("short_attn_kernel");
 }
 
-int short_attention(const AttnParams &p, int mode, int dtype, hipStream_t stream) {
+// Where units are few, a unit's features are dealt to two or four workgroups: each scores all keys (and reads them, from the
+// same L2), but copies, multiplies and merges its share of the values only.  Every output has the same sum either way, bit for
+// bit.  `units`: those that are live in a batch of one-length blocks, which is what refinement steps are.  Time against whole
+// units (bf16, D = 128, 1 to 16 requests of 32 / 32, 28 / 4 and 8 / 2 heads, 300 to 2 000 keys, blocks of 8 and 32 rows):
+//   up to  64 units, four parts   plain 0.79 to 0.92, key side 0.81 to 0.93, query side 0.82 to 0.92 (two: 0.85 to 0.93)
+//   up to 128 units, two parts    plain 0.88 to 0.92
+// One request of 32 heads and 1 300 keys 16.1 -> 13.0 us.  (Parts of the keys instead would have to meet in memory: a second
+// launch or a counter that every call finds at zero.)
+template <int DTYPE, int D, int MODE>
+static int launch_parts(const AttnParams &p, int64_t units, hipStream_t stream) {
+  if (D == 128 && units * 4 <= 256) return launch_short<DTYPE, D, MODE, D == 128 ? 4 : 1>(p, stream);
+  if (D == 128 && units * 2 <= 256) return launch_short<DTYPE, D, MODE, D == 128 ? 2 : 1>(p, stream);
+  return launch_short<DTYPE, D, MODE, 1>(p, stream);
+}
+
+int short_attention(const AttnParams &p, int64_t units, int mode, int dtype, hipStream_t stream) {
 #define ACACHE_SHORT_MODE(DT, DD, MM) \
-  if (dtype == DT && p.head_dim == DD && mode == MM) return launch_short<DT, DD, MM>(p, stream);
+  if (dtype == DT && p.head_dim == DD && mode == MM) return launch_parts<DT, DD, MM>(p, units, stream);
 #define ACACHE_SHORT_ALL(DT, DD)            \
   ACACHE_SHORT_MODE(DT, DD, MODE_PLAIN)     \
   ACACHE_SHORT_MODE(DT, DD, MODE_KEY_SIDE)  \

@@ -109,3 +109,25 @@ def test_scores_far_below_zero(device, B, shared):
 def test_one_head_per_unit_from_a_few_hundred_keys(device, mode, H, Hkv, D, dtype, keys):
     """Batches of up to 256 units of one head take the wave-private form from 256, 400 or 512 keys on average."""
     _check(*_case([32, 1, 17, 0, 33], [31, 97, -1, 64, 255], H, Hkv, D, dtype, mode, keys, keys_per_request=keys), device)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mode", ["plain", "key", "query"])
+@pytest.mark.parametrize("H,Hkv,batches", [(32, 32, (2, 4, 6)), (28, 4, (2, 4, 7)), (12, 3, (5, 10, 15))])
+def test_few_units_in_parts_have_the_same_bits(device, mode, H, Hkv, batches, dtype):
+    """One request alone (up to 64 units: its features over four workgroups) and repeated in batches of up to 64, 128 and more
+    units (four, two, one workgroup each): the same bits, in the bound against the oracle."""
+    assert [1 + (B * H > 64) + (B * H > 128) for B in batches] == [1, 2, 3]
+    q_len, keys = 32 if Hkv == 32 else 13, 515
+    t, kw = _case([q_len], [keys], H, Hkv, 128, dtype, mode, H)
+    alone = _check(t, kw, device)
+    for B in batches:
+        rep = lambda cu: torch.arange(B + 1, dtype=torch.int32) * cu[1]
+        tb = [t[0].repeat(B, 1, 1), t[1], t[2], rep(t[3]), rep(t[4]), t[5].repeat(B)]
+        kwb = {k: v.repeat(B) if k in ("affix_shifts", "shared_kv_lens") else v for k, v in kw.items()}
+        q, kc, vc, cu_q, cu_k, slots = (x.to(device) for x in tb)
+        shape = (kc.shape[0] // 16, 16, *kc.shape[1:])
+        kwb = {k: v.to(device) if torch.is_tensor(v) else v for k, v in kwb.items()}
+        got = ops.acache_attention(q, kc.view(shape), vc.view(shape), cu_q, cu_k, slots, **kwb).cpu()
+        for b in range(B):
+            assert torch.equal(got[b * q_len:(b + 1) * q_len], alone), (B, b)
