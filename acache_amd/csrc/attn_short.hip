@@ -409,7 +409,7 @@ static int launch_short(AttnParams p, hipStream_t stream) {
 // bit.  `units`: those that are live in a batch of one-length blocks, which is what refinement steps are.  Time against whole
 // units (bf16, D = 128, 1 to 16 requests of 32 / 32, 28 / 4 and 8 / 2 heads, 300 to 2 000 keys, blocks of 8 and 32 rows):
 //   up to  64 units, four parts   plain 0.79 to 0.92, key side 0.81 to 0.93, query side 0.82 to 0.92 (two: 0.85 to 0.93)
-//   up to 128 units, two parts    plain 0.88 to 0.92
+//   up to 128 units, two parts    plain 0.86 to 0.99, key side 0.86 to 0.94, query side 0.88 to 1.01
 // One request of 32 heads and 1 300 keys 16.1 -> 13.0 us.  (Parts of the keys instead would have to meet in memory: a second
 // launch or a counter that every call finds at zero.)
 template <int DTYPE, int D, int MODE>

