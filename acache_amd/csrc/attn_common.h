@@ -38,6 +38,11 @@ struct AttnParams {
   int32_t H_kv;
   int32_t num_tiles;  // upper bound on the number of BM-row query tiles
   int32_t head_dim;   // real head_dim (read by the padded any-head_dim variant only)
+  int32_t small_cache;  // 32-bit copy offsets reach the whole cache (read by the short-query kernel)
+  int64_t num_slots;
+  int64_t q_token_bytes, q_head_bytes;
+  int64_t o_token_bytes, o_head_bytes;
+  int64_t kv_slot_bytes, kv_head_bytes;
   // MODE_PAGED: up to 64 requests of q_block query rows and seqlens[b] keys, no more than total_k in all; key n of request b
   // lies in block tables[b * max_blocks + (n >> block_shift)], absent where that is negative or past max_blocks
   const int32_t *seqlens;
@@ -46,11 +51,6 @@ struct AttnParams {
   int32_t max_blocks;
   int32_t block_shift;
   int32_t q_block;
-  int32_t small_cache;  // 32-bit copy offsets reach the whole cache (read by the short-query kernel)
-  int64_t num_slots;
-  int64_t q_token_bytes, q_head_bytes;
-  int64_t o_token_bytes, o_head_bytes;
-  int64_t kv_slot_bytes, kv_head_bytes;
 };
 
 // Which (request, query tile) does global tile index `tile` address?  Lane i loads
@@ -109,12 +109,14 @@ __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const
   const int key = ((kv < 0x1ffffff ? (kv > 0 ? kv : 0) : 0x1ffffff) << 6) | (63 - lane);
   int before = 0;  // query tiles of the requests sorted in front of this lane's request
   int all = 0;     // and of all requests
-  // Selects on one key, four requests a turn (lanes past B have no tiles).  As a branch on two compares per request the
+  // Selects on one key, two requests a turn (lanes past B have no tiles; four a turn cost planned launches, which jump over
+  // this code, 1.1 us: it is fetched with theirs).  As a branch on two compares per request the
   // ranking took most of a short unit: whole calls of 28 / 4 heads, 32 queries and 300 keys a request, before / now: 64
   // requests 52.0 / 35.5 us, 32: 22.9 / 18.0; of 1 100 keys 64: 78.4 / 61.8, 32: 38.8 / 31.5, 16: 25.0 / 23.6.
-  for (int j0 = 0; j0 < B; j0 += 4) {
+#pragma nounroll
+  for (int j0 = 0; j0 < B; j0 += 2) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < 2; ++j) {
       const int key_j = __builtin_amdgcn_readlane(key, j0 + j);
       const int tiles_j = __builtin_amdgcn_readlane(tiles, j0 + j);
       before += key_j > key ? tiles_j : 0;
