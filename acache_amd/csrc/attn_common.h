@@ -110,9 +110,9 @@ __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const
   int before = 0;  // query tiles of the requests sorted in front of this lane's request
   int all = 0;     // and of all requests
   // Selects on one key, two requests a turn (lanes past B have no tiles; four a turn cost planned launches, which jump over
-  // this code, 1.1 us: it is fetched with theirs).  As a branch on two compares per request the
-  // ranking took most of a short unit: whole calls of 28 / 4 heads, 32 queries and 300 keys a request, before / now: 64
-  // requests 52.0 / 35.5 us, 32: 22.9 / 18.0; of 1 100 keys 64: 78.4 / 61.8, 32: 38.8 / 31.5, 16: 25.0 / 23.6.
+  // this code, 1.1 us: it is fetched with theirs).  As a branch on two compares per request the ranking took most of a short
+  // unit: whole calls of 32 query rows, before / now: 64 requests of 32 heads and 200 keys 69.6 / 55.2 us, of 8 heads and 300
+  // keys 27.1 / 21.6, 32 of those 14.3 / 13.0; 16 requests of 32 heads, 300 keys 21.0 / 19.6, 1 100 keys 54.5 / 53.4.
 #pragma nounroll
   for (int j0 = 0; j0 < B; j0 += 2) {
 #pragma unroll
