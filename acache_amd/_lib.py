@@ -80,6 +80,7 @@ SIGNATURES = {
         c_int32, c_int32, c_int32, c_int32, c_int64,
         c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
         c_void_p, c_int64, c_void_p]),
+    "acache_varlen_attn_form": (c_int32, [c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32]),
     "acache_varlen_attn_plan": (c_int64, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p, c_int64]),
 }
 

@@ -991,10 +991,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_pair_kernel(AttnParams p) 
 }
 
 template <int DTYPE, int D>
-static int launch_pairs(const AttnParams &p0, int mode, int64_t total_q, hipStream_t stream) {
-  AttnParams p = p0;
-  p.num_tiles = (int32_t)((total_q + 31) / 32) + p.B;
-  const int64_t blocks = attn_grid_blocks(p, (p.H / p.H_kv + 1) / 2);
+static int launch_pairs(const AttnParams &p, int mode, int64_t blocks, hipStream_t stream) {
   if (blocks > 0x7fffffffLL) return fail(ACACHE_E_SHAPE, "varlen_attn: grid too large");
   const bool small = small_cache(p);
   const dim3 grid((unsigned)blocks), block(256);
@@ -1010,11 +1007,8 @@ static int launch_pairs(const AttnParams &p0, int mode, int64_t total_q, hipStre
 }
 
 template <int DTYPE, int D, int NQ16>
-static int launch_attn(const AttnParams &p0, int mode, int64_t total_q, int64_t plan_blocks, hipStream_t stream) {
-  AttnParams p = p0;
+static int launch_attn(const AttnParams &p, int mode, int64_t blocks, hipStream_t stream) {
   // One 4-wave workgroup per (request, 128-row query tile, head), two workgroups per CU.
-  p.num_tiles = (int32_t)((total_q + 127) / 128) + p.B;
-  const int64_t blocks = p.plan ? plan_blocks : attn_grid_blocks(p);
   if (blocks > 0x7fffffffLL) return fail(ACACHE_E_SHAPE, "varlen_attn: grid too large");
   const bool small = small_cache(p);
   const dim3 grid((unsigned)blocks), block(256);
@@ -1037,12 +1031,8 @@ static int launch_attn(const AttnParams &p0, int mode, int64_t total_q, int64_t 
 // 16 query rows per wave, all three relocation modes.  A correctness path for model shapes outside the two
 // tuned widths, not a tuned one.
 template <int DTYPE>
-static int launch_attn_any_head_dim(const AttnParams &p0, int mode, int64_t total_q, hipStream_t stream) {
-  AttnParams p = p0;
-  constexpr int BM = 64, DPAD = 256;
-  p.num_tiles = (int32_t)((total_q + BM - 1) / BM) + p.B;
-  int64_t blocks = (int64_t)p.num_tiles * p.H;
-  blocks = (blocks + 7) / 8 * 8;
+static int launch_attn_any_head_dim(const AttnParams &p, int mode, int64_t blocks, hipStream_t stream) {
+  constexpr int DPAD = 256;
   if (blocks > 0x7fffffffLL) return fail(ACACHE_E_SHAPE, "varlen_attn: grid too large");
   dim3 grid((unsigned)blocks), block(256);
   switch (mode) {
@@ -1086,6 +1076,20 @@ static bool takes_short_kernel(AttnParams &p, int mode, int64_t total_q, int64_t
   if (attn_grid_blocks(p) <= 256) return true;
   p.num_tiles = p.B;
   return total_q % B == 0 && attn_grid_blocks(p) <= 256;
+}
+
+// Where units are few, a unit's features are dealt to two or four workgroups: each scores all keys (and reads them, from the
+// same L2), but copies, multiplies and merges its share of the values only.  Every output has the same sum either way, bit for
+// bit.  Units are
+// counted as in a batch of one-length blocks, which is what refinement steps are, where the total allows it.  Time against whole
+// units (bf16, D = 128, 1 to 16 requests of 32 / 32, 28 / 4 and 8 / 2 heads, 300 to 2 000 keys, blocks of 8 and 32 rows):
+//   up to  64 units, four parts   plain 0.79 to 0.92, key side 0.81 to 0.93, query side 0.82 to 0.92 (two: 0.85 to 0.93)
+//   up to 128 units, two parts    plain 0.86 to 0.99, key side 0.86 to 0.94, query side 0.88 to 1.01
+// One request of 32 heads and 1 300 keys 16.1 -> 13.0 us.  (Parts of the keys instead would have to meet in memory: a second
+// launch or a counter that every call finds at zero.)
+static int parts_per_unit(const AttnParams &p, int64_t total_q) {
+  const int64_t units = (total_q % p.B == 0 ? p.B : p.num_tiles) * (int64_t)p.H;
+  return p.head_dim != 128 ? 1 : units * 4 <= 256 ? 4 : units * 2 <= 256 ? 2 : 1;
 }
 
 // Several heads of a group per unit of eight waves (attn_group.hip), one unit per CU; sets p.num_tiles.  Returns the heads, 0
@@ -1137,6 +1141,35 @@ static bool takes_pair_kernel(AttnParams &p, int64_t total_q) {
   if (p.head_dim != 128 || total_q > 32 * (int64_t)p.B || total_q % p.B != 0 || p.H == p.H_kv) return false;
   p.num_tiles = p.B;
   return attn_grid_blocks(p) > 512;
+}
+
+// The kernel that a call takes, what a unit of it is, and its grid.  (Lengths on the device: a rule over sizes only.)
+enum { FORM_UNITS = 0, FORM_SHORT = 1, FORM_GROUP = 2, FORM_PAIRS = 3, FORM_ANY_HEAD_DIM = 4 };
+struct AttnForm {
+  int kind;
+  int share;      // FORM_SHORT: workgroups per unit; FORM_GROUP, FORM_PAIRS: heads per unit
+  int32_t tiles;  // query tiles that the grid holds units for
+  int64_t blocks;
+};
+static AttnForm attention_form(const AttnParams &p0, int mode, int64_t total_q, int64_t total_k) {
+  AttnParams p = p0;
+  const int group = p.H / p.H_kv;
+  if (takes_short_kernel(p, mode, total_q, total_k)) {
+    const int parts = parts_per_unit(p, total_q);
+    return {FORM_SHORT, parts, p.num_tiles, attn_grid_blocks(p, group * parts)};
+  }
+  if (const int heads = heads_per_group_unit(p, mode, total_q, total_k))
+    return {FORM_GROUP, heads, p.num_tiles, attn_grid_blocks(p, (group + heads - 1) / heads)};
+  if (takes_pair_kernel(p, total_q)) {
+    p.num_tiles = (int32_t)((total_q + 31) / 32) + p.B;
+    return {FORM_PAIRS, 2, p.num_tiles, attn_grid_blocks(p, (group + 1) / 2)};
+  }
+  if (p.head_dim == 128 || p.head_dim == 64) {
+    p.num_tiles = (int32_t)((total_q + 127) / 128) + p.B;
+    return {FORM_UNITS, 1, p.num_tiles, attn_grid_blocks(p)};
+  }
+  p.num_tiles = (int32_t)((total_q + 63) / 64) + p.B;
+  return {FORM_ANY_HEAD_DIM, 1, p.num_tiles, ((int64_t)p.num_tiles * p.H + 7) / 8 * 8};
 }
 
 // Keys given by lengths and block tables (acache_decode_attn): the short-block kernels read those themselves, for the others
@@ -1196,13 +1229,13 @@ static int attention_call(
   const int mode = query_side ? MODE_QUERY_SIDE : (relocate ? MODE_KEY_SIDE : MODE_PLAIN);
   hipStream_t st = (hipStream_t)stream;
   p.small_cache = 0;
-  const bool takes_short = takes_short_kernel(p, mode, total_q, total_k);
-  const int heads = takes_short ? 0 : heads_per_group_unit(p, mode, total_q, total_k);
+  const AttnForm form = attention_form(p, mode, total_q, total_k);
+  p.num_tiles = form.tiles;
   int short_mode = mode;
   if (paged) {
     // a chunk of 32 keys has to lie in one block; one request per lane
     const int bs = paged->block_size;
-    if ((takes_short || heads) && B <= 64 && bs >= 32 && (bs & (bs - 1)) == 0) {
+    if ((form.kind == FORM_SHORT || form.kind == FORM_GROUP) && B <= 64 && bs >= 32 && (bs & (bs - 1)) == 0) {
       short_mode = MODE_PAGED;
       p.seqlens = paged->seqlens; p.tables = paged->tables; p.total_k = total_k;
       p.max_blocks = paged->max_blocks; p.q_block = paged->q_len; p.block_shift = __builtin_ctz(bs);
@@ -1212,20 +1245,20 @@ static int attention_call(
       return rc;
     }
   }
-  if (takes_short) return short_attention(p, (total_q % B == 0 ? B : (int64_t)p.num_tiles) * H, short_mode, dtype, st);
-  if (heads) return group_attention(p, heads, short_mode, dtype, st);
-  if (takes_pair_kernel(p, total_q))
-    return dtype == ACACHE_BF16 ? launch_pairs<ACACHE_BF16, 128>(p, mode, total_q, st)
-                                : launch_pairs<ACACHE_F16, 128>(p, mode, total_q, st);
-#define ACACHE_ATTN(DT, DD) \
-  if (dtype == DT && D == DD) return launch_attn<DT, DD, 2>(p, mode, total_q, plan_blocks, st);
-  ACACHE_ATTN(ACACHE_BF16, 128)
-  ACACHE_ATTN(ACACHE_BF16, 64)
-  ACACHE_ATTN(ACACHE_F16, 128)
-  ACACHE_ATTN(ACACHE_F16, 64)
-#undef ACACHE_ATTN
-  if (dtype == ACACHE_BF16) return launch_attn_any_head_dim<ACACHE_BF16>(p, mode, total_q, st);
-  return launch_attn_any_head_dim<ACACHE_F16>(p, mode, total_q, st);
+  const bool bf = dtype == ACACHE_BF16;
+  switch (form.kind) {
+    case FORM_SHORT: return short_attention(p, form.share, short_mode, dtype, st);
+    case FORM_GROUP: return group_attention(p, form.share, short_mode, dtype, st);
+    case FORM_PAIRS:
+      return bf ? launch_pairs<ACACHE_BF16, 128>(p, mode, form.blocks, st) : launch_pairs<ACACHE_F16, 128>(p, mode, form.blocks, st);
+    case FORM_UNITS: {
+      const int64_t blocks = p.plan ? plan_blocks : form.blocks;
+      if (D == 128) return bf ? launch_attn<ACACHE_BF16, 128, 2>(p, mode, blocks, st) : launch_attn<ACACHE_F16, 128, 2>(p, mode, blocks, st);
+      return bf ? launch_attn<ACACHE_BF16, 64, 2>(p, mode, blocks, st) : launch_attn<ACACHE_F16, 64, 2>(p, mode, blocks, st);
+    }
+  }
+  return bf ? launch_attn_any_head_dim<ACACHE_BF16>(p, mode, form.blocks, st)
+            : launch_attn_any_head_dim<ACACHE_F16>(p, mode, form.blocks, st);
 }
 
 }  // namespace acache
@@ -1275,4 +1308,17 @@ extern "C" int acache_varlen_attn(
                                     shared_kv_lens, affix_shifts, rope_cos, rope_sin, rope_rows, B, total_q, total_k,
                                     H, H_kv, D, dtype, num_slots, q_token_stride, q_head_stride, out_token_stride,
                                     out_head_stride, kv_slot_stride, kv_head_stride, nullptr, 0, stream);
+}
+
+extern "C" int acache_varlen_attn_form(int64_t form[4], int32_t B, int64_t total_q, int64_t total_k, int32_t H, int32_t H_kv,
+                                       int32_t D, int32_t mode) {
+  if (!form) return fail(ACACHE_E_NULL, "varlen_attn_form: NULL pointer");
+  if (B <= 0 || total_q <= 0 || total_k < 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || D < 16 || D > 256 || D % 16 != 0 ||
+      mode < MODE_PLAIN || mode > MODE_QUERY_SIDE)
+    return fail(ACACHE_E_SHAPE, "varlen_attn_form: bad size");
+  AttnParams p{};
+  p.B = B; p.H = H; p.H_kv = H_kv; p.head_dim = D;
+  const AttnForm f = attention_form(p, mode, total_q, total_k);
+  form[0] = f.kind; form[1] = f.share; form[2] = f.tiles; form[3] = f.blocks;
+  return 0;
 }

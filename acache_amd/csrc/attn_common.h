@@ -292,8 +292,8 @@ inline bool small_cache(const AttnParams &p) {
          p.num_slots * p.kv_slot_bytes + 4096 <= 0xffffffffLL;
 }
 
-// attn_short.hip: batches of short query blocks, head dims 64 and 128; `units` of them are live if the blocks have one length.
-int short_attention(const AttnParams &p, int64_t units, int mode, int dtype, hipStream_t stream);
+// attn_short.hip: batches of short query blocks, head dims 64 and 128; `parts` workgroups per unit (1, 2 or 4).
+int short_attention(const AttnParams &p, int parts, int mode, int dtype, hipStream_t stream);
 
 // attn_group.hip: grouped-query batches of short query blocks, head dim 128.
 int group_attention(const AttnParams &p, int heads_per_unit, int mode, int dtype, hipStream_t stream);

@@ -404,24 +404,16 @@ static int launch_short(AttnParams p, hipStream_t stream) {
   return launch_status("short_attn_kernel");
 }
 
-// Where units are few, a unit's features are dealt to two or four workgroups: each scores all keys (and reads them, from the
-// same L2), but copies, multiplies and merges its share of the values only.  Every output has the same sum either way, bit for
-// bit.  `units`: those that are live in a batch of one-length blocks, which is what refinement steps are.  Time against whole
-// units (bf16, D = 128, 1 to 16 requests of 32 / 32, 28 / 4 and 8 / 2 heads, 300 to 2 000 keys, blocks of 8 and 32 rows):
-//   up to  64 units, four parts   plain 0.79 to 0.92, key side 0.81 to 0.93, query side 0.82 to 0.92 (two: 0.85 to 0.93)
-//   up to 128 units, two parts    plain 0.86 to 0.99, key side 0.86 to 0.94, query side 0.88 to 1.01
-// One request of 32 heads and 1 300 keys 16.1 -> 13.0 us.  (Parts of the keys instead would have to meet in memory: a second
-// launch or a counter that every call finds at zero.)
 template <int DTYPE, int D, int MODE>
-static int launch_parts(const AttnParams &p, int64_t units, hipStream_t stream) {
-  if (D == 128 && units * 4 <= 256) return launch_short<DTYPE, D, MODE, D == 128 ? 4 : 1>(p, stream);
-  if (D == 128 && units * 2 <= 256) return launch_short<DTYPE, D, MODE, D == 128 ? 2 : 1>(p, stream);
+static int launch_parts(const AttnParams &p, int parts, hipStream_t stream) {
+  if (D == 128 && parts == 4) return launch_short<DTYPE, D, MODE, D == 128 ? 4 : 1>(p, stream);
+  if (D == 128 && parts == 2) return launch_short<DTYPE, D, MODE, D == 128 ? 2 : 1>(p, stream);
   return launch_short<DTYPE, D, MODE, 1>(p, stream);
 }
 
-int short_attention(const AttnParams &p, int64_t units, int mode, int dtype, hipStream_t stream) {
+int short_attention(const AttnParams &p, int parts, int mode, int dtype, hipStream_t stream) {
 #define ACACHE_SHORT_MODE(DT, DD, MM) \
-  if (dtype == DT && p.head_dim == DD && mode == MM) return launch_parts<DT, DD, MM>(p, units, stream);
+  if (dtype == DT && p.head_dim == DD && mode == MM) return launch_parts<DT, DD, MM>(p, parts, stream);
 #define ACACHE_SHORT_ALL(DT, DD)            \
   ACACHE_SHORT_MODE(DT, DD, MODE_PLAIN)     \
   ACACHE_SHORT_MODE(DT, DD, MODE_KEY_SIDE)  \

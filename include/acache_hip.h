@@ -350,6 +350,18 @@ int acache_decode_attn(
     int64_t kv_slot_stride, int64_t kv_head_stride, void *stream);
 
 /*
+ * Which kernel acache_varlen_attn takes for these sizes (mode 0: plain, 1: key-side, 2: query-side relocation) and the grid
+ * that it is launched with, on the host alone:
+ *   form[0]  0 units of a head and 128 rows, 1 wave-private key chunks, 2 heads of a group in eight waves, 3 pairs of heads in
+ *            four, 4 any other head dim
+ *   form[1]  1: workgroups per unit, 2 and 3: heads per unit, otherwise 1
+ *   form[2]  query tiles that the grid has units for; those of 1 and 2 take the further ones in another turn
+ *   form[3]  workgroups of an unplanned launch
+ */
+int acache_varlen_attn_form(int64_t form[4], int32_t B, int64_t total_q, int64_t total_k, int32_t H, int32_t H_kv, int32_t D,
+                            int32_t mode);
+
+/*
  * Slot layout of a batch of requests that reuse a shared affix (device-side form of
  * Sequence.finalize_slot_mapping, nano-vdllm/sequence.py:169-202, which the reference
  * evaluates per request in Python before prepare_caching_acache,
