@@ -973,7 +973,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_pair_kernel(AttnParams p) 
   __shared__ __attribute__((aligned(1024))) char lds[4 * TILE_BYTES + (MODE == MODE_KEY_SIDE ? 2 * D * 4 : 0)];
   const int group = p.H / p.H_kv;
   int rank, kvh, slice, b = 0, q_begin = 0, q_len = 0, tile = 0, kv_begin = 0, kv_len = 0;
-  if (!block_to_tile_slice(p, (group + 1) / 2, rank, kvh, slice)) return;
+  if (!block_to_tile_slice(p, p.num_tiles, (group + 1) / 2, rank, kvh, slice)) return;
   if (p.B <= 64) {
     if (!locate_query_tile_lpt(p.cu_q, p.cu_k, p.B, 32, rank, b, q_begin, q_len, tile, kv_begin, kv_len)) return;
   } else {
@@ -1052,7 +1052,14 @@ static int launch_attn_any_head_dim(const AttnParams &p, int mode, int64_t block
 // Which batches of short query blocks (32 rows per request on average at most) leave the per-head units of launch_attn.
 // Their plan, if any, is not needed.  The lengths are on the device: the host knows totals only.
 
-// Wave-private key chunks (attn_short.hip), a unit of 32 query rows per CU; sets p.num_tiles to the tiles of its grid.
+// Query tiles of a grid of `blocks` workgroups (a multiple of 8) with `slices` units per tile and KV head.  Room for more
+// tiles than a batch of one-length blocks has costs nothing where CUs would stay idle; `most` are enough for any lengths.
+static int32_t tiles_in_grid(const AttnParams &p, int slices, int64_t blocks, int64_t most) {
+  const int64_t tiles = p.H_kv < 8 && 8 % p.H_kv == 0 ? blocks / (8 * slices) * (8 / p.H_kv) : blocks / ((int64_t)slices * p.H_kv);
+  return (int32_t)(tiles < most ? tiles : most);
+}
+
+// Wave-private key chunks (attn_short.hip), a unit of 32 query rows per CU; sets p.num_tiles to the most tiles of such a batch.
 // Measured as time against the per-head units (bf16, 1 to 32 requests of 32 / 32, 28 / 4, 16 / 16 and 8 / 2 heads, ragged
 // keys, blocks of 8 and 32 rows, every key private or most of them shared):
 //   keys per request       100           200           300           400           600           1000          2000
@@ -1072,24 +1079,28 @@ static bool takes_short_kernel(AttnParams &p, int mode, int64_t total_q, int64_t
   const int64_t B = p.B;
   if ((p.head_dim != 128 && p.head_dim != 64) || total_q > 32 * B) return false;
   if (total_k < B * (mode == MODE_QUERY_SIDE ? 256 : p.head_dim == 64 ? 512 : 400)) return false;
-  p.num_tiles = (int32_t)((total_q + 31 * B) / 32);
-  if (attn_grid_blocks(p) <= 256) return true;
-  p.num_tiles = p.B;
-  return total_q % B == 0 && attn_grid_blocks(p) <= 256;
+  const int32_t most = (int32_t)((total_q + 31 * B) / 32);
+  p.num_tiles = total_q % B == 0 ? p.B : most;
+  if (attn_grid_blocks(p) > 256) return false;
+  p.num_tiles = most;
+  return true;
 }
 
 // Where units are few, a unit's features are dealt to two or four workgroups: each scores all keys (and reads them, from the
 // same L2), but copies, multiplies and merges its share of the values only.  Every output has the same sum either way, bit for
-// bit.  Units are
-// counted as in a batch of one-length blocks, which is what refinement steps are, where the total allows it.  Time against whole
-// units (bf16, D = 128, 1 to 16 requests of 32 / 32, 28 / 4 and 8 / 2 heads, 300 to 2 000 keys, blocks of 8 and 32 rows):
+// bit.  All parts run at once: their grid has a workgroup per CU at most, counting units as in a batch of one-length blocks,
+// which is what refinement steps are, where the total allows it.  Time against whole units (bf16, D = 128, 1 to 16 requests of
+// 32 / 32, 28 / 4 and 8 / 2 heads, 300 to 2 000 keys, blocks of 8 and 32 rows):
 //   up to  64 units, four parts   plain 0.79 to 0.92, key side 0.81 to 0.93, query side 0.82 to 0.92 (two: 0.85 to 0.93)
 //   up to 128 units, two parts    plain 0.86 to 0.99, key side 0.86 to 0.94, query side 0.88 to 1.01
 // One request of 32 heads and 1 300 keys 16.1 -> 13.0 us.  (Parts of the keys instead would have to meet in memory: a second
 // launch or a counter that every call finds at zero.)
 static int parts_per_unit(const AttnParams &p, int64_t total_q) {
-  const int64_t units = (total_q % p.B == 0 ? p.B : p.num_tiles) * (int64_t)p.H;
-  return p.head_dim != 128 ? 1 : units * 4 <= 256 ? 4 : units * 2 <= 256 ? 2 : 1;
+  AttnParams t = p;
+  if (total_q % p.B == 0) t.num_tiles = p.B;
+  for (int parts = 4; parts > 1; parts /= 2)
+    if (p.head_dim == 128 && attn_grid_blocks(t, p.H / p.H_kv * parts) <= 256) return parts;
+  return 1;
 }
 
 // Several heads of a group per unit of eight waves (attn_group.hip), one unit per CU; sets p.num_tiles.  Returns the heads, 0
@@ -1156,6 +1167,7 @@ static AttnForm attention_form(const AttnParams &p0, int mode, int64_t total_q, 
   const int group = p.H / p.H_kv;
   if (takes_short_kernel(p, mode, total_q, total_k)) {
     const int parts = parts_per_unit(p, total_q);
+    p.num_tiles = tiles_in_grid(p, group * parts, 256, p.num_tiles);
     return {FORM_SHORT, parts, p.num_tiles, attn_grid_blocks(p, group * parts)};
   }
   if (const int heads = heads_per_group_unit(p, mode, total_q, total_k))

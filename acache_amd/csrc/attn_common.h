@@ -152,20 +152,57 @@ struct ShortUnit {
   int shared_len, shift;  // clamped; 0 in the modes that have none
 };
 
-// Query tile `rank` (BM rows) in batch order.  For up to 64 requests everything is loaded in one round trip, one request
-// per lane, and a batch of one tile per request, which is what blocks of one length are, needs no prefix sum: 0.3 us
-// from the loads to the unit, where ranking one request by its keys takes 0.9 and sixteen 1.6.
+// The lengths of up to 64 requests, one per lane, in one round trip, and how many query tiles (BM rows) they make, which is
+// what the grid of such a kernel is dealt by.  A batch of one tile per request, which is what blocks of one length are, needs
+// no prefix sum: 0.3 us from the loads to the unit, where ranking one request by its keys takes 0.9 and sixteen 1.6.  More
+// requests are looked up unit by unit.
+struct ShortBatch {
+  int q0, q1, k0, k1, shared, shift;
+  int incl;      // tiles up to and with this lane's request; not set where every request has one
+  bool single;   // every request has one tile
+  int live;      // tiles of the batch; past any number of them for more than 64 requests
+};
 template <int MODE>
-__device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, int rank, ShortUnit &u) {
+__device__ __forceinline__ ShortBatch load_short_batch(const AttnParams &p, int BM) {
   const int lane = opaque_tid() & 63;
-  int shared = 0, shift = 0;
+  ShortBatch t;
+  t.shared = t.shift = t.incl = 0;
+  t.single = true;
+  t.live = 0x7fffffff;
   if (MODE == MODE_PAGED) {
-    const int tiles = (p.q_block + BM - 1) / BM;
+    t.k1 = lane < p.B ? p.seqlens[lane] : 0;
+    t.live = p.B * ((p.q_block + BM - 1) / BM);
+  } else if (p.B <= 64) {
+    const int l = lane < p.B ? lane : p.B - 1;
+    t.q0 = p.cu_q[l]; t.q1 = p.cu_q[l + 1]; t.k0 = p.cu_k[l]; t.k1 = p.cu_k[l + 1];
+    if (MODE == MODE_QUERY_SIDE) t.shared = p.shared_kv_lens[l];
+    if (relocates(MODE)) t.shift = p.affix_shifts[l];
+    const int tiles = lane < p.B && t.q1 > t.q0 ? (t.q1 - t.q0 + BM - 1) / BM : 0;
+    t.single = __builtin_amdgcn_ballot_w64(lane < p.B && tiles != 1) == 0;
+    t.live = p.B;
+    if (!t.single) {
+      t.incl = tiles;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(t.incl, d);
+        if (lane >= d) t.incl += up;
+      }
+      t.live = __builtin_amdgcn_readlane(t.incl, 63);
+    }
+  }
+  return t;
+}
+
+// Query tile `rank` (BM rows) in batch order.
+template <int MODE>
+__device__ __forceinline__ bool locate_short_unit(const AttnParams &p, const ShortBatch &t, int BM, int rank, ShortUnit &u) {
+  int shared, shift;
+  if (MODE == MODE_PAGED) {
+    const int lane = opaque_tid() & 63, tiles = (p.q_block + BM - 1) / BM;
     u.b = rank / tiles;
     u.tile = rank - u.b * tiles;
     if (u.b >= p.B) return false;
-    const int len = lane < p.B ? p.seqlens[lane] : 0;
-    int before = lane < u.b ? len : 0;        // keys of the requests in front: the caller's total bounds them all
+    int before = lane < u.b ? t.k1 : 0;       // keys of the requests in front: the caller's total bounds them all
     before += __builtin_amdgcn_update_dpp(0, before, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
     before += __builtin_amdgcn_update_dpp(0, before, 0x112, 0xf, 0xf, false);
     before += __builtin_amdgcn_update_dpp(0, before, 0x114, 0xf, 0xf, false);
@@ -173,7 +210,7 @@ __device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, i
     int start = 0;
 #pragma unroll
     for (int row = 0; row < 4; ++row) start += __builtin_amdgcn_readlane(before, 16 * row + 15);
-    const int64_t end = (int64_t)start + __builtin_amdgcn_readlane(len, u.b);
+    const int64_t end = (int64_t)start + __builtin_amdgcn_readlane(t.k1, u.b);
     const int64_t from = start < 0 ? 0 : (start > p.total_k ? p.total_k : start);
     u.q_begin = u.b * p.q_block;
     u.q_len = p.q_block;
@@ -183,34 +220,19 @@ __device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, i
     return true;
   }
   if (p.B <= 64) {
-    const int l = lane < p.B ? lane : p.B - 1;
-    const int q0 = p.cu_q[l], q1 = p.cu_q[l + 1], k0 = p.cu_k[l], k1 = p.cu_k[l + 1];
-    if (MODE == MODE_QUERY_SIDE) shared = p.shared_kv_lens[l];
-    if (relocates(MODE)) shift = p.affix_shifts[l];
-    const int tiles = lane < p.B && q1 > q0 ? (q1 - q0 + BM - 1) / BM : 0;
-    int src = rank;
+    if (rank >= t.live) return false;
+    u.b = rank;
     u.tile = 0;
-    if (__builtin_amdgcn_ballot_w64(lane < p.B && tiles != 1) == 0) {
-      if (rank >= p.B) return false;
-    } else {
-      int incl = tiles;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(incl, d);
-        if (lane >= d) incl += up;
-      }
-      const uint64_t hit = __builtin_amdgcn_ballot_w64(incl > rank);
-      if (hit == 0) return false;
-      src = __builtin_ctzll(hit);
-      u.tile = rank - (__builtin_amdgcn_readlane(incl, src) - __builtin_amdgcn_readlane(tiles, src));
+    if (!t.single) {
+      u.b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(t.incl > rank));
+      u.tile = u.b == 0 ? rank : rank - __builtin_amdgcn_readlane(t.incl, u.b - 1);
     }
-    u.b = src;
-    u.q_begin = __builtin_amdgcn_readlane(q0, src);
-    u.q_len = __builtin_amdgcn_readlane(q1, src) - u.q_begin;
-    u.kv_begin = __builtin_amdgcn_readlane(k0, src);
-    u.kv_len = __builtin_amdgcn_readlane(k1, src) - u.kv_begin;
-    if (MODE == MODE_QUERY_SIDE) shared = __builtin_amdgcn_readlane(shared, src);
-    if (relocates(MODE)) shift = __builtin_amdgcn_readlane(shift, src);
+    u.q_begin = __builtin_amdgcn_readlane(t.q0, u.b);
+    u.q_len = __builtin_amdgcn_readlane(t.q1, u.b) - u.q_begin;
+    u.kv_begin = __builtin_amdgcn_readlane(t.k0, u.b);
+    u.kv_len = __builtin_amdgcn_readlane(t.k1, u.b) - u.kv_begin;
+    shared = MODE == MODE_QUERY_SIDE ? __builtin_amdgcn_readlane(t.shared, u.b) : 0;
+    shift = relocates(MODE) ? __builtin_amdgcn_readlane(t.shift, u.b) : 0;
   } else {
     if (!locate_query_tile(p.cu_q, p.B, BM, rank, u.b, u.q_begin, u.q_len, u.tile)) return false;
     u.b = __builtin_amdgcn_readfirstlane(u.b);
@@ -219,8 +241,8 @@ __device__ __forceinline__ bool locate_short_unit(const AttnParams &p, int BM, i
     u.tile = __builtin_amdgcn_readfirstlane(u.tile);
     u.kv_begin = p.cu_k[u.b];
     u.kv_len = p.cu_k[u.b + 1] - u.kv_begin;
-    if (MODE == MODE_QUERY_SIDE) shared = p.shared_kv_lens[u.b];
-    if (relocates(MODE)) shift = p.affix_shifts[u.b];
+    shared = MODE == MODE_QUERY_SIDE ? p.shared_kv_lens[u.b] : 0;
+    shift = relocates(MODE) ? p.affix_shifts[u.b] : 0;
   }
   u.shared_len = shared < 0 ? 0 : (shared > u.kv_len ? u.kv_len : shared);
   u.shift = shift < 0 || shift >= p.rope_rows ? 0 : shift;
@@ -247,13 +269,14 @@ __device__ __forceinline__ int slot_of_entry(const AttnParams &p, int entry, int
 // The grid must hold attn_grid_blocks(p) blocks.  Returns false for a block without work.
 // `group` is the number of units per KV head and query tile: the query heads of the KV head, or fewer for a kernel whose
 // units take several of them.
-__device__ __forceinline__ bool block_to_tile_slice(const AttnParams &p, int group, int &tile, int &kvh, int &hg) {
-  const int per_xcd = gridDim.x >> 3;
+// `num_tiles` of them are dealt, of the tiles that the grid holds: a kernel that knows how many there are gives every XCD its
+// share of those.
+__device__ __forceinline__ bool block_to_tile_slice(const AttnParams &p, int num_tiles, int group, int &tile, int &kvh, int &hg) {
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   if (p.H_kv % 8 == 0) {
     const int heads_per_xcd = (p.H_kv >> 3) * group;
     tile = idx / heads_per_xcd;
-    if (tile >= p.num_tiles) return false;
+    if (tile >= num_tiles) return false;
     const int r = idx - tile * heads_per_xcd;
     kvh = xcd * (p.H_kv >> 3) + r / group;
     hg = r % group;
@@ -261,20 +284,21 @@ __device__ __forceinline__ bool block_to_tile_slice(const AttnParams &p, int gro
     const int xcds_per_head = 8 / p.H_kv;
     kvh = xcd / xcds_per_head;
     tile = (idx / group) * xcds_per_head + xcd % xcds_per_head;
-    if (tile >= p.num_tiles) return false;
+    if (tile >= num_tiles) return false;
     hg = idx % group;
   } else {
+    const int units = num_tiles * group * p.H_kv, per_xcd = (units + 7) >> 3;
     const int w = xcd * per_xcd + idx;
-    if (w >= p.num_tiles * group * p.H_kv) return false;
+    if (idx >= per_xcd || w >= units) return false;
     hg = w % group;
-    tile = (w / group) % p.num_tiles;
-    kvh = w / (group * p.num_tiles);
+    tile = (w / group) % num_tiles;
+    kvh = w / (group * num_tiles);
   }
   return true;
 }
 
 __device__ __forceinline__ bool block_to_tile_head(const AttnParams &p, int &tile, int &kvh, int &hg) {
-  return block_to_tile_slice(p, p.H / p.H_kv, tile, kvh, hg);
+  return block_to_tile_slice(p, p.num_tiles, p.H / p.H_kv, tile, kvh, hg);
 }
 
 inline int64_t attn_grid_blocks(const AttnParams &p, int group) {

@@ -379,14 +379,20 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 1) void group_attn_kernel(AttnPar
   __shared__ float stats[GROUP_WAVES * 2 * 2 * 16];
   __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 2 * D : 4];
   const int group = p.H / p.H_kv;
+  // The grid holds num_tiles units per slice, of which the live ones are dealt; a batch of more takes further turns.
+  ShortBatch t = load_short_batch<MODE>(p, 32);
+  const int tiles = t.live < p.num_tiles ? t.live : p.num_tiles;
   int rank, kvh, slice;
-  if (!block_to_tile_slice(p, (group + HU - 1) / HU, rank, kvh, slice)) return;
+  if (!block_to_tile_slice(p, tiles, (group + HU - 1) / HU, rank, kvh, slice)) return;
   const int first = slice * HU, heads = group - first < HU ? group - first : HU;
-  // The grid holds num_tiles units per slice: all of them, or one per request, and the others follow in a second turn.
   ShortUnit u;
-  for (; locate_short_unit<MODE>(p, 32, rank, u); rank += p.num_tiles) {
+  const int live = t.live;
+  while (locate_short_unit<MODE>(p, t, 32, rank, u)) {
     group_attn_unit<DTYPE, D, MODE, HU>(p, lds, lds_q, stats, lds_rope, landed, kvh, kvh * group + first, heads, u);
+    rank += tiles;
+    if (rank >= live) return;
     __syncthreads();
+    t = load_short_batch<MODE>(p, 32);
   }
 }
 

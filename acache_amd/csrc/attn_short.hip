@@ -385,13 +385,19 @@ __global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(1024))) char lds_q[(MODE == MODE_QUERY_SIDE ? 2 : 1) * 32 * D * 2];
   __shared__ float stats[NW * 2 * 2 * 16];
   __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 256 : 4];
+  // The grid holds num_tiles units per head, of which the live ones are dealt; a batch of more takes further turns.
+  ShortBatch t = load_short_batch<MODE>(p, 32);
+  const int tiles = t.live < p.num_tiles ? t.live : p.num_tiles;
   int rank, kvh, slice;
-  if (!block_to_tile_slice(p, p.H / p.H_kv * FS, rank, kvh, slice)) return;
-  // The grid holds num_tiles units per head: all of them, or one per request, and the others follow in a second turn.
+  if (!block_to_tile_slice(p, tiles, p.H / p.H_kv * FS, rank, kvh, slice)) return;
   ShortUnit u;
-  for (; locate_short_unit<MODE>(p, 32, rank, u); rank += p.num_tiles) {
+  const int live = t.live;
+  while (locate_short_unit<MODE>(p, t, 32, rank, u)) {
     short_attn_unit<DTYPE, D, MODE, FS>(p, lds, lds_q, stats, lds_rope, kvh, kvh * (p.H / p.H_kv) + slice / FS, slice % FS, u);
+    rank += tiles;
+    if (rank >= live) return;
     __syncthreads();
+    t = load_short_batch<MODE>(p, 32);
   }
 }
 

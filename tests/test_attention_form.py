@@ -42,3 +42,31 @@ def test_other_head_dims_and_bad_sizes():
                 (1, 1, 1, 1, 1, 100, 0), (1, 1, 1, 1, 1, 128, 3)]:
         with pytest.raises(ValueError):
             form(*bad)
+
+
+def most_tiles(B, total_q):
+    return (total_q + 31 * B) // 32                              # of 32 rows, whatever the lengths
+
+
+def grid(tiles, H, Hkv, slices):
+    """Workgroups for `slices` units per tile and KV head: the fullest of the eight XCDs, times eight."""
+    if Hkv < 8 and 8 % Hkv == 0:
+        return 8 * slices * -(-tiles * Hkv // 8)
+    return -(-tiles * slices * Hkv // 8) * 8
+
+
+def test_wave_private_units_run_at_once():
+    """A workgroup of these fills its CU: blocks of one length never wait for a second turn, and where CUs are left, their
+    tiles are those of the longest blocks that the total allows."""
+    seen = set()
+    for B, total_q, total_k, H, Hkv, D in sizes():
+        for q in (total_q, total_q + 1):
+            for mode in (PLAIN, QUERY_SIDE):
+                kind, parts, tiles, blocks = form(B, q, total_k, H, Hkv, D, mode)
+                if kind == SHORT:
+                    assert blocks <= 256, (B, q, total_k, H, Hkv, D, mode)
+                    assert tiles >= (B if q % B == 0 else most_tiles(B, q))
+                    assert blocks == grid(tiles, H, Hkv, H // Hkv * parts)
+                    assert tiles == most_tiles(B, q) or grid(tiles + 1, H, Hkv, H // Hkv * parts) > 256
+                    seen.add((Hkv, parts))
+    assert {(3, 2), (3, 4), (4, 4), (32, 4), (8, 1)} <= seen
