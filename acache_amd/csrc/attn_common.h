@@ -367,9 +367,13 @@ __device__ __forceinline__ const char *uniform_ptr(const char *p) {
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
   return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
 }
-// The copy with the source given as a wave-uniform base plus a 32-bit byte offset per lane.
+// The copy with the source given as a wave-uniform base plus a 32-bit byte offset per lane.  A vector memory instruction must
+// not read a scalar register within five wait states of a vector instruction that wrote it, and the compiler, which knows
+// nothing of the read in here, reloads spilled scalars from vector lanes right in front.  The base is moved by a scalar
+// instruction, which waits for that write and needs no wait behind itself (and is the wait state after M0).
 __device__ __forceinline__ void lds_dma16_off(const char *base, uint32_t offset, uint32_t lds_offset) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "{m0}"(lds_offset) : "memory");
+  uint64_t moved;
+  asm volatile("s_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0" : "=&s"(moved) : "v"(offset), "s"(base), "{m0}"(lds_offset) : "memory");
 }
 
 // Online-softmax update of one key tile, in two steps shared by both attention kernels so that
