@@ -1052,10 +1052,10 @@ static int launch_attn_any_head_dim(const AttnParams &p, int mode, int64_t block
 // Which batches of short query blocks (32 rows per request on average at most) leave the per-head units of launch_attn.
 // Their plan, if any, is not needed.  The lengths are on the device: the host knows totals only.
 
-// Query tiles of a grid of `blocks` workgroups (a multiple of 8) with `slices` units per tile and KV head.  Room for more
-// tiles than a batch of one-length blocks has costs nothing where CUs would stay idle; `most` are enough for any lengths.
+// Tiles of a grid of up to `blocks` workgroups: `most` are enough for any lengths, and room for more than a batch of one-length
+// blocks has costs nothing where CUs would stay idle.
 static int32_t tiles_in_grid(const AttnParams &p, int slices, int64_t blocks, int64_t most) {
-  const int64_t tiles = p.H_kv < 8 && 8 % p.H_kv == 0 ? blocks / (8 * slices) * (8 / p.H_kv) : blocks / ((int64_t)slices * p.H_kv);
+  const int64_t tiles = tiles_in_grid(p, slices, blocks);
   return (int32_t)(tiles < most ? tiles : most);
 }
 
@@ -1071,10 +1071,12 @@ static int32_t tiles_in_grid(const AttnParams &p, int slices, int64_t blocks, in
 //   D 64, query side       0.94 to 1.00  0.87 to 0.96  0.81 to 0.89  0.79 to 0.88  0.75 to 0.79  0.63 to 0.69  0.47 to 0.60
 // (the eight waves' set-up and merge against a chain of short tiles).  Plain and key side share their lines: a key-side call
 // has the bits of a plain one over a materialised copy.
-// A request of more than 32 rows is several units.  They all fit the CUs if even the worst lengths do (two LLaDA requests
-// of 33 and 31 rows and 1300 keys: 24.5 us in per-head units, 30.3 with units in two turns, 18.8 in one).  Beyond that the
-// grid has a unit per request and head, further ones wait (8 Dream requests of 33 and 31 rows: 25.1 / 32.1 us), and the
-// batch has to look like blocks of one length, which is what refinement steps are.
+// A request of more than 32 rows is several units.  The grid has room for all that lengths of such a total can make, as far as
+// the CUs go (two requests of 33 and 31 rows, 32 / 32 heads and 1300 keys: 24.5 us in per-head units, 30.3 with units in two
+// turns, 18.8 in one), and for one per request and head at least.  What is behind that waits for a second turn, so a batch
+// that could make more has to look like blocks of one length, which is what refinement steps are; one that only looks so
+// pays: 8 requests of 33 and 31 rows, per-head units / here, 28 / 4 heads 400 keys 13.1 / 17.0 us plain, 1 100 keys 24.6 /
+// 26.8, 32 / 32 heads 1 100 keys 29.6 / 32.2.
 static bool takes_short_kernel(AttnParams &p, int mode, int64_t total_q, int64_t total_k) {
   const int64_t B = p.B;
   if ((p.head_dim != 128 && p.head_dim != 64) || total_q > 32 * B) return false;
@@ -1122,23 +1124,25 @@ static int parts_per_unit(const AttnParams &p, int64_t total_q) {
 // Two heads take one turn of the CUs, four up to two, where the last leaves at most a quarter of the CUs idle (with more
 // idle: plain 0.83 to 1.15, query side 0.75 to 1.04).  A batch that fits 256 units of one
 // head stays with those.  Plain and key side share their lines: a key-side call has the bits of a plain one over a
-// materialised copy.  All 32-row tiles get a unit where the worst lengths of such a batch fit the grid; beyond that it has
-// to look like blocks of one length, as for the kernel above.
+// materialised copy.  As above, the grid has room for all 32-row tiles as far as the CUs go (28 requests of up to 32 rows but
+// one of 45, 28 / 4 heads, 1 100 keys: per-head units 31.3 us, four heads in two turns 51.6, in one 31.3), a batch that could
+// make more has to look like blocks of one length, and one that only looks so runs in units of four heads where those fit:
+// 16 requests of 33 and 31 rows, 28 / 4 heads, 1 100 keys, per-head units / here: plain 29.2 / 31.9, key side 43.4 / 37.4.
 static int heads_per_group_unit(AttnParams &p, int mode, int64_t total_q, int64_t total_k) {
   const int64_t B = p.B;
   const int group = p.H / p.H_kv;
   if (p.head_dim != 128 || group < 2 || total_q > 32 * B) return 0;
   const bool query_side = mode == MODE_QUERY_SIDE;
-  const int32_t worst = (int32_t)((total_q + 31 * B) / 32);
-  p.num_tiles = total_q % B == 0 ? p.B : worst;
+  const int32_t most = (int32_t)((total_q + 31 * B) / 32);
+  p.num_tiles = total_q % B == 0 ? p.B : most;
   if (attn_grid_blocks(p) <= 256) return 0;
-  p.num_tiles = worst;
-  if (attn_grid_blocks(p, (group + 1) / 2) > 256) {
-    if (total_q % B != 0) return 0;
-    p.num_tiles = p.B;
+  if (attn_grid_blocks(p, (group + 1) / 2) <= 256) {
+    p.num_tiles = tiles_in_grid(p, (group + 1) / 2, 256, most);
+    return query_side || total_k >= 256 * B ? 2 : 0;
   }
-  if (attn_grid_blocks(p, (group + 1) / 2) <= 256) return query_side || total_k >= 256 * B ? 2 : 0;
+  if (total_q % B != 0) return 0;
   const int64_t units = attn_grid_blocks(p, (group + 3) / 4), idle = (512 - units) % 256;
+  p.num_tiles = tiles_in_grid(p, (group + 3) / 4, units <= 256 ? 256 : 512, most);
   return units <= 512 && (query_side ? idle <= 64 : idle < 64 && total_k <= 1536 * B) ? 4 : 0;
 }
 

@@ -308,6 +308,10 @@ inline int64_t attn_grid_blocks(const AttnParams &p, int group) {
   }
   return ((int64_t)p.num_tiles * group * p.H_kv + 7) / 8 * 8;  // the XCD remap needs a multiple of 8
 }
+// Query tiles of a grid of `blocks` workgroups, a multiple of 8, with `slices` units per tile and KV head.
+__host__ __device__ inline int64_t tiles_in_grid(const AttnParams &p, int slices, int64_t blocks) {
+  return p.H_kv < 8 && 8 % p.H_kv == 0 ? blocks / (8 * slices) * (8 / p.H_kv) : blocks / ((int64_t)slices * p.H_kv);
+}
 inline int64_t attn_grid_blocks(const AttnParams &p) { return attn_grid_blocks(p, p.H / p.H_kv); }
 
 // 32-bit copy offsets when the whole cache lies within 4 GiB of a head's base and the factors fit 24 bits

@@ -378,16 +378,10 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
   }
 }
 
+// The units of this workgroup: `tiles` query tiles of the batch are dealt in one turn, and what is behind them in others.
 template <int DTYPE, int D, int MODE, int FS>
-__global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
-  // the waves' buffers, the queries (and q'), the waves' (reference, denominator) pairs, the cos / sin rows of the shift
-  __shared__ __attribute__((aligned(1024))) char lds[NW * 32 * (D + D / FS) * 2];
-  __shared__ __attribute__((aligned(1024))) char lds_q[(MODE == MODE_QUERY_SIDE ? 2 : 1) * 32 * D * 2];
-  __shared__ float stats[NW * 2 * 2 * 16];
-  __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 256 : 4];
-  // The grid holds num_tiles units per head, of which the live ones are dealt; a batch of more takes further turns.
-  ShortBatch t = load_short_batch<MODE>(p, 32);
-  const int tiles = t.live < p.num_tiles ? t.live : p.num_tiles;
+__device__ __forceinline__ void short_attn_units(const AttnParams &p, char *lds, char *lds_q, float *stats, float *lds_rope,
+                                                 ShortBatch t, int tiles) {
   int rank, kvh, slice;
   if (!block_to_tile_slice(p, tiles, p.H / p.H_kv * FS, rank, kvh, slice)) return;
   ShortUnit u;
@@ -399,6 +393,26 @@ __global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
     __syncthreads();
     t = load_short_batch<MODE>(p, 32);
   }
+}
+
+template <int DTYPE, int D, int MODE, int FS>
+__global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
+  // the waves' buffers, the queries (and q'), the waves' (reference, denominator) pairs, the cos / sin rows of the shift
+  constexpr int FEWER = FS > 1 && MODE != MODE_PAGED ? FS / 2 : FS;
+  __shared__ __attribute__((aligned(1024))) char lds[NW * 32 * (D + D / FEWER) * 2];
+  __shared__ __attribute__((aligned(1024))) char lds_q[(MODE == MODE_QUERY_SIDE ? 2 : 1) * 32 * D * 2];
+  __shared__ float stats[NW * 2 * 2 * 16];
+  __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 256 : 4];
+  const ShortBatch t = load_short_batch<MODE>(p, 32);
+  // The grid holds num_tiles units per head, of which the live ones are dealt.  More than those (parts are counted for blocks
+  // of one length, other lengths make up to twice the tiles) run in half as many parts, which the grid holds: one turn of the
+  // CUs instead of two.  4 requests of 33 and 31 rows, 28 / 4 heads, 1 100 keys: plain 24.1 -> 15.3 us, key side 36.9 -> 21.9;
+  // 2 of 32 / 32 heads: 22.6 -> 14.7, 33.7 -> 20.5.  (The common body comes first: behind the other it took 2 to 5 % longer.)
+  if (FEWER == FS || __builtin_expect(p.B > 64 || t.live <= p.num_tiles, true))
+    short_attn_units<DTYPE, D, MODE, FS>(p, lds, lds_q, stats, lds_rope, t, t.live < p.num_tiles ? t.live : p.num_tiles);
+  else
+    short_attn_units<DTYPE, D, MODE, FEWER>(p, lds, lds_q, stats, lds_rope, t,
+                                            t.live < 2 * p.num_tiles ? t.live : 2 * p.num_tiles);
 }
 
 template <int DTYPE, int D, int MODE, int FS>

@@ -70,3 +70,21 @@ def test_wave_private_units_run_at_once():
                     assert tiles == most_tiles(B, q) or grid(tiles + 1, H, Hkv, H // Hkv * parts) > 256
                     seen.add((Hkv, parts))
     assert {(3, 2), (3, 4), (4, 4), (32, 4), (8, 1)} <= seen
+
+
+def test_grouped_units_have_room_for_longer_blocks():
+    """Two heads per unit: a turn of the CUs.  Four: up to two.  Where CUs are left, for the tiles of the longest blocks that
+    the total allows."""
+    seen = set()
+    for B, total_q, total_k, H, Hkv, D in sizes():
+        for q in (total_q, total_q + 1):
+            for mode in (PLAIN, QUERY_SIDE):
+                kind, heads, tiles, blocks = form(B, q, total_k, H, Hkv, D, mode)
+                if kind == GROUP:
+                    slices = -(-(H // Hkv) // heads)
+                    turns = 1 if heads == 2 or grid(B, H, Hkv, slices) <= 256 else 2
+                    assert blocks == grid(tiles, H, Hkv, slices) <= 256 * turns
+                    assert tiles >= (B if q % B == 0 else most_tiles(B, q))
+                    assert tiles == most_tiles(B, q) or grid(tiles + 1, H, Hkv, slices) > 256 * turns, (B, q, total_k, H, Hkv, D, mode)
+                    seen.add((heads, turns))
+    assert seen == {(2, 1), (4, 1), (4, 2)}

@@ -7,6 +7,7 @@ import torch
 
 from acache_amd import ops
 from oracle import acache_oracle as O
+from tests.test_attention_form import GROUP, SHORT, form, grid
 from tests.test_gpu_attention_short import A, START, _case, _check
 
 pytestmark = pytest.mark.gpu
@@ -131,3 +132,46 @@ def test_few_units_in_parts_have_the_same_bits(device, mode, H, Hkv, batches, dt
         got = ops.acache_attention(q, kc.view(shape), vc.view(shape), cu_q, cu_k, slots, **kwb).cpu()
         for b in range(B):
             assert torch.equal(got[b * q_len:(b + 1) * q_len], alone), (B, b)
+
+
+MODES = ["plain", "key", "query"]
+
+
+def _alternating(B):
+    q_lens = [33 - 2 * (b % 2) for b in range(B)]
+    q_lens[-1] += 32 * B - sum(q_lens)
+    return q_lens, sum(-(-q // 32) for q in q_lens)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("H,Hkv,B,parts", [(32, 32, 2, 4), (28, 4, 4, 2), (12, 3, 5, 4), (12, 3, 8, 2), (7, 1, 16, 2)])
+def test_more_tiles_than_requests_run_in_fewer_parts(device, mode, H, Hkv, B, parts, dtype):
+    """Blocks of 33 and 31 rows look like blocks of 32: their grid holds a tile per request (and what CUs are left), the
+    kernel deals all tiles in half as many parts.  The bits of whole units, which three times as many requests are."""
+    q_lens, tiles = _alternating(B)
+    t, kw = _case(q_lens, [470 + 13 * b for b in range(B)], H, Hkv, 128, dtype, mode, H + B)
+    total_k = t[5].numel()
+    kind, share, room, _ = form(B, 32 * B, total_k, H, Hkv, 128, MODES.index(mode))
+    assert (kind, share) == (SHORT, parts) and room < tiles
+    got = _check(t, kw, device)
+    n = 1
+    while form(n * B, 32 * n * B, n * total_k, H, Hkv, 128, MODES.index(mode))[:2] != (SHORT, 1):
+        n += 1
+    cu = lambda c: torch.cat([c[:1]] + [c[1:] + i * c[-1] for i in range(n)])
+    tb = [t[0].repeat(n, 1, 1), t[1], t[2], cu(t[3]), cu(t[4]), t[5].repeat(n)]
+    kwb = {k: v.repeat(n) if k in ("affix_shifts", "shared_kv_lens") else v for k, v in kw.items()}
+    assert torch.equal(_check(tb, kwb, device)[-32 * B:], got)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("H,Hkv,B,fits", [(28, 4, 16, True), (24, 8, 16, True), (12, 3, 40, True), (32, 8, 12, True), (32, 16, 16, False)])
+def test_more_tiles_than_requests_run_four_heads_per_unit(device, mode, H, Hkv, B, fits, dtype):
+    """The same for two heads per unit: units of four where the grid holds them, otherwise in a second turn."""
+    q_lens, tiles = _alternating(B)
+    t, kw = _case(q_lens, [250 + 5 * b for b in range(B)], H, Hkv, 128, dtype, mode, H + B)
+    kind, share, room, blocks = form(B, 32 * B, t[5].numel(), H, Hkv, 128, MODES.index(mode))
+    assert (kind, share) == (GROUP, 2) and room < tiles
+    assert (grid(tiles, H, Hkv, -(-(H // Hkv) // 4)) <= blocks) == fits
+    _check(t, kw, device)
