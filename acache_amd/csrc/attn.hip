@@ -1113,16 +1113,14 @@ static int parts_per_unit(const AttnParams &p, int64_t total_q) {
 //     plain                      0.88 to 1.18  0.82 to 1.09  0.80 to 1.03  0.85 to 1.03  0.85 to 1.03  0.85 to 0.94
 //     key side                   0.84 to 1.08  0.80 to 0.94  0.77 to 0.85  0.73 to 0.81  0.70 to 0.76  0.70 to 0.75
 //     query side                 0.78 to 0.91  0.81 to 0.94  0.78 to 0.90  0.78 to 0.87  0.72 to 0.82  0.63 to 0.72
-//   4 heads, 193 to 256 units
-//     plain                      0.78 to 0.92  0.77 to 0.90  0.82 to 0.94  0.88 to 0.99  0.97 to 1.03  0.93 to 1.06
-//     key side                   0.72 to 0.82  0.71 to 0.77  0.75 to 0.82  0.79 to 0.83  0.82 to 0.86  0.88 to 0.90
-//     query side                 0.66 to 0.74  0.72 to 0.78  0.74 to 0.81  0.81 to 0.88  0.85 to 0.93  0.84 to 0.88
-//   4 heads, 385 to 512 units
-//     plain                      0.78 to 0.83  0.80 to 0.86  0.84 to 0.90  0.89 to 0.94  0.86 to 0.99  0.83 to 1.03
-//     key side                   0.72 to 0.73  0.73 to 0.74  0.75          0.79 to 0.82  0.82 to 0.84  0.86 to 0.87
-//     query side                 0.67 to 0.70  0.73          0.75 to 0.76  0.81 to 0.83  0.84 to 0.86  0.85 to 0.88
-// Two heads take one turn of the CUs, four up to two, where the last leaves at most a quarter of the CUs idle (with more
-// idle: plain 0.83 to 1.15, query side 0.75 to 1.04).  A batch that fits 256 units of one
+//   4 heads, up to 512 units of which fewer than 64 are missing to full turns (groups of 3 to 7)
+//     plain                      0.65 to 1.03  0.69 to 1.05  0.76 to 1.05  0.84 to 1.06  0.83 to 1.11  0.82 to 1.11
+//     key side                   0.63 to 1.01  0.64 to 0.93  0.69 to 0.90  0.74 to 0.98  0.79 to 0.98  0.84 to 1.06
+//     query side                 0.55 to 0.83  0.61 to 0.89  0.65 to 0.87  0.72 to 0.90  0.78 to 0.93  0.77 to 0.94
+// Two heads take one turn of the CUs, four up to two, where the last leaves at most a quarter of the CUs idle (64 to 127 idle:
+// plain 0.74 to 1.18, key side 0.70 to 1.12, query side 0.63 to 1.00) and more than half of the waves have a head (otherwise
+// plain 0.84 to 1.76, key side 0.85 to 1.59, query side 0.78 to 1.56: groups of two, whose units lose half of their waves, and
+// groups of five that just do not fit in units of two, 12 requests of 40 / 8 heads).  A batch that fits 256 units of one
 // head stays with those.  Plain and key side share their lines: a key-side call has the bits of a plain one over a
 // materialised copy.  As above, the grid has room for all 32-row tiles as far as the CUs go (28 requests of up to 32 rows but
 // one of 45, 28 / 4 heads, 1 100 keys: per-head units 31.3 us, four heads in two turns 51.6, in one 31.3), a batch that could
@@ -1141,9 +1139,10 @@ static int heads_per_group_unit(AttnParams &p, int mode, int64_t total_q, int64_
     return query_side || total_k >= 256 * B ? 2 : 0;
   }
   if (total_q % B != 0) return 0;
-  const int64_t units = attn_grid_blocks(p, (group + 3) / 4), idle = (512 - units) % 256;
-  p.num_tiles = tiles_in_grid(p, (group + 3) / 4, units <= 256 ? 256 : 512, most);
-  return units <= 512 && (query_side ? idle <= 64 : idle < 64 && total_k <= 1536 * B) ? 4 : 0;
+  const int64_t units = attn_grid_blocks(p, (group + 3) / 4), turn = units <= 256 ? 256 : 512, idle = turn - units;
+  if (idle < 0 || B * p.H <= 2 * turn) return 0;
+  p.num_tiles = tiles_in_grid(p, (group + 3) / 4, turn, most);
+  return (query_side ? idle <= 64 : idle < 64 && total_k <= 1536 * B) ? 4 : 0;
 }
 
 // Two heads of a group per unit: where a unit per head is more than the two workgroup slots of every CU, which saves a

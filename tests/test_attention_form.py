@@ -88,3 +88,16 @@ def test_grouped_units_have_room_for_longer_blocks():
                     assert tiles == most_tiles(B, q) or grid(tiles + 1, H, Hkv, slices) > 256 * turns, (B, q, total_k, H, Hkv, D, mode)
                     seen.add((heads, turns))
     assert seen == {(2, 1), (4, 1), (4, 2)}
+
+
+def test_four_heads_per_unit_keep_most_waves_busy():
+    """Units of four heads have two waves per head: groups of two would leave half of them without one."""
+    groups = set()
+    for B, total_q, total_k, H, Hkv, D in sizes():
+        for mode in (PLAIN, QUERY_SIDE):
+            kind, heads, _, _ = form(B, total_q, total_k, H, Hkv, D, mode)
+            if kind == GROUP and heads == 4:
+                turns = 1 if grid(B, H, Hkv, -(-(H // Hkv) // 4)) <= 256 else 2
+                assert 8 * 256 * turns < 2 * 2 * B * H, (B, H, Hkv, mode)
+                groups.add(H // Hkv)
+    assert groups >= {3, 4, 7} and 2 not in groups
