@@ -364,6 +364,19 @@ __device__ __forceinline__ void lds_dma16_at(const char *src, uint32_t lds_offse
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(lds_offset) : "memory");
 }
 
+// The same with 4 bytes per lane, from any address of a float.
+__device__ __forceinline__ void lds_dma4_at(const float *src, uint32_t lds_offset) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "{m0}"(lds_offset) : "memory");
+}
+// Waves 0 .. D / 32 - 1 of a workgroup copy the cos and the sin row of `shift` into LDS, 64 floats each.  (By 16 bytes one
+// wave would do, but the tables are floats of any alignment.)
+template <int D>
+__device__ __forceinline__ void copy_rope_rows(const AttnParams &p, int shift, int wave, int lane, const float *lds_rope) {
+  if (wave >= D / 32) return;
+  const float *row = (wave < D / 64 ? p.cos_tab : p.sin_tab) + (int64_t)shift * D + wave % (D / 64) * 64;
+  lds_dma4_at(row + lane, __builtin_amdgcn_readfirstlane(lds_offset_of((const char *)lds_rope) + (uint32_t)wave * 256));
+}
+
 // A pointer every lane holds the same value of, moved to scalar registers.
 __device__ __forceinline__ const char *uniform_ptr(const char *p) {
   const uint64_t v = reinterpret_cast<uint64_t>(p);

@@ -195,11 +195,7 @@ __device__ __forceinline__ void group_attn_unit(const AttnParams &p, char *lds, 
     lds_dma16_at(src, __builtin_amdgcn_readfirstlane(lds_offset_of(lds_q) + (uint32_t)((wave * QCOPIES + i) * RPI * ROW_BYTES)));
   }
   if (lane == 0) landed[wave] = 0;
-  static_assert(2 * D * 4 == 64 * 16, "cos and sin row are one copy instruction");
-  if (relocates(MODE) && wave == 0) {
-    const float *row = (lane < 32 ? p.cos_tab : p.sin_tab) + (int64_t)shift * D;
-    lds_dma16_at(reinterpret_cast<const char *>(row) + (lane % 32) * 16, __builtin_amdgcn_readfirstlane(lds_offset_of((const char *)lds_rope)));
-  }
+  if (relocates(MODE)) copy_rope_rows<D>(p, shift, wave, lane, lds_rope);
   take_slots(0);
   copy_round(my_dst);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI) : "memory");  // queries and table rows have landed

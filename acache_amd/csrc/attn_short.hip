@@ -221,10 +221,7 @@ __device__ __forceinline__ void short_attn_unit(const AttnParams &p, char *lds, 
                       ((dma_piece ^ ((row / RW) % CH)) << 4);
     lds_dma16_at(src, __builtin_amdgcn_readfirstlane(lds_offset_of(lds_q) + (uint32_t)(wave * RPI * ROW_BYTES)));
   }
-  if (relocates(MODE) && wave == 0) {  // (at head dim 64 both rows twice)
-    const float *row = (lane / (D / 4) % 2 == 0 ? p.cos_tab : p.sin_tab) + (int64_t)shift * D;
-    lds_dma16_at(reinterpret_cast<const char *>(row) + (lane % (D / 4)) * 16, __builtin_amdgcn_readfirstlane(lds_offset_of((const char *)lds_rope)));
-  }
+  if (relocates(MODE)) copy_rope_rows<D>(p, shift, wave, lane, lds_rope);
   take_slots(0);
   copy_keys();                              // (a wave without a chunk copies zero rows)
   copy_values();
@@ -402,7 +399,7 @@ __global__ __launch_bounds__(64 * NW, 1) void short_attn_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(1024))) char lds[NW * 32 * (D + D / FEWER) * 2];
   __shared__ __attribute__((aligned(1024))) char lds_q[(MODE == MODE_QUERY_SIDE ? 2 : 1) * 32 * D * 2];
   __shared__ float stats[NW * 2 * 2 * 16];
-  __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 256 : 4];
+  __shared__ __attribute__((aligned(16))) float lds_rope[relocates(MODE) ? 2 * D : 4];
   const ShortBatch t = load_short_batch<MODE>(p, 32);
   // The grid holds num_tiles units per head, of which the live ones are dealt.  More than those (parts are counted for blocks
   // of one length, other lengths make up to twice the tiles) run in half as many parts, which the grid holds: one turn of the

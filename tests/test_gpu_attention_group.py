@@ -175,3 +175,20 @@ def test_more_tiles_than_requests_run_four_heads_per_unit(device, mode, H, Hkv, 
     assert (kind, share) == (GROUP, 2) and room < tiles
     assert (grid(tiles, H, Hkv, -(-(H // Hkv) // 4)) <= blocks) == fits
     _check(t, kw, device)
+
+
+@pytest.mark.parametrize("mode", ["key", "query"])
+@pytest.mark.parametrize("H,Hkv,D,B,kind", [(32, 32, 128, 1, SHORT), (16, 16, 64, 3, SHORT), (28, 4, 128, 12, GROUP), (28, 4, 128, 30, GROUP)])
+def test_rope_tables_of_any_alignment(device, mode, H, Hkv, D, B, kind):
+    """Tables are contiguous floats, not 16-byte aligned ones: the same bits from a view one float into an allocation."""
+    t, kw = _case([32] * B, [560] * B, H, Hkv, D, torch.bfloat16, mode, B)
+    assert form(B, 32 * B, t[5].numel(), H, Hkv, D, MODES.index(mode))[0] == kind
+    got = _check(t, kw, device)
+    q, kc, vc, cu_q, cu_k, slots = (x.to(device) for x in t)
+    kw = {k: v.to(device) if torch.is_tensor(v) else v for k, v in kw.items()}
+    for name, by in (("rope_cos", 1), ("rope_sin", 3)):
+        moved = torch.empty(kw[name].numel() + by, device=device)[by:].view(kw[name].shape)
+        kw[name] = moved.copy_(kw[name])
+        assert moved.data_ptr() % 16 == 4 * by and moved.is_contiguous()
+    shape = (kc.shape[0] // 16, 16, *kc.shape[1:])
+    assert torch.equal(ops.acache_attention(q, kc.view(shape), vc.view(shape), cu_q, cu_k, slots, **kw).cpu(), got)
