@@ -37,9 +37,14 @@ def _code(t: torch.Tensor) -> int:
         raise ValueError(f"unsupported dtype {t.dtype}; expected bfloat16, float16 or float32") from None
 
 
-# The host side of a launch.  A short call (the attention of one request: 13 to 15 us on the GPU) is bound by it, and
+# The host side of a launch.  A short call (the attention of one request: 11.4 us on the GPU) is bound by it, and
 # entering a device context and building a Stream object took 3.4 of its 16.5 us.
 _HERE = nullcontext()
+try:
+    from torch._C import _cuda_getCurrentRawStream as _raw_stream
+except ImportError:  # a function of torch's own use, which another version may not have
+    def _raw_stream(index: int) -> int:
+        return torch.cuda.current_stream(index).cuda_stream
 
 
 def _on(t: torch.Tensor):
@@ -49,7 +54,7 @@ def _on(t: torch.Tensor):
 
 def _stream(t: torch.Tensor) -> int:
     """Handle of the stream that is current on ``t``'s device."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    return _raw_stream(t.get_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:

@@ -79,3 +79,20 @@ def test_ops_fail_loudly_when_the_library_is_missing(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "libacache_hip.so")
     with pytest.raises(_lib.AcacheLibraryError, match="no fallback"):
         _lib.load()
+
+
+def test_streams_are_found_without_torchs_raw_stream_function(monkeypatch):
+    """The function that hands out stream handles is torch's own: a torch without it launches on its Stream objects."""
+    import importlib.util
+    from types import SimpleNamespace
+
+    import torch
+
+    from acache_amd import ops
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    spec = importlib.util.spec_from_file_location("acache_amd.ops_of_another_torch", ops.__file__)
+    other = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(other)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda index: SimpleNamespace(cuda_stream=100 + index))
+    assert other._stream(SimpleNamespace(get_device=lambda: 3)) == 103
