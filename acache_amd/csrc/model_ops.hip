@@ -36,10 +36,13 @@ __global__ __launch_bounds__(256) void swiglu_kernel(char *out, const char *gu, 
 // rounded to the storage type before the weight multiplies it and the product rounded again, which is where the
 // reference's layer norm rounds (llada/model/modeling_llada.py:338-350: x.to(og_dtype), then weight * x).
 // Without delta the sum is x itself and is not written.  One 256-thread block per row; a thread keeps its
-// chunks of the row in registers between the two steps (rows of up to 256 * 16 bytes * kMaxChunks).
+// chunks of the row in registers between the two steps (rows of up to 256 * 16 bytes * kMaxChunks): a kernel for every number
+// of chunks, so that a row holds no more registers than it has.  (One kernel for all holds 62 to 66 since everything is asked
+// for at once, and fp16 rows of 2 048 x 4 096 elements took 14.5 us, 13.1 with loads one after the other, 13.9 now; 2 048 x
+// 5 120 18.0, 15.9, 17.2.  Weights behind the row's own loads: 10 % slower at 4 096 rows.)
 constexpr int kMaxChunks = 4;
 
-template <int DTYPE>
+template <int DTYPE, int CHUNKS>
 __global__ __launch_bounds__(256) void add_rms_norm_kernel(char *sum, const char *x, const char *delta,
                                                            const char *weight, char *y, int chunks_per_row,
                                                            int64_t sum_row_bytes, int64_t x_row_bytes,
@@ -54,9 +57,9 @@ __global__ __launch_bounds__(256) void add_rms_norm_kernel(char *sum, const char
   char *yr = y + (int64_t)blockIdx.x * y_row_bytes;
   // Everything the row needs is asked for at once: a row is one latency, not one per chunk and one for the weight (32 rows of
   // 4 096 bf16 elements 4.8 -> 3.9 us).
-  vec16 rx[kMaxChunks], rd[kMaxChunks], rw[kMaxChunks];
+  vec16 rx[CHUNKS], rd[CHUNKS], rw[CHUNKS];
 #pragma unroll
-  for (int i = 0; i < kMaxChunks; ++i) {
+  for (int i = 0; i < CHUNKS; ++i) {
     const int c = tid + i * 256;
     if (c < chunks_per_row) {
       rx[i] = load16(xr + c * 16);
@@ -64,10 +67,10 @@ __global__ __launch_bounds__(256) void add_rms_norm_kernel(char *sum, const char
       rw[i] = load16(weight + c * 16);
     }
   }
-  float v[kMaxChunks][VEC];
+  float v[CHUNKS][VEC];
   float ss = 0.0f;
 #pragma unroll
-  for (int i = 0; i < kMaxChunks; ++i) {
+  for (int i = 0; i < CHUNKS; ++i) {
     const int c = tid + i * 256;
     if (c < chunks_per_row) {
       E::unpack(rx[i], v[i]);
@@ -91,7 +94,7 @@ __global__ __launch_bounds__(256) void add_rms_norm_kernel(char *sum, const char
   __syncthreads();
   const float scale = rsqrtf((part[0] + part[1] + part[2] + part[3]) * inv_d + eps);
 #pragma unroll
-  for (int i = 0; i < kMaxChunks; ++i) {
+  for (int i = 0; i < CHUNKS; ++i) {
     const int c = tid + i * 256;
     if (c < chunks_per_row) {
       float w[VEC], o[VEC];
@@ -158,17 +161,22 @@ extern "C" int acache_add_rms_norm(void *sum, const void *x, const void *delta, 
   if (M > 0x7fffffffLL) return fail(ACACHE_E_SHAPE, "add_rms_norm: too many rows");
   hipStream_t s = (hipStream_t)stream;
   const int cpr = (int)(d * es / 16);
-#define ACACHE_CASE(DT)                                                                                          \
-  if (dtype == DT) {                                                                                             \
-    hipLaunchKernelGGL((add_rms_norm_kernel<DT>), dim3((unsigned)M), dim3(256), 0, s, (char *)sum,               \
+  const int chunks = (cpr + 255) / 256;
+  static_assert(kMaxChunks == 4, "a kernel for every number of chunks");
+#define ACACHE_CHUNKS(DT, N)                                                                                     \
+  if (chunks == N) {                                                                                             \
+    hipLaunchKernelGGL((add_rms_norm_kernel<DT, N>), dim3((unsigned)M), dim3(256), 0, s, (char *)sum,            \
                        (const char *)x, (const char *)delta, (const char *)weight, (char *)y, cpr,               \
                        sum_row_stride * es, x_row_stride * es, delta_row_stride * es, y_row_stride * es, eps,    \
                        1.0f / (float)d);                                                                         \
     return launch_status("add_rms_norm_kernel");                                                                 \
   }
+#define ACACHE_CASE(DT) \
+  if (dtype == DT) { ACACHE_CHUNKS(DT, 1) ACACHE_CHUNKS(DT, 2) ACACHE_CHUNKS(DT, 3) ACACHE_CHUNKS(DT, 4) }
   ACACHE_CASE(ACACHE_BF16)
   ACACHE_CASE(ACACHE_F16)
   ACACHE_CASE(ACACHE_F32)
 #undef ACACHE_CASE
+#undef ACACHE_CHUNKS
   return fail(ACACHE_E_DTYPE, "add_rms_norm: unknown dtype %d", dtype);
 }

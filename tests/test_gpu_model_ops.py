@@ -75,6 +75,25 @@ def test_add_rms_norm_matches_fp32_reference(device, dtype, M, d):
     _close(y0, xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5) * w.float(), dtype, scale=2.0)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("chunk", [1, 2, 3, 4])
+@pytest.mark.parametrize("over", [-1, 0, 1])
+def test_add_rms_norm_at_the_edges_of_a_threads_chunks(device, dtype, chunk, over):
+    """A kernel for every number of 16-byte chunks that a thread holds of a row: rows that just fill it, and one chunk to both
+    sides."""
+    per = 16 // torch.empty(0, dtype=dtype).element_size()
+    d = per * (256 * chunk + over)
+    if d > 1024 * per:
+        return                                                       # refused: the test above
+    g = torch.Generator(device=device).manual_seed(d)
+    x, delta = (torch.randn(5, d, generator=g, device=device).to(dtype) for _ in range(2))
+    w = (1 + 0.1 * torch.randn(d, generator=g, device=device)).to(dtype)
+    total, y = ops.add_rms_norm(x, delta, w, 1e-5)
+    assert torch.equal(total, x + delta)
+    s = total.float()
+    _close(y, s * torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-5) * w.float(), dtype, scale=2.0)
+
+
 def test_add_rms_norm_argument_errors(device):
     x = torch.zeros(2, 8200, device=device, dtype=torch.bfloat16)
     with pytest.raises(ValueError):                                   # row longer than the kernel keeps in registers
