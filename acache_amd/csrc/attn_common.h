@@ -38,7 +38,7 @@ struct AttnParams {
   int32_t H_kv;
   int32_t num_tiles;  // upper bound on the number of BM-row query tiles
   int32_t head_dim;   // real head_dim (read by the padded any-head_dim variant only)
-  int32_t small_cache;  // 32-bit copy offsets reach the whole cache (read by the short-query kernel)
+  int32_t small_cache;  // 32-bit copy offsets reach the whole cache (read by the short-block kernels)
   int64_t num_slots;
   int64_t q_token_bytes, q_head_bytes;
   int64_t o_token_bytes, o_head_bytes;
@@ -94,8 +94,7 @@ __device__ __forceinline__ bool locate_query_tile(const int32_t *cu_q, int B, in
 // list scheduling: the short blocks fill the gaps at the end instead of the long ones sticking out.
 __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const int32_t *cu_k, int B, int BM,
                                                       int rank, int &b_out, int &q_begin, int &q_len,
-                                                      int &tile_in_request, int &kv_begin, int &kv_len,
-                                                      int *live_tiles = nullptr) {
+                                                      int &tile_in_request, int &kv_begin, int &kv_len) {
   const int lane = threadIdx.x & 63;
   // four unconditional loads at a clamped index: one memory round trip (loads under a lane mask end up in
   // separate blocks, each with its own wait)
@@ -108,7 +107,6 @@ __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const
   // One key per request orders them (longer first, then lower index; the clamp only bounds how fine the order is).
   const int key = ((kv < 0x1ffffff ? (kv > 0 ? kv : 0) : 0x1ffffff) << 6) | (63 - lane);
   int before = 0;  // query tiles of the requests sorted in front of this lane's request
-  int all = 0;     // and of all requests
   // Selects on one key, two requests a turn (lanes past B have no tiles; four a turn cost planned launches, which jump over
   // this code, 1.1 us: it is fetched with theirs).  As a branch on two compares per request the ranking took most of a short
   // unit: whole calls of 32 query rows, before / now: 64 requests of 32 heads and 200 keys 69.6 / 55.2 us, of 8 heads and 300
@@ -120,10 +118,8 @@ __device__ __forceinline__ bool locate_query_tile_lpt(const int32_t *cu_q, const
       const int key_j = __builtin_amdgcn_readlane(key, j0 + j);
       const int tiles_j = __builtin_amdgcn_readlane(tiles, j0 + j);
       before += key_j > key ? tiles_j : 0;
-      all += tiles_j;
     }
   }
-  if (live_tiles) *live_tiles = all;
   const uint64_t hit = __builtin_amdgcn_ballot_w64(lane < B && rank >= before && rank < before + tiles);
   if (hit == 0) return false;
   const int src = __builtin_ctzll(hit);
