@@ -23,7 +23,7 @@ def _units(B, H, Hkv, heads):
 @pytest.mark.parametrize("mode", ["plain", "key", "query"])
 @pytest.mark.parametrize("heads,B,H,Hkv,dtype", [(2, 10, 28, 4, torch.bfloat16), (2, 16, 32, 8, torch.float16),
                                                  (2, 23, 12, 3, torch.float16), (2, 28, 10, 2, torch.bfloat16),
-                                                 (4, 29, 28, 4, torch.bfloat16), (4, 52, 10, 2, torch.float16),
+                                                 (4, 30, 24, 8, torch.bfloat16), (4, 29, 28, 4, torch.bfloat16), (4, 52, 10, 2, torch.float16),
                                                  (4, 118, 14, 2, torch.bfloat16), (4, 32, 48, 8, torch.float16)])
 def test_ragged_batches_against_the_oracle(device, mode, heads, B, H, Hkv, dtype):
     n = B - 1                                                    # the last request raises the average to 256 keys
@@ -62,7 +62,7 @@ def test_absent_rows_are_zero_and_64_bit_addresses_change_nothing(device):
     assert torch.equal(ops.acache_attention(q, *wide, cu_q, cu_k, few), ops.acache_attention(q, kc[:24], vc[:24], cu_q, cu_k, few))
 
 
-@pytest.mark.parametrize("keys", [200, 300])
+@pytest.mark.parametrize("keys", [200, 255, 256, 300, 1536, 1537])
 @pytest.mark.parametrize("H,Hkv,B", [(28, 4, 10), (32, 8, 16), (28, 4, 30)])
 def test_key_side_equals_a_materialised_copy(device, keys, H, Hkv, B):
     """On both sides of the lines of the dispatch, plain attention over a relocated copy takes the form that key-side

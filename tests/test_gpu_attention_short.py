@@ -8,6 +8,7 @@ import torch
 
 from acache_amd import ops
 from oracle import acache_oracle as O
+from tests.test_attention_form import SHORT, form
 
 pytestmark = pytest.mark.gpu
 A, START = 40, 9      # shared rows (slots 0 .. A-1) and, in the relocation modes, private keys in front of them
@@ -84,14 +85,16 @@ def test_more_tiles_than_units(device, mode, H, Hkv, q_lens):
     _check(t, kw, device)
 
 
+@pytest.mark.parametrize("H,Hkv,parts", [(2, 1, 4), (96, 8, 2), (160, 8, 1)])
 @pytest.mark.parametrize("mode", ["plain", "key", "query"])
-def test_slots_are_refilled_and_absent_rows_are_zero(device, mode):
+def test_slots_are_refilled_and_absent_rows_are_zero(device, mode, H, Hkv, parts):
     # the keys behind the first 4096 have values around 40: they carry 145 / 4241 of the weight, so the result moves by more
     # than 1 without them and by 0.3 for every chunk of 32 that is read from other slots
-    t, kw = _case([32], [4241], 2, 1, 128, torch.bfloat16, mode, 4)
+    t, kw = _case([32], [4241], H, Hkv, 128, torch.bfloat16, mode, 4)
+    assert form(1, 32, t[5].numel(), H, Hkv, 128, 0)[:2] == (SHORT, parts)
     t[2][t[5][4096:].long()] += 40
     assert _check(t, kw, device).float().mean() > 1
-    if mode == "plain":
+    if mode == "plain" and H == 2:
         t, kw = _case([20, 32], [150, 77], 2, 2, 128, torch.bfloat16, mode, 5, holes=True, keys_per_request=1024)
         present = (t[5] >= 0) & (t[5] < t[1].shape[0])
         zero = t[1].shape[0] - 1                                 # what an absent row reads as
@@ -151,7 +154,8 @@ def test_plan_and_slot_pitch_do_not_change_the_bits(device):
         assert torch.equal(ops.acache_attention(q, *wide, *args), ops.acache_attention(q, kc, vc, *args))
 
 
-@pytest.mark.parametrize("D,keys", [(128, 700), (128, 900), (128, 1100), (64, 400), (64, 600)])
+@pytest.mark.parametrize("D,keys", [(128, 300), (128, 399), (128, 400), (128, 700), (128, 900), (128, 1100), (64, 400), (64, 511),
+                                    (64, 512), (64, 600)])
 @pytest.mark.parametrize("H,Hkv,B", [(4, 4, 3), (28, 4, 7), (16, 16, 8), (16, 16, 9)])
 def test_key_side_equals_a_materialised_copy(device, D, keys, H, Hkv, B):
     """On both sides of every line of the dispatch, plain attention over a relocated copy takes the form that key-side
