@@ -1095,7 +1095,7 @@ static bool takes_short_kernel(AttnParams &p, int mode, int64_t total_q, int64_t
 // 32 / 32, 28 / 4 and 8 / 2 heads, 300 to 2 000 keys, blocks of 8 and 32 rows):
 //   up to  64 units, four parts   plain 0.79 to 0.92, key side 0.81 to 0.93, query side 0.82 to 0.92 (two: 0.85 to 0.93)
 //   up to 128 units, two parts    plain 0.86 to 0.99, key side 0.86 to 0.94, query side 0.88 to 1.01
-// One request of 32 heads and 1 300 keys 16.1 -> 13.0 us.  (Parts of the keys instead would have to meet in memory: a second
+// One request of 32 heads and 1 300 keys 14.7 -> 12.2 us.  (Parts of the keys instead would have to meet in memory: a second
 // launch or a counter that every call finds at zero.)
 static int parts_per_unit(const AttnParams &p, int64_t total_q) {
   AttnParams t = p;

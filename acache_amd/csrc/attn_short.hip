@@ -20,11 +20,13 @@
 // lookup of one request at a time it was 5.0 us of one request's 14.9.
 //
 // Measured (bf16, D = 128, 32 query rows and about 1 300 keys per request, three quarters of them shared in the relocation
-// modes, microseconds per call, varlen_attn_unit_kernel / this kernel with a set-up per wave / now):
-//   32 / 32 heads, plain 1 request 18.4 / 16.3 / 14.7, 4: 22.6 / 23.0 / 20.2; query side 1: 23.6 / 19.0 / 15.5, 4: 30.8 /
-//   23.6 / 19.3, 8: 33.5 / 26.1 / 21.1; key side 1: 29.4 / 24.5 / 21.1.  28 / 4 heads, plain 1: 18.6 / 16.7 / 14.9, 8: 19.5 /
-//   19.5 / 16.9; query side 8: 25.6 / 22.1 / 17.7; key side 8: 31.1 / 28.8 / 23.6.  One request of 32 heads
-//   keeps 32 CUs busy with 590 KB of keys and values each, which takes 5.4 us by copies alone (110 GB/s into one CU).
+// modes, microseconds per call, varlen_attn_unit_kernel / this kernel with a set-up per wave / whole units / now, in parts
+// where units are few):
+//   32 / 32 heads, plain 1 request 18.4 / 16.3 / 14.7 / 12.2, 4: 22.6 / 23.0 / 20.2 / 20.1; query side 1: 23.6 / 19.0 / 15.5 /
+//   13.0, 4: 30.8 / 23.6 / 19.3 / 15.8, 8: 33.5 / 26.1 / 21.1 / 20.6; key side 1: 29.4 / 24.5 / 21.1 / 18.7.  28 / 4 heads,
+//   plain 1: 18.6 / 16.7 / 14.9 / 12.5, 8: 19.5 / 19.5 / 16.9 / 16.6; query side 8: 25.6 / 22.1 / 17.7 / 17.1; key side 8: 31.1 /
+//   28.8 / 23.6 / 23.6.  In whole units one request of 32 heads and 1 150 keys is 32 CUs with 590 KB of keys and values each,
+//   which take 5.4 us by copies alone (110 GB/s into one CU); in four parts 128 CUs with 370 KB each.
 #include "attn_common.h"
 
 namespace acache {

@@ -601,9 +601,9 @@ __global__ __launch_bounds__(256) void importance_colsum_lds_kernel(ImportancePa
 //
 // LLaDA heads, 256 rows a request, relocated, both launches of the call, two passes / this form: 16 requests with 300 /
 // 600 / 1000 / 1100 / 1200 keys 68 / 90 / 120 / 134 / 139 -> 41 / 52 / 68 / 79 / 88 us; one request of 300 / 1000 keys
-// 33 / 55 -> 13 / 20 us.  By the counters of the 1000-key launch a wave spends 512 matrix-pipe cycles and 350 vector
+// 33 / 55 -> 13 / 20 us.  By the counters of the 1000-key launch a wave spends 512 matrix-pipe cycles and 325 vector
 // instructions on a 16-row tile (rotation, stores and the keys' way into registers included), two waves per SIMD, the matrix
-// pipe is busy 22 % of the time and 30 % of the wave cycles wait.  Sums of a
+// pipe is busy 23 % of the time and 30 % of the wave cycles wait.  Sums of a
 // whole chunk of up to 256 rows instead of 64 took 64 us at 1000 keys, but their order followed the batch.
 // Measured and not taken: the two waves of a SIMD at different priorities (no change); scoring a wave's keys in two
 // halves with references of their own, the first half's exponentials between the matrix instructions of the second
@@ -780,7 +780,7 @@ __global__ __launch_bounds__(kFusedThreads) void importance_fused_kernel(Importa
 #pragma nounroll
       for (int r = tid / PAIRS; r < now.rows; r += kFusedThreads / PAIRS) {
         vec16 lo = load16(q_rows + G::offset(r, ch)), hi = load16(q_rows + G::offset(r, ch + PAIRS));
-        rotate_pair_half_fast<DTYPE>(lo, hi, cs, sn, 0, 8, -1.0f);  // (188 -> 100 instructions a turn of this loop)
+        rotate_pair_half_fast<DTYPE>(lo, hi, cs, sn, 0, 8, -1.0f);  // (188 -> 85 instructions a turn of this loop)
         store16(q_rows + G::offset(r, ch), lo);
         store16(q_rows + G::offset(r, ch + PAIRS), hi);
       }

@@ -78,7 +78,8 @@ __global__ __launch_bounds__(256) void block_table_slots_kernel(
 // What a step over a batch of block-table requests needs, from their lengths alone: both prefix sums and the slot map, in
 // one launch.  A block sums the lengths in front of its request by itself (a few hundred bytes from L2), so nothing has to
 // be scanned first: the launch is one latency, where zero-fill, scan, cast, copy, arange and slot map were six (16 requests
-// of 1 400 tokens: the whole attention call 52 us, now 30).
+// of 1 400 tokens, with the attention of per-head units behind it: 52 -> 30 us).  The short-block kernels read lengths and
+// tables themselves; this is for the other kernels, more than 64 requests and cache blocks those do not take.
 __global__ __launch_bounds__(256) void decode_layout_kernel(int32_t *cu_q, int32_t *cu_k, int32_t *out, const int32_t *seqlens,
                                                             const int32_t *tables, int q_len, int max_blocks,
                                                             int block_size, int64_t total_k) {
