@@ -40,9 +40,9 @@ MEASURED_TRAFFIC = {
                            "sources": ["acache_amd/csrc/relocate.hip", "acache_amd/csrc/common.h"]},
     "relocate_fp32": {"bytes": 1879.1e6, "commit": "b696828",
                       "sources": ["acache_amd/csrc/relocate.hip", "acache_amd/csrc/common.h"]},
-    "scatter_28_layers": {"bytes": 332.0e6, "commit": "51864f1",
+    "scatter_28_layers": {"bytes": 332.0e6, "commit": "9893795",
                           "sources": ["acache_amd/csrc/scatter.hip", "acache_amd/csrc/common.h"]},
-    "attention": {"bytes": 340.1e6, "commit": "211649d",
+    "attention": {"bytes": 341.2e6, "commit": "9893795",
                   "sources": ["acache_amd/csrc/attn.hip", "acache_amd/csrc/attn_common.h", "acache_amd/csrc/mma.h",
                               "acache_amd/csrc/common.h", "acache_amd/csrc/attn_plan.hip"]},
 }
