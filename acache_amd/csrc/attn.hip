@@ -973,7 +973,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_pair_kernel(AttnParams p) 
   __shared__ __attribute__((aligned(1024))) char lds[4 * TILE_BYTES + (MODE == MODE_KEY_SIDE ? 2 * D * 4 : 0)];
   const int group = p.H / p.H_kv;
   int rank, kvh, slice, b = 0, q_begin = 0, q_len = 0, tile = 0, kv_begin = 0, kv_len = 0;
-  if (!block_to_tile_slice(p, p.num_tiles, (group + 1) / 2, rank, kvh, slice)) return;
+  if (!block_to_tile_slice<false>(p, p.num_tiles, (group + 1) / 2, rank, kvh, slice)) return;
   if (p.B <= 64) {
     if (!locate_query_tile_lpt(p.cu_q, p.cu_k, p.B, 32, rank, b, q_begin, q_len, tile, kv_begin, kv_len)) return;
   } else {

@@ -265,9 +265,11 @@ __device__ __forceinline__ int slot_of_entry(const AttnParams &p, int entry, int
 // The grid must hold attn_grid_blocks(p) blocks.  Returns false for a block without work.
 // `group` is the number of units per KV head and query tile: the query heads of the KV head, or fewer for a kernel whose
 // units take several of them.
-// `num_tiles` of them are dealt, of the tiles that the grid holds: a kernel that knows how many there are gives every XCD its
-// share of those.
+// LIVE: a kernel that knows how many tiles there are (`num_tiles`), of those that its grid holds, gives every XCD its share of
+// them in the last case.
+template <bool LIVE>
 __device__ __forceinline__ bool block_to_tile_slice(const AttnParams &p, int num_tiles, int group, int &tile, int &kvh, int &hg) {
+  int per_xcd = gridDim.x >> 3;
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   if (p.H_kv % 8 == 0) {
     const int heads_per_xcd = (p.H_kv >> 3) * group;
@@ -283,9 +285,10 @@ __device__ __forceinline__ bool block_to_tile_slice(const AttnParams &p, int num
     if (tile >= num_tiles) return false;
     hg = idx % group;
   } else {
-    const int units = num_tiles * group * p.H_kv, per_xcd = (units + 7) >> 3;
+    const int units = num_tiles * group * p.H_kv;
+    if (LIVE) per_xcd = (units + 7) >> 3;
     const int w = xcd * per_xcd + idx;
-    if (idx >= per_xcd || w >= units) return false;
+    if ((LIVE && idx >= per_xcd) || w >= units) return false;
     hg = w % group;
     tile = (w / group) % num_tiles;
     kvh = w / (group * num_tiles);
@@ -294,7 +297,7 @@ __device__ __forceinline__ bool block_to_tile_slice(const AttnParams &p, int num
 }
 
 __device__ __forceinline__ bool block_to_tile_head(const AttnParams &p, int &tile, int &kvh, int &hg) {
-  return block_to_tile_slice(p, p.num_tiles, p.H / p.H_kv, tile, kvh, hg);
+  return block_to_tile_slice<false>(p, p.num_tiles, p.H / p.H_kv, tile, kvh, hg);
 }
 
 inline int64_t attn_grid_blocks(const AttnParams &p, int group) {

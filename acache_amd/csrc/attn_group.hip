@@ -370,7 +370,7 @@ __device__ __forceinline__ void group_attn_units(const AttnParams &p, char *lds,
                                                  ShortBatch t, int tiles) {
   const int group = p.H / p.H_kv;
   int rank, kvh, slice;
-  if (!block_to_tile_slice(p, tiles, (group + HU - 1) / HU, rank, kvh, slice)) return;
+  if (!block_to_tile_slice<true>(p, tiles, (group + HU - 1) / HU, rank, kvh, slice)) return;
   const int first = slice * HU, heads = group - first < HU ? group - first : HU;
   ShortUnit u;
   const int live = t.live;

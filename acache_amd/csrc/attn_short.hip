@@ -382,7 +382,7 @@ template <int DTYPE, int D, int MODE, int FS>
 __device__ __forceinline__ void short_attn_units(const AttnParams &p, char *lds, char *lds_q, float *stats, float *lds_rope,
                                                  ShortBatch t, int tiles) {
   int rank, kvh, slice;
-  if (!block_to_tile_slice(p, tiles, p.H / p.H_kv * FS, rank, kvh, slice)) return;
+  if (!block_to_tile_slice<true>(p, tiles, p.H / p.H_kv * FS, rank, kvh, slice)) return;
   ShortUnit u;
   const int live = t.live;
   while (locate_short_unit<MODE>(p, t, 32, rank, u)) {
