@@ -42,7 +42,7 @@ MEASURED_TRAFFIC = {
                       "sources": ["acache_amd/csrc/relocate.hip", "acache_amd/csrc/common.h"]},
     "scatter_28_layers": {"bytes": 332.0e6, "commit": "9893795",
                           "sources": ["acache_amd/csrc/scatter.hip", "acache_amd/csrc/common.h"]},
-    "attention": {"bytes": 341.2e6, "commit": "9893795",
+    "attention": {"bytes": 340.5e6, "commit": "93692cd",
                   "sources": ["acache_amd/csrc/attn.hip", "acache_amd/csrc/attn_common.h", "acache_amd/csrc/mma.h",
                               "acache_amd/csrc/common.h", "acache_amd/csrc/attn_plan.hip"]},
 }
